@@ -107,6 +107,7 @@ struct su2hip_batch {
   MucaDev *d_muca = nullptr;
   BlockMap *d_blk = nullptr;
   int nblk = 0, nblk_cap = 0;
+  int one = -1;                   // the only slot in use, else -1
   std::vector<BlockMap> h_blk;
   long long *d_cnt = nullptr;
   double *d_partial = nullptr;
@@ -244,6 +245,7 @@ static LaunchCtx ctx_of(su2hip_batch *b) {
   c.muca = b->d_muca;
   c.blk = b->d_blk;
   c.nblk = b->nblk;
+  c.one = b->one;
   c.cnt = b->d_cnt;
   c.partial = b->d_partial;
   c.sums = b->d_sums;
@@ -539,6 +541,10 @@ static int rebuild_map(su2hip_batch *b) {
     b->partial_cap = need;
   }
   b->nblk = n;
+  b->one = -1;
+  int used = 0;
+  for (int i = 0; i < b->max_slots; i++)
+    if (b->slots[i].used) b->one = used++ ? -1 : i;
   b->h_blk = phys;
   if (n) {
     HIPTRY(hipMemcpyAsync(b->d_blk, phys.data(), sizeof(BlockMap) * n, hipMemcpyHostToDevice,

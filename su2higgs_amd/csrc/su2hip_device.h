@@ -128,6 +128,32 @@ template <typename T>
 __device__ __forceinline__ T qdot(const Q<T> &x, const Q<T> &y) {
   return x.a * y.a + x.b * y.b + x.c * y.c + x.d * y.d;
 }
+// p q + r s with the fused product named (W = 1: p q, W = 2: r s).  Left to
+// the compiler, the choice depends on the code around the sum, and in FP32 a
+// Metropolis or heatbath draw turns one rounding into another accept
+// decision now and then; where code around a sum of products changed, its
+// rounding is pinned to what it was.
+__device__ __forceinline__ float ffma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double ffma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+template <int W, typename T>
+__device__ __forceinline__ T sum2(T p, T q, T r, T s) {
+  return W == 1 ? ffma(p, q, r * s) : ffma(r, s, p * q);
+}
+template <int W, typename T>
+__device__ __forceinline__ T qdot_w(const Q<T> &x, const Q<T> &y) {
+  return ffma(x.d, y.d, ffma(x.c, y.c, sum2<W>(x.a, y.a, x.b, y.b)));
+}
+// qmul with its products' roundings pinned: in the vector part, the second
+// product of each x.a y.v + x.v y.a is the fused one with W = 2
+template <int W, typename T>
+__device__ __forceinline__ Q<T> qmul_w(const Q<T> &x, const Q<T> &y) {
+  Q<T> r;
+  r.a = ffma(-x.d, y.d, ffma(-x.c, y.c, ffma(x.a, y.a, -(x.b * y.b))));
+  r.b = sum2<W>(x.a, y.b, x.b, y.a) - ffma(x.c, y.d, -(x.d * y.c));
+  r.c = sum2<W>(x.a, y.c, x.c, y.a) - ffma(x.d, y.b, -(x.b * y.d));
+  r.d = sum2<W>(x.a, y.d, x.d, y.a) - ffma(x.b, y.c, -(x.c * y.b));
+  return r;
+}
 // exp(-i alpha sigma_3) as a quaternion (src/staples.c:161-177)
 template <typename T>
 __device__ __forceinline__ Q<T> u1twist(T alpha) {
@@ -161,6 +187,10 @@ template <typename T>
 struct V3 {
   T x, y, z;
 };
+template <int W, typename T>
+__device__ __forceinline__ T vdot_w(const V3<T> &x, const V3<T> &y) {
+  return ffma(x.z, y.z, sum2<W>(x.x, y.x, x.y, y.y));
+}
 // R(U) v = vector part of U (0,v) U^dagger
 template <typename T>
 __device__ __forceinline__ V3<T> rotate(const Q<T> &u, const V3<T> &v) {

@@ -25,6 +25,7 @@
 namespace su2 {
 
 constexpr int BLK = 256;          // threads per workgroup in every site kernel
+constexpr unsigned NXCD = 8;      // chiplets: workgroup b goes to XCD b % NXCD, each with its own L2
 constexpr int NCOUNT = 12;        // counter rows: pass kinds SU2HIP_K_LINK_HEATBATH .. SINGLET_METROPOLIS,
                                   // then the second doublet's two kinds
 constexpr int CNT_DOUBLET2_OR = 10;
@@ -130,6 +131,7 @@ struct LaunchCtx {
   MucaDev *muca;       // device, [max_slots]
   const BlockMap *blk; // device, [nblk]
   int nblk;
+  int one = -1;        // the slot of the handle's only lattice, else -1
   long long *cnt;      // device, [NCOUNT][2][nblk]
   double *partial;     // device, [nblk][SU2HIP_NSUMS]
   double *sums;        // device, [max_slots][SU2HIP_NSUMS]

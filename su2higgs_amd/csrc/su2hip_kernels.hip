@@ -117,6 +117,12 @@ __device__ __forceinline__ Q<T> link_staple(const LatDesc &L, const T *U, const 
   return V;
 }
 
+// the fused product of a link staple's norm (sum2)
+template <typename T, int M>
+constexpr int staple_norm_w() {
+  return (M & M_H2) != 0 && (sizeof(T) == 4 || (M & M_U1) != 0) ? 2 : 1;
+}
+
 // staple_doublet (src/staples.c:243-302)
 template <typename T, int M>
 __device__ __forceinline__ void doublet_hops(const LatDesc &L, const T *U, const T *A, const T *F,
@@ -262,6 +268,8 @@ __device__ __forceinline__ Q<double> qd(const Q<T> &q) {
 
 // higgspotential of two doublets (src/su2u1.c:528-554), f1 = phi_1 and
 // f2 = phi_2 at one site
+// (W: the fused product of its last sum, sum2)
+template <int W = 1>
 __device__ __forceinline__ double pot2(const LatDesc &L, const Q<double> &h1, const Q<double> &h2) {
   double f11 = 0.5 * qdot(h1, h1), f22 = 0.5 * qdot(h2, h2);
   // get_phi12 (src/su2u1.c:513-520)
@@ -270,7 +278,7 @@ __device__ __forceinline__ double pot2(const LatDesc &L, const Q<double> &h1, co
   return L.msq * f11 + L.lambda * f11 * f11 + L.msq2 * f22 + L.m12re * R - L.m12im * I +
          L.lam2 * f22 * f22 + L.lam3 * f11 * f22 + L.lam4 * (R * R + I * I) +
          L.lam5re * (R * R - I * I) - 2.0 * L.lam5im * R * I + f11 * (L.lam6re * R - L.lam6im * I) +
-         f22 * (L.lam7re * R + L.lam7im * I);
+         f22 * sum2<W>(L.lam7re, R, L.lam7im, I);
 }
 
 // overrelax_higgs2's move (src/overrelax.c:295-417) for doublet h of two:
@@ -304,7 +312,7 @@ __device__ __forceinline__ void higgs2_or(const LatDesc &L, int h, const Q<doubl
   double cH = 0.5 * (L.m12re + Hsq * l67re), cG = 0.5 * (-1.0 * L.m12im + Hsq * l67im);
   Q<double> s{-(st.a + cH * H.a + cG * G.a), -(st.b + cH * H.b + cG * G.b),
               -(st.c + cH * H.c + cG * G.c), -(st.d + cH * H.d + cG * G.d)};
-  double F = ::sqrt(qdot(s, s));
+  double F = ::sqrt(qdot_w<1>(s, s));
   e = Q<double>{s.a / F, s.b / F, s.c / F, s.d / F};
   X = qdot(f, e);
   Q<double> Y{f.a - X * e.a, f.b - X * e.b, f.c - X * e.c, f.d - X * e.d};
@@ -478,13 +486,14 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
       oldact = hop_triplet(old, a1, a2);
     }
     Q<T> V = link_staple<T, M>(L, U, A, F, x, mu);
+    constexpr int WV = staple_norm_w<T, M>();
     T r1, r2, r3, d, a0;
     int loop = 1;
     // a full wavefront shares the FP64 direction's rejection tries
     // (hb_dir_wave); the results are those of the per-lane loop
     const bool wave = sizeof(T) == 8 && __ballot(1) == ~0ull;
     if constexpr (sizeof(T) == 8) {
-      T a = ::sqrt(qdot(V, V));
+      T a = ::sqrt(qdot_w<WV>(V, V));
       V = qscale(V, (T)-1 / a);
       a *= (T)2;
       do {
@@ -498,7 +507,7 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
       } while (r3 * r3 > (T)1 - (T)0.5 * d && loop <= 200);
     } else {
       // the same Kennedy-Pendleton loop on the hardware log/cos
-      T ia = frsqrt(qdot(V, V));
+      T ia = frsqrt(qdot_w<WV>(V, V));
       V = qscale(V, -ia);
       ia *= (T)0.5;  // 1 / (2 |V|)
       do {
@@ -572,7 +581,7 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
     } else {
       R = qscale(R, frsqrt(qdot(R, R)));
     }
-    Q<T> nu = qmul(old, R);
+    Q<T> nu = qmul_w<2>(old, R);
     (void)reunit;  // FP32 links are renormalised by their packed storage
     Q<T> du{nu.a - old.a, nu.b - old.b, nu.c - old.c, nu.d - old.d};
     T diff = (T)2 * qmul(du, V).a;
@@ -589,13 +598,14 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
     // hopping term as in src/heatbath.c:107-120
     Q<T> old = ldU<M>(U, Vh, mu, par, s);
     Q<T> V = link_staple<T, M>(L, U, A, F, x, mu);
+    constexpr int WV = staple_norm_w<T, M>();
     Q<T> w;
     if constexpr (sizeof(T) == 8) {
-      T a = ::sqrt(qdot(V, V));
+      T a = ::sqrt(qdot_w<WV>(V, V));
       if (a == (T)0) return 1;
       w = qconj(Q<T>{V.a / a, V.b / a, V.c / a, V.d / a});
     } else {
-      T n2 = qdot(V, V);
+      T n2 = qdot_w<WV>(V, V);
       if (n2 == (T)0) return 1;
       w = qconj(qscale(V, frsqrt(n2)));
     }
@@ -702,11 +712,12 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
       nf = Q<T>{ft.a + (T)1 * (uni<T>(r) - (T)0.5), ft.b + (T)1 * (uni<T>(r) - (T)0.5),
                 ft.c + (T)1 * (uni<T>(r) - (T)0.5), ft.d + (T)1 * (uni<T>(r) - (T)0.5)};
       Q<double> n = qd(nf);
-      double o2 = qdot(f, f), n2 = qdot(n, n);
+      constexpr int W = sizeof(T) == 4 ? 2 : 1;
+      double o2 = qdot_w<1>(f, f), n2 = qdot_w<W>(n, n);
       double pn = mu ? pot2(L, H, n) : pot2(L, n, H);
-      double po = mu ? pot2(L, H, f) : pot2(L, f, H);
-      double diff = (n.a - f.a) * st.a + (n.b - f.b) * st.b + (n.c - f.c) * st.c +
-                    (n.d - f.d) * st.d + 3.0 * (n2 - o2) + (pn - po);
+      double po = mu ? pot2<W>(L, H, f) : pot2<W>(L, f, H);
+      double diff = qdot_w<W>(Q<double>{n.a - f.a, n.b - f.b, n.c - f.c, n.d - f.d}, st) +
+                    3.0 * (n2 - o2) + (pn - po);
       if (!metro_accept((T)diff, r)) return 0;
     }
     stF(Fh, Vh, par, s, nf);
@@ -760,9 +771,10 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
       // localact_doublet = (f'-f).s + B(|f'|^2-|f|^2) + C(|f'|^4-|f|^4)
       nf = Q<T>{f.a + (T)1 * (uni<T>(r) - (T)0.5), f.b + (T)1 * (uni<T>(r) - (T)0.5),
                 f.c + (T)1 * (uni<T>(r) - (T)0.5), f.d + (T)1 * (uni<T>(r) - (T)0.5)};
-      T o2 = qdot(f, f), n2 = qdot(nf, nf);
-      T diff = (nf.a - f.a) * st.a + (nf.b - f.b) * st.b + (nf.c - f.c) * st.c +
-               (nf.d - f.d) * st.d + (T)B0 * (n2 - o2) + (T)C * (n2 * n2 - o2 * o2);
+      constexpr int W = sizeof(T) == 4 ? 2 : 1;
+      T o2 = qdot_w<1>(f, f), n2 = qdot_w<W>(nf, nf);
+      T diff = qdot_w<W>(Q<T>{nf.a - f.a, nf.b - f.b, nf.c - f.c, nf.d - f.d}, st) +
+               (T)B0 * (n2 - o2) + (T)C * (n2 * n2 - o2 * o2);
       if (!metro_accept(diff, r)) return 0;
     }
     stF(F, Vh, par, s, nf);
@@ -811,8 +823,9 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
       }
       ng = V3<T>{g.x + (T)1 * (uni<T>(r) - (T)0.5), g.y + (T)1 * (uni<T>(r) - (T)0.5),
                  g.z + (T)1 * (uni<T>(r) - (T)0.5)};
-      T o2 = g.x * g.x + g.y * g.y + g.z * g.z, n2 = ng.x * ng.x + ng.y * ng.y + ng.z * ng.z;
-      T diff = (ng.x - g.x) * st.x + (ng.y - g.y) * st.y + (ng.z - g.z) * st.z +
+      constexpr int W = sizeof(T) == 4 ? 2 : 1;
+      T o2 = vdot_w<1>(g, g), n2 = vdot_w<W>(ng, ng);
+      T diff = vdot_w<W>(V3<T>{ng.x - g.x, ng.y - g.y, ng.z - g.z}, st) +
                (T)B0 * (n2 - o2) + (T)C * (n2 * n2 - o2 * o2);
       if (!metro_accept(diff, r)) return 0;
     }
@@ -926,17 +939,60 @@ __device__ __forceinline__ double orderparam_at(const LatDesc &L, int op, int pa
 // ------------------------------------------------------------------------
 // the pass kernel
 
+// *p += n, for counters only this workgroup touches during the kernel (so
+// the workgroup's scope is enough: the XCD's own L2 adds)
+__device__ __forceinline__ void count_up(long long *p, int n) {
+  __hip_atomic_fetch_add(p, (long long)n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// The start and the end of a pass decide its small cases: a wavefront of a
+// 64^3 pass lives 4.8 us of which 0.6 us is arithmetic, the rest a chain of
+// latencies.  Before, four to six scalar loads waited for one another (block
+// table, descriptor, active, budget, extents, field pointers) and two
+// barriers and a read-modify-write of the counters ended each workgroup.
+// With the batch of loads below, no table for one lattice and counters added
+// by atomics that return nothing, graph-replayed sweeps (us, one GPU
+// session, before -> after): FP32 32^3 166 -> 138, 64^3 217 -> 181, 96^3
+// SU(2)xU(1) 525 -> 454, 144^3 1333 -> 1261, 32-lattice scan 660 -> 616; FP64
+// 96^3 1097 -> 1037.
+
+// The block-table entry of this workgroup.  A handle with one lattice
+// (one >= 0) computes it: the table deals workgroup j + 8k to XCD j, whose
+// run of chunks is contiguous (deal_to_xcds on the host), and a dependent
+// load before the descriptor's costs a whole memory latency per workgroup.
+__device__ __forceinline__ BlockMap block_of(const BlockMap *__restrict__ blk, int nblk, int one,
+                                             int chunk) {
+  if (one < 0) return blk[blockIdx.x];
+  const int j = (int)(blockIdx.x % NXCD), k = (int)(blockIdx.x / NXCD);
+  const int q = nblk / (int)NXCD, r = nblk % (int)NXCD;
+  return BlockMap{one, (j * q + (j < r ? j : r) + k) * chunk};
+}
+
+// Everything of the descriptor a pass of this kind reads before its field
+// loads, in registers here: one batch of scalar loads in flight together
+// instead of one per branch that needs them.
+template <int M, int KIND>
+__device__ __forceinline__ void pin_desc(const LatDesc &L) {
+  asm volatile("" ::"s"(L.U), "s"(L.Vh), "s"(L.h0), "s"(L.L0), "s"(L.L1), "s"(L.L2),
+               "s"(L.div_h0.m), "s"(L.div_h0.l), "s"(L.div_L1.m), "s"(L.div_L1.l), "s"(L.key0),
+               "s"(L.key1), "s"(L.pass), "s"(L.active), "s"(L.budget));
+  if constexpr ((M & M_NH) != 0) asm volatile("" ::"s"(L.F), "s"(L.H));
+  if constexpr ((M & M_U1) != 0) asm volatile("" ::"s"(L.A));
+  if constexpr (KIND <= SU2HIP_K_LINK_OVERRELAX) asm volatile("" ::"s"(L.beta));
+}
+
 template <typename T, int M, int KIND>
 __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
                                           const MucaDev *__restrict__ mucas,
-                                          const BlockMap *__restrict__ blk, int par_in, int mu_in,
-                                          int pass_off, int step, int reunit,
+                                          const BlockMap *__restrict__ blk, int one, int chunk,
+                                          int par_in, int mu_in, int pass_off, int step, int reunit,
                                           long long *__restrict__ cnt, int nblk,
                                           double *__restrict__ partial,
                                           const uint8_t *__restrict__ order, int npass,
                                           double *lds) {
-  const BlockMap bm = blk[blockIdx.x];
-  const LatDesc &L = lats[bm.lat];
+  const BlockMap bm = block_of(blk, nblk, one, chunk);
+  const LatDesc L = lats[bm.lat];
+  pin_desc<M, KIND>(L);
   if (!L.active || L.budget == 0) return;
   int par = par_in, mu = mu_in;
   if (order) {
@@ -990,16 +1046,17 @@ __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
       acc = site_update<T, M, KIND>(L, x, par, s, mu, r, reunit);
     }
   }
-  int nacc = __syncthreads_count(acc);
-  int ntot = __syncthreads_count(upd);
-  if (threadIdx.x == 0) {
+  // counted wavefront by wavefront with atomics that return nothing: no
+  // barrier and no load to wait for before the wavefront ends
+  const uint64_t am = __ballot(acc), tm = __ballot(upd);
+  if ((threadIdx.x & 63) == 0 && tm) {
     int row = KIND;
     if constexpr ((M & M_H2) != 0 && KIND == SU2HIP_K_DOUBLET_OVERRELAX)
       row = mu ? CNT_DOUBLET2_OR : KIND;
     if constexpr ((M & M_H2) != 0 && KIND == SU2HIP_K_DOUBLET_METROPOLIS)
       row = mu ? CNT_DOUBLET2_METRO : KIND;
-    cnt[(size_t)(row * 2 + 0) * nblk + blockIdx.x] += nacc;
-    cnt[(size_t)(row * 2 + 1) * nblk + blockIdx.x] += ntot;
+    count_up(&cnt[(size_t)(row * 2 + 0) * nblk + blockIdx.x], __popcll(am));
+    count_up(&cnt[(size_t)(row * 2 + 1) * nblk + blockIdx.x], __popcll(tm));
   }
   if (muca) {
     double v = valid ? orderparam_at<T, M>(L, op, par, s) : 0.0;
@@ -1010,14 +1067,14 @@ __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
 
 #define K_PASS_ARGS                                                                          \
   const LatDesc *__restrict__ lats, const MucaDev *__restrict__ mucas,                       \
-      const BlockMap *__restrict__ blk, int par_in, int mu_in, int pass_off, int step,       \
-      int reunit, long long *__restrict__ cnt, int nblk, double *__restrict__ partial,       \
+      const BlockMap *__restrict__ blk, int one, int chunk, int par_in, int mu_in,           \
+      int pass_off, int step, int reunit, long long *__restrict__ cnt, int nblk, double *__restrict__ partial,       \
       const uint8_t *__restrict__ order, int npass
 
 template <typename T, int M, int KIND>
 __global__ __launch_bounds__(BLK) void k_pass(K_PASS_ARGS) {
   __shared__ double lds[BLK / 64];
-  pass_body<T, M, KIND>(lats, mucas, blk, par_in, mu_in, pass_off, step, reunit, cnt, nblk,
+  pass_body<T, M, KIND>(lats, mucas, blk, one, chunk, par_in, mu_in, pass_off, step, reunit, cnt, nblk,
                         partial, order, npass, lds);
 }
 
@@ -1030,7 +1087,7 @@ template <typename T, int M, int KIND>
 __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(5))) void k_pass_w5(
     K_PASS_ARGS) {
   __shared__ double lds[BLK / 64];
-  pass_body<T, M, KIND>(lats, mucas, blk, par_in, mu_in, pass_off, step, reunit, cnt, nblk,
+  pass_body<T, M, KIND>(lats, mucas, blk, one, chunk, par_in, mu_in, pass_off, step, reunit, cnt, nblk,
                         partial, order, npass, lds);
 }
 
@@ -1042,9 +1099,10 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(5))) void k
 // sincos once per round instead of once per pass.
 template <typename T, int M>
 __global__ __launch_bounds__(BLK) void k_hop(const LatDesc *__restrict__ lats,
-                                             const BlockMap *__restrict__ blk) {
-  const BlockMap bm = blk[blockIdx.x];
-  const LatDesc &L = lats[bm.lat];
+                                             const BlockMap *__restrict__ blk, int nblk, int one) {
+  const BlockMap bm = block_of(blk, nblk, one, BLK);
+  const LatDesc L = lats[bm.lat];
+  pin_desc<M, SU2HIP_K_AUX>(L);
   if (!L.active || L.budget == 0 || !L.H) return;
   const int s = bm.s0 + (int)threadIdx.x;
   if (s >= L.Vh) return;
@@ -2219,8 +2277,6 @@ constexpr int FLOW_GROUPS = 6;
 // share the entry's neighbourhood in one L2 instead of fetching it into six
 // of them (2.7x the algorithmic bytes when consecutive blocks took the six
 // groups of one entry).
-constexpr unsigned NXCD = 8;
-
 constexpr unsigned flow_grid(unsigned n) {
   return FLOW_GROUPS * NXCD * ((n + NXCD - 1) / NXCD);
 }
@@ -2362,11 +2418,11 @@ static hipError_t pass_one(const LaunchCtx &c, int parity, int dir, int pass_off
       if (c.waves == 5) {
         if (c.ev_start || c.ev_stop) {
           hipExtLaunchKernelGGL((k_pass_w5<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream,
-                                c.ev_start, c.ev_stop, 0, c.desc, c.muca, c.blk, parity, dir,
+                                c.ev_start, c.ev_stop, 0, c.desc, c.muca, c.blk, c.one, c.block, parity, dir,
                                 pass_off, step, reunit, c.cnt, c.nblk, c.partial, c.order, c.npass);
         } else {
           hipLaunchKernelGGL((k_pass_w5<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream,
-                             c.desc, c.muca, c.blk, parity, dir, pass_off, step, reunit, c.cnt,
+                             c.desc, c.muca, c.blk, c.one, c.block, parity, dir, pass_off, step, reunit, c.cnt,
                              c.nblk, c.partial, c.order, c.npass);
         }
         return hipGetLastError();
@@ -2374,11 +2430,11 @@ static hipError_t pass_one(const LaunchCtx &c, int parity, int dir, int pass_off
     }
     if (c.ev_start || c.ev_stop) {
       hipExtLaunchKernelGGL((k_pass<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream,
-                            c.ev_start, c.ev_stop, 0, c.desc, c.muca, c.blk, parity, dir, pass_off,
+                            c.ev_start, c.ev_stop, 0, c.desc, c.muca, c.blk, c.one, c.block, parity, dir, pass_off,
                             step, reunit, c.cnt, c.nblk, c.partial, c.order, c.npass);
     } else {
       hipLaunchKernelGGL((k_pass<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream, c.desc,
-                         c.muca, c.blk, parity, dir, pass_off, step, reunit, c.cnt, c.nblk,
+                         c.muca, c.blk, c.one, c.block, parity, dir, pass_off, step, reunit, c.cnt, c.nblk,
                          c.partial, c.order, c.npass);
     }
     return hipGetLastError();
@@ -2417,7 +2473,8 @@ hipError_t launch_hop(const LaunchCtx &c) {
     return with_model_of<T>(c.model, [&](auto m) -> hipError_t {
       constexpr int M = decltype(m)::value;
       if constexpr (hop_cached<M>()) {
-        hipLaunchKernelGGL((k_hop<T, M>), dim3(c.nblk), dim3(BLK), 0, c.stream, c.desc, c.blk);
+        hipLaunchKernelGGL((k_hop<T, M>), dim3(c.nblk), dim3(BLK), 0, c.stream, c.desc, c.blk,
+                           c.nblk, c.one);
         return hipGetLastError();
       }
       return hipSuccess;
