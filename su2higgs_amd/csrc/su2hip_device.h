@@ -2,6 +2,8 @@
 // kernels (gfx950).  Included by su2hip_kernels.hip only.
 #pragma once
 
+#include <type_traits>
+
 #include "su2hip_internal.h"
 
 namespace su2 {
@@ -143,15 +145,16 @@ template <int W, typename T>
 __device__ __forceinline__ T qdot_w(const Q<T> &x, const Q<T> &y) {
   return ffma(x.d, y.d, ffma(x.c, y.c, sum2<W>(x.a, y.a, x.b, y.b)));
 }
-// qmul with its products' roundings pinned: in the vector part, the second
-// product of each x.a y.v + x.v y.a is the fused one with W = 2
-template <int W, typename T>
+// qmul with its products' roundings pinned, by the fused product of: the real
+// part's first sum (A), and in the vector part each x.a y.v + x.v y.a (W)
+// and each cross product term (V)
+template <int W, int A = 1, int V = 1, typename T>
 __device__ __forceinline__ Q<T> qmul_w(const Q<T> &x, const Q<T> &y) {
   Q<T> r;
-  r.a = ffma(-x.d, y.d, ffma(-x.c, y.c, ffma(x.a, y.a, -(x.b * y.b))));
-  r.b = sum2<W>(x.a, y.b, x.b, y.a) - ffma(x.c, y.d, -(x.d * y.c));
-  r.c = sum2<W>(x.a, y.c, x.c, y.a) - ffma(x.d, y.b, -(x.b * y.d));
-  r.d = sum2<W>(x.a, y.d, x.d, y.a) - ffma(x.b, y.c, -(x.c * y.b));
+  r.a = ffma(-x.d, y.d, ffma(-x.c, y.c, sum2<A>(x.a, y.a, -x.b, y.b)));
+  r.b = sum2<W>(x.a, y.b, x.b, y.a) - sum2<V>(x.c, y.d, -x.d, y.c);
+  r.c = sum2<W>(x.a, y.c, x.c, y.a) - sum2<V>(x.d, y.b, -x.b, y.d);
+  r.d = sum2<W>(x.a, y.d, x.d, y.a) - sum2<V>(x.b, y.c, -x.c, y.b);
   return r;
 }
 // exp(-i alpha sigma_3) as a quaternion (src/staples.c:161-177)
@@ -395,6 +398,34 @@ __device__ __forceinline__ void stU(T *__restrict__ U, int Vh, int d, int par, i
                  __builtin_fmaf(q.d, e, q.d)});
   } else {
     st4(U + ((size_t)(d * 2 + par) * Vh + s) * 4, q);
+  }
+}
+// The same with the (direction, parity) run of links as a uniform base and a
+// 32-bit byte offset (a run is at most 2^27 links of 32 bytes): one
+// instruction of address arithmetic per load instead of five.
+template <int M, typename T>
+__device__ __forceinline__ const T *link_run(const T *U, int Vh, int d, int par) {
+  return U + (size_t)(d * 2 + par) * Vh * (packed_links<M, T>() ? 3 : 4);
+}
+// a link as it is stored, loaded now and rebuilt where it is used
+template <int M, typename T>
+struct LinkRaw {
+  std::conditional_t<packed_links<M, T>(), F3, Q<T>> w;
+  __device__ __forceinline__ Q<T> get() const {
+    if constexpr (packed_links<M, T>())
+      return link_unpack(w);
+    else
+      return w;
+  }
+};
+template <int M, typename T>
+__device__ __forceinline__ LinkRaw<M, T> ldL(const T *run, int s) {
+  const char *b = reinterpret_cast<const char *>(run);
+  if constexpr (packed_links<M, T>()) {
+    gptr<const float> p = gmem(reinterpret_cast<const float *>(b + (size_t)((uint32_t)s * 12u)));
+    return LinkRaw<M, T>{F3{p[0], p[1], p[2]}};
+  } else {
+    return LinkRaw<M, T>{ld4(reinterpret_cast<const T *>(b + (size_t)((uint32_t)s * (uint32_t)(4 * sizeof(T)))))};
   }
 }
 template <typename T>

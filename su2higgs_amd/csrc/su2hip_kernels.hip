@@ -86,6 +86,34 @@ __device__ __forceinline__ Q<T> wilson_staple(const LatDesc &L, const T *U, cons
   return W;
 }
 
+// wilson_staple of the update passes, with the direction a constant: the six
+// links of one transverse direction, loaded together and multiplied later.
+// The roundings are pinned (sum2) to those of wilson_staple inlined there.
+template <typename T, int M, int MU, int NU>
+struct StapleLinks {
+  LinkRaw<M, T> xp, xn, x0, xpm, xm_mu, xm;
+  __device__ __forceinline__ void load(const LatDesc &L, const T *U, const Site &x, const Site &sp) {
+    const int op = x.par ^ 1;
+    const T *mu_o = link_run<M>(U, L.Vh, MU, op);
+    const T *nu_s = link_run<M>(U, L.Vh, NU, x.par), *nu_o = link_run<M>(U, L.Vh, NU, op);
+    const Site sn = shift(L, x, NU, +1), sm = shift(L, x, NU, -1), spm = shift(L, sp, NU, -1);
+    xp = ldL<M>(nu_o, sp.s);
+    xn = ldL<M>(mu_o, sn.s);
+    x0 = ldL<M>(nu_s, x.s);
+    xpm = ldL<M>(nu_s, spm.s);
+    xm_mu = ldL<M>(mu_o, sm.s);
+    xm = ldL<M>(nu_o, sm.s);
+  }
+  __device__ __forceinline__ void add_to(Q<T> &W) const {
+    // a stored four-component link enters conjugated by a sign, a packed one
+    // through its rebuilt components
+    constexpr bool pk = packed_links<M, T>();
+    constexpr int W1 = pk ? 1 : 2, V1 = pk ? 1 : 2, A2 = !pk && sizeof(T) == 4 ? 2 : 1;
+    W = qadd(W, qmul_w<2, A2, V1>(qmul_w<W1, 1, V1>(xp.get(), qconj(xn.get())), qconj(x0.get())));
+    W = qadd(W, qmul_w<2>(qmul_w<1>(qconj(xpm.get()), qconj(xm_mu.get())), xm.get()));
+  }
+};
+
 // With one doublet the hopping term of the staple is read from the cache
 // k_hop fills (the same arithmetic, done once per round of link passes),
 // when the handle keeps one (LatDesc::H not null).
@@ -104,15 +132,78 @@ __device__ __forceinline__ Q<T> hop_term(const LatDesc &L, const T *A, const T *
   return qscale(t, (T)-0.5);
 }
 
+// The SU(2) link kinds built with a constant direction (one copy each).  FP64
+// with a doublet keeps the run-time direction: constant, it holds 118
+// registers instead of 94 (four wavefronts per SIMD) or spills, and the 96^3
+// overrelaxation takes 26.8 us instead of 18.9.
 template <typename T, int M>
+constexpr bool const_dir() {
+  return sizeof(T) == 4 || (M & M_NH) == 0;
+}
+
+// su2link_staple and the link itself.  With a constant direction FP32 issues
+// every load of the site before any arithmetic, so that a wavefront waits
+// for one memory latency and not for three (sweeps, us: 32^3 138 -> 130-133,
+// 32-lattice scan 616 -> 583; 96^3 overrelaxation 9.3 -> 8.5 of which 1.8 is
+// an empty launch and 6.5 its 45 MB at the fabric's 7 TB/s); FP64 takes the transverse
+// directions one at a time, whose registers leave room for more wavefronts.
+template <typename T, int M, int MU>
 __device__ __forceinline__ Q<T> link_staple(const LatDesc &L, const T *U, const T *A, const T *F,
-                                            const Site &x, int mu) {
+                                            const Site &x, Q<T> &old) {
+  constexpr int N1 = MU == 0 ? 1 : 0, N2 = MU == 2 ? 1 : 2;
+  const Site sp = shift(L, x, MU, +1);
+  Q<T> W{(T)0, (T)0, (T)0, (T)0};
+  StapleLinks<T, M, MU, N1> s1;
+  StapleLinks<T, M, MU, N2> s2;
+  s1.load(L, U, x, sp);
+  if constexpr (sizeof(T) == 8) {
+    s1.add_to(W);
+    asm volatile("" : "+v"(W.a), "+v"(W.b), "+v"(W.c), "+v"(W.d) : : "memory");
+  }
+  s2.load(L, U, x, sp);
+  const auto o = ldL<M>(link_run<M>(U, L.Vh, MU, x.par), x.s);
+  // the cached hopping term, or the doublet it is formed from
+  Q<T> h{(T)0, (T)0, (T)0, (T)0}, fp = h;
+  T al = (T)0;
+  if constexpr ((M & M_NH) != 0) {
+    const bool cached = hop_cached<M>() && L.H;
+    h = ldF(cached ? (const T *)L.H + (size_t)MU * 8 * L.Vh : F, L.Vh, x.par, x.s);
+    if (!cached) {
+      fp = F_at(L, F, sp);
+      if constexpr ((M & M_U1) != 0) al = A_at(L, A, x, MU);
+    }
+  }
+  if constexpr (sizeof(T) == 4) {
+    __builtin_amdgcn_sched_barrier(0);
+    s1.add_to(W);
+  }
+  s2.add_to(W);
+  old = o.get();
+  const T k = (T)(-0.5 * L.beta);
+  if constexpr ((M & M_NH) == 0) {
+    return qscale(W, k);
+  } else {
+    if (!(hop_cached<M>() && L.H)) {
+      if constexpr ((M & M_U1) != 0) fp = qmul_u1(fp, u1twist<T>(al));
+      h = qscale(qmul(fp, qconj(h)), (T)-0.5);
+    }
+    // -beta/2 W + the first doublet's term, one rounding
+    Q<T> V{ffma(W.a, k, h.a), ffma(W.b, k, h.b), ffma(W.c, k, h.c), ffma(W.d, k, h.d)};
+    // the second doublet's (the doublet loop of src/staples.c:150-190)
+    if constexpr ((M & M_H2) != 0) V = qadd(V, hop_term<T, M>(L, A, (const T *)L.F2, x, MU));
+    return V;
+  }
+}
+
+// the same with the direction at run time
+template <typename T, int M>
+__device__ __forceinline__ Q<T> link_staple_rt(const LatDesc &L, const T *U, const T *A, const T *F,
+                                               const Site &x, int mu, Q<T> &old) {
+  old = ldU<M>(U, L.Vh, mu, x.par, x.s);
   Q<T> V = qscale(wilson_staple<T, M>(L, U, x, mu), (T)(-0.5 * L.beta));
   if constexpr (hop_cached<M>())
     if (L.H) return qadd(V, ld4((const T *)L.H + ((size_t)(mu * 2 + x.par) * L.Vh + x.s) * 4));
   if constexpr ((M & M_NH) != 0) V = qadd(V, hop_term<T, M>(L, A, F, x, mu));
-  // the second doublet's hopping term (the doublet loop of
-  // src/staples.c:150-190)
   if constexpr ((M & M_H2) != 0) V = qadd(V, hop_term<T, M>(L, A, (const T *)L.F2, x, mu));
   return V;
 }
@@ -464,9 +555,12 @@ struct Fields {
   void *U, *A, *F, *G, *S, *B;
 };
 
-template <typename T, int M, int KIND>
-__device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int par, int s, int mu,
+// MU: the direction of an SU(2) link kind (-1 for the others, which take it
+// or the doublet from mu)
+template <typename T, int M, int KIND, int MU>
+__device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int par, int s, int mu_in,
                                            Rng &r, int reunit) {
+  const int mu = MU >= 0 ? MU : mu_in;
   T *U = (T *)L.U;
   T *A = (T *)L.A;
   T *F = (T *)L.F;
@@ -476,16 +570,19 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
 
   if constexpr (KIND == SU2HIP_K_LINK_HEATBATH) {
     // heatbath_su2link (src/heatbath.c:15-124), Kennedy-Pendleton
-    Q<T> old{};
+    Q<T> old;
     T oldact = 0;
     V3<T> a1{}, a2{};
     if constexpr ((M & M_TR) != 0) {
-      old = ldU<M>(U, Vh, mu, par, s);
       a1 = ldG(G, Vh, par, s);
       a2 = G_at(L, G, shift(L, x, mu, +1));
-      oldact = hop_triplet(old, a1, a2);
     }
-    Q<T> V = link_staple<T, M>(L, U, A, F, x, mu);
+    Q<T> V;
+    if constexpr (MU >= 0)
+      V = link_staple<T, M, MU>(L, U, A, F, x, old);
+    else
+      V = link_staple_rt<T, M>(L, U, A, F, x, mu, old);
+    if constexpr ((M & M_TR) != 0) oldact = hop_triplet(old, a1, a2);
     constexpr int WV = staple_norm_w<T, M>();
     T r1, r2, r3, d, a0;
     int loop = 1;
@@ -568,8 +665,12 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
   } else if constexpr (KIND == SU2HIP_K_LINK_METROPOLIS) {
     // metro_su2link (src/metropolis.c:15-41), random_su2link (src/init.c:43-58);
     // Delta S = 2 Re[(U'-U) V]_0 + Delta(triplet hop), from the staple
-    Q<T> old = ldU<M>(U, Vh, mu, par, s);
-    Q<T> V = link_staple<T, M>(L, U, A, F, x, mu);
+    Q<T> old;
+    Q<T> V;
+    if constexpr (MU >= 0)
+      V = link_staple<T, M, MU>(L, U, A, F, x, old);
+    else
+      V = link_staple_rt<T, M>(L, U, A, F, x, mu, old);
     Q<T> R;
     R.a = (T)10 * (uni<T>(r) - (T)0.5);
     R.b = (T)1 * (uni<T>(r) - (T)0.5);
@@ -596,8 +697,12 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
     // SU(2) link overrelaxation, U' = W^+ U^+ W^+ with W = staple/|staple|
     // (no reference counterpart); with a triplet a Metropolis test on its
     // hopping term as in src/heatbath.c:107-120
-    Q<T> old = ldU<M>(U, Vh, mu, par, s);
-    Q<T> V = link_staple<T, M>(L, U, A, F, x, mu);
+    Q<T> old;
+    Q<T> V;
+    if constexpr (MU >= 0)
+      V = link_staple<T, M, MU>(L, U, A, F, x, old);
+    else
+      V = link_staple_rt<T, M>(L, U, A, F, x, mu, old);
     constexpr int WV = staple_norm_w<T, M>();
     Q<T> w;
     if constexpr (sizeof(T) == 8) {
@@ -960,11 +1065,27 @@ __device__ __forceinline__ void count_up(long long *p, int n) {
 // (one >= 0) computes it: the table deals workgroup j + 8k to XCD j, whose
 // run of chunks is contiguous (deal_to_xcds on the host), and a dependent
 // load before the descriptor's costs a whole memory latency per workgroup.
+//
+// rev: each XCD takes its run from the end, on every other pass.  The L2s
+// (4 MB per XCD) keep their lines from one launch to the next, and a pass
+// streams more than they hold, so in one fixed order a pass evicts every
+// line before the next pass asks for it; turning round, the next pass begins
+// with the lines the last one left.  Large passes are bound by what crosses
+// the fabric to the Infinity Cache (7 TB/s, as a plain read of the same
+// bytes), so each hit is time: sweeps (us, fixed order -> alternating, one
+// GPU session) FP32 96^3 468 -> 448, 144^3 1253 -> 1186, 32-lattice scan
+// 597 -> 545; FP64 four 48^3 adjoint lattices 530 -> 500, 96^3 1037 -> 980;
+// no change below 32 MB of fields.
+//
+// idx is the entry's place in the table (its counters' row).
 __device__ __forceinline__ BlockMap block_of(const BlockMap *__restrict__ blk, int nblk, int one,
-                                             int chunk) {
-  if (one < 0) return blk[blockIdx.x];
-  const int j = (int)(blockIdx.x % NXCD), k = (int)(blockIdx.x / NXCD);
+                                             int chunk, int rev, int &idx) {
+  const int j = (int)(blockIdx.x % NXCD);
+  int k = (int)(blockIdx.x / NXCD);
   const int q = nblk / (int)NXCD, r = nblk % (int)NXCD;
+  if (rev) k = q + (j < r ? 1 : 0) - 1 - k;
+  idx = j + k * (int)NXCD;
+  if (one < 0) return blk[idx];
   return BlockMap{one, (j * q + (j < r ? j : r) + k) * chunk};
 }
 
@@ -990,7 +1111,8 @@ __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
                                           double *__restrict__ partial,
                                           const uint8_t *__restrict__ order, int npass,
                                           double *lds) {
-  const BlockMap bm = block_of(blk, nblk, one, chunk);
+  int idx;
+  const BlockMap bm = block_of(blk, nblk, one, chunk, pass_off & 1, idx);
   const LatDesc L = lats[bm.lat];
   pin_desc<M, KIND>(L);
   if (!L.active || L.budget == 0) return;
@@ -1030,20 +1152,20 @@ __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
     Site x = site_of(L, par, s);
     Rng r;
     rng_init(r, L.key0, L.key1, L.pass + (uint64_t)pass_off, (uint32_t)(par * L.Vh + s));
-    if constexpr (KIND == SU2HIP_K_U1_METROPOLIS && sizeof(T) == 4) {
+    if constexpr ((KIND <= SU2HIP_K_LINK_OVERRELAX && const_dir<T, M>()) ||
+                  (KIND == SU2HIP_K_U1_METROPOLIS && sizeof(T) == 4)) {
       // one inlined copy per link direction: the neighbour offsets and the
       // plaquettes' directions become constants, so a site's loads issue
-      // together instead of one direction at a time (6.8 -> 6.4 us at 96^3).
-      // The SU(2) link kinds and FP64 lose more to the extra registers
-      // (a wave per SIMD fewer, or spills) than they gain.
+      // together instead of one direction at a time (U(1), 96^3: 6.8 ->
+      // 6.4 us).  The FP64 U(1) kind loses more to the extra registers.
       if (mu == 0)
-        acc = site_update<T, M, KIND>(L, x, par, s, 0, r, reunit);
+        acc = site_update<T, M, KIND, 0>(L, x, par, s, 0, r, reunit);
       else if (mu == 1)
-        acc = site_update<T, M, KIND>(L, x, par, s, 1, r, reunit);
+        acc = site_update<T, M, KIND, 1>(L, x, par, s, 1, r, reunit);
       else
-        acc = site_update<T, M, KIND>(L, x, par, s, 2, r, reunit);
+        acc = site_update<T, M, KIND, 2>(L, x, par, s, 2, r, reunit);
     } else {
-      acc = site_update<T, M, KIND>(L, x, par, s, mu, r, reunit);
+      acc = site_update<T, M, KIND, -1>(L, x, par, s, mu, r, reunit);
     }
   }
   // counted wavefront by wavefront with atomics that return nothing: no
@@ -1055,8 +1177,8 @@ __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
       row = mu ? CNT_DOUBLET2_OR : KIND;
     if constexpr ((M & M_H2) != 0 && KIND == SU2HIP_K_DOUBLET_METROPOLIS)
       row = mu ? CNT_DOUBLET2_METRO : KIND;
-    count_up(&cnt[(size_t)(row * 2 + 0) * nblk + blockIdx.x], __popcll(am));
-    count_up(&cnt[(size_t)(row * 2 + 1) * nblk + blockIdx.x], __popcll(tm));
+    count_up(&cnt[(size_t)(row * 2 + 0) * nblk + idx], __popcll(am));
+    count_up(&cnt[(size_t)(row * 2 + 1) * nblk + idx], __popcll(tm));
   }
   if (muca) {
     double v = valid ? orderparam_at<T, M>(L, op, par, s) : 0.0;
@@ -1100,7 +1222,8 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(5))) void k
 template <typename T, int M>
 __global__ __launch_bounds__(BLK) void k_hop(const LatDesc *__restrict__ lats,
                                              const BlockMap *__restrict__ blk, int nblk, int one) {
-  const BlockMap bm = block_of(blk, nblk, one, BLK);
+  int idx;
+  const BlockMap bm = block_of(blk, nblk, one, BLK, 1, idx);
   const LatDesc L = lats[bm.lat];
   pin_desc<M, SU2HIP_K_AUX>(L);
   if (!L.active || L.budget == 0 || !L.H) return;
