@@ -122,14 +122,24 @@ constexpr bool hop_cached() {
   return (M & M_NH) != 0 && (M & M_H2) == 0;
 }
 
-// -1/2 Phi(x+mu) exp(-i alpha sigma_3) Phi(x)^+ of link (x, mu)
+// -1/2 Phi(x+mu) exp(-i alpha sigma_3) Phi(x)^+ of a link, from Phi(x+mu),
+// alpha and Phi(x): the same roundings (sum2) in the cache and in a pass
+template <typename T, int M>
+__device__ __forceinline__ Q<T> hop_of(Q<T> fp, T al, const Q<T> &f) {
+  if constexpr ((M & M_U1) != 0) {
+    const Q<T> u = u1twist<T>(al);
+    const T c = u.a, d = u.d;
+    fp = Q<T>{ffma(fp.a, c, -(fp.d * d)), ffma(fp.b, c, -(fp.c * d)), ffma(fp.c, c, fp.b * d),
+              ffma(fp.d, c, fp.a * d)};
+  }
+  return qscale(qmul_w<2, 1, 2>(fp, qconj(f)), (T)-0.5);
+}
 template <typename T, int M>
 __device__ __forceinline__ Q<T> hop_term(const LatDesc &L, const T *A, const T *F, const Site &x,
                                          int mu) {
-  Q<T> b = F_at(L, F, shift(L, x, mu, +1));
-  if constexpr ((M & M_U1) != 0) b = qmul_u1(b, u1twist<T>(A_at(L, A, x, mu)));
-  Q<T> t = qmul(b, qconj(F_at(L, F, x)));
-  return qscale(t, (T)-0.5);
+  T al = (T)0;
+  if constexpr ((M & M_U1) != 0) al = A_at(L, A, x, mu);
+  return hop_of<T, M>(F_at(L, F, shift(L, x, mu, +1)), al, F_at(L, F, x));
 }
 
 // The SU(2) link kinds built with a constant direction (one copy each).  FP64
@@ -183,10 +193,7 @@ __device__ __forceinline__ Q<T> link_staple(const LatDesc &L, const T *U, const 
   if constexpr ((M & M_NH) == 0) {
     return qscale(W, k);
   } else {
-    if (!(hop_cached<M>() && L.H)) {
-      if constexpr ((M & M_U1) != 0) fp = qmul_u1(fp, u1twist<T>(al));
-      h = qscale(qmul(fp, qconj(h)), (T)-0.5);
-    }
+    if (!(hop_cached<M>() && L.H)) h = hop_of<T, M>(fp, al, h);
     // -beta/2 W + the first doublet's term, one rounding
     Q<T> V{ffma(W.a, k, h.a), ffma(W.b, k, h.b), ffma(W.c, k, h.c), ffma(W.d, k, h.d)};
     // the second doublet's (the doublet loop of src/staples.c:150-190)
