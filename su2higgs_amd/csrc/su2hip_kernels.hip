@@ -1679,22 +1679,58 @@ __device__ double alpha_proj(const LatDesc &L, const T *U, const T *G, const Sit
   return ::atan2(u1.im[0] + u1.im[3], u1.re[0] + u1.re[3]) * ::sqrt(L.beta);
 }
 
+// the loads that follow start only once v is computed
+__device__ __forceinline__ void fence_loads(double &v) { asm volatile("" : "+v"(v) : : "memory"); }
+
 template <typename T, int M>
 __device__ void measure_site(const LatDesc &L, int par, int s, double *acc) {
   const T *U = (const T *)L.U, *A = (const T *)L.A, *F = (const T *)L.F, *G = (const T *)L.G,
           *S = (const T *)L.S;
   Site x = site_of(L, par, s);
+  // Every link and angle of the site's plaquettes in flight at once; the
+  // doublets after the plaquettes have freed their links' registers.  Left to
+  // itself the compiler waits for each term's loads (the cosines branch) and
+  // still holds 212 registers in FP64 SU(2)xU(1)+Higgs, two wavefronts per
+  // SIMD; now 160, three.  With the sums' reduction cut to the model's own,
+  // a whole measure call at 96^3 went from 83 to 68 us in FP64 (the kernel
+  // 48 -> 41, its fields 19 us at the fabric's rate and its FP64 arithmetic
+  // 20 us) and from 73 to 55 us in FP32.
+  LinkRaw<M, T> u0[3], un[3][3];
+  T a0[3], an[3][3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    u0[d] = ldL<M>(link_run<M>(U, L.Vh, d, par), s);
+    if constexpr ((M & M_U1) != 0) a0[d] = A_at(L, A, x, d);
+  }
+#pragma unroll
+  for (int n = 0; n < 3; n++) {
+    const Site xn = shift(L, x, n, +1);
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+      if (d != n) {
+        un[d][n] = ldL<M>(link_run<M>(U, L.Vh, d, xn.par), xn.s);
+        if constexpr ((M & M_U1) != 0) an[d][n] = A_at(L, A, xn, d);
+      }
+  }
+  __builtin_amdgcn_sched_barrier(0);
   // local_su2wilson (src/su2u1.c:143-157)
   double wl = 0.0;
 #pragma unroll
   for (int d1 = 0; d1 < 3; d1++)
 #pragma unroll
     for (int d2 = 0; d2 < d1; d2++) {
-      Q<double> t = qmul(qmul(qmul(qd(U_at<M>(L, U, x, d2)), qd(U_at<M>(L, U, shift(L, x, d2, +1), d1))),
-                              qconj(qd(U_at<M>(L, U, shift(L, x, d1, +1), d2)))),
-                         qconj(qd(U_at<M>(L, U, x, d1))));
+      Q<double> t = qmul(qmul(qmul(qd(u0[d2].get()), qd(un[d1][d2].get())), qconj(qd(un[d2][d1].get()))),
+                         qconj(qd(u0[d1].get())));
       wl += (1.0 - 0.5 * (2.0 * t.a));
     }
+  fence_loads(wl);
+  Q<T> f0{}, fn[3];
+  if constexpr ((M & M_NH) != 0) {
+    f0 = ldF(F, L.Vh, par, s);
+#pragma unroll
+    for (int d = 0; d < 3; d++) fn[d] = F_at(L, F, shift(L, x, d, +1));
+    __builtin_amdgcn_sched_barrier(0);
+  }
   wl *= L.beta;
   double action = wl;
   acc[SU2HIP_SUM_WILSON] += wl;
@@ -1705,8 +1741,7 @@ __device__ void measure_site(const LatDesc &L, int par, int s, double *acc) {
     for (int d1 = 0; d1 < 3; d1++)
 #pragma unroll
       for (int d2 = 0; d2 < d1; d2++) {
-        double pl = (double)A_at(L, A, x, d2) + (double)A_at(L, A, shift(L, x, d2, +1), d1) -
-                    (double)A_at(L, A, shift(L, x, d1, +1), d2) - (double)A_at(L, A, x, d1);
+        double pl = (double)a0[d2] + (double)an[d1][d2] - (double)an[d2][d1] - (double)a0[d1];
         u += (1.0 - ::cos(L.r_u1 * pl));
       }
     u *= L.betau1;
@@ -1715,17 +1750,18 @@ __device__ void measure_site(const LatDesc &L, int par, int s, double *acc) {
   }
   double mod = 0.0, tmod = 0.0;
   if constexpr ((M & M_NH) != 0) {
-    Q<double> f = qd(F_at(L, F, x));
+    Q<double> f = qd(f0);
     mod = 0.5 * qdot(f, f);
     // covariant_doublet (src/su2u1.c:477-488)
     double cov = 0.0;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-      Q<double> t = qmul(qmul(qconj(f), qd(U_at<M>(L, U, x, d))), qd(F_at(L, F, shift(L, x, d, +1))));
+      Q<double> t = qmul(qmul(qconj(f), qd(u0[d].get())), qd(fn[d]));
       double hop;
       if constexpr ((M & M_U1) != 0) {
-        double al = A_at(L, A, x, d);
-        hop = -(t.a * ::cos(al) + t.d * ::sin(al));
+        double sn, cs;
+        ::sincos((double)a0[d], &sn, &cs);
+        hop = -(t.a * cs + t.d * sn);
       } else {
         hop = -t.a;
       }
@@ -1878,18 +1914,66 @@ __device__ __forceinline__ double magcharge_site(const LatDesc &L, int par, int 
   return ch;
 }
 
+// the volume sums a model has, as bits; the rest are 0
+constexpr uint32_t sum_bit(int j) { return 1u << j; }
+constexpr uint32_t live_sums(int m) {
+  uint32_t v = sum_bit(SU2HIP_SUM_ACTION) | sum_bit(SU2HIP_SUM_WILSON);
+  if (m & M_U1) v |= sum_bit(SU2HIP_SUM_U1WILSON);
+  if (m & M_NH) v |= sum_bit(SU2HIP_SUM_COV_PHI) | sum_bit(SU2HIP_SUM_PHI2) | sum_bit(SU2HIP_SUM_PHI4);
+  if (m & M_H2)
+    v |= sum_bit(SU2HIP_SUM_COV_PHI_2) | sum_bit(SU2HIP_SUM_PHI2_2) | sum_bit(SU2HIP_SUM_PHI4_2) |
+         sum_bit(SU2HIP_SUM_R12) | sum_bit(SU2HIP_SUM_I12);
+  if (m & M_TR) {
+    v |= sum_bit(SU2HIP_SUM_HOP_SIGMA) | sum_bit(SU2HIP_SUM_SIGMA2) | sum_bit(SU2HIP_SUM_SIGMA4) |
+         sum_bit(SU2HIP_SUM_MAGCHARGE) | sum_bit(SU2HIP_SUM_MAGCHARGE_ABS);
+    if (m & M_NH) v |= sum_bit(SU2HIP_SUM_PHI2SIGMA2);
+  }
+  if (m & M_SG) {
+    v |= sum_bit(SU2HIP_SUM_S_COV) | sum_bit(SU2HIP_SUM_S) | sum_bit(SU2HIP_SUM_S2) |
+         sum_bit(SU2HIP_SUM_S3) | sum_bit(SU2HIP_SUM_S4);
+    if (m & M_NH) v |= sum_bit(SU2HIP_SUM_SPHISQ) | sum_bit(SU2HIP_SUM_S2PHISQ);
+  }
+  return v;
+}
+constexpr uint32_t MAG_SUMS = sum_bit(SU2HIP_SUM_MAGCHARGE) | sum_bit(SU2HIP_SUM_MAGCHARGE_ABS);
+
+// the k-th (from 0) set bit of v
+__device__ __forceinline__ int nth_sum(uint32_t v, int k) {
+  for (; k > 0; k--) v &= v - 1;
+  return __ffs((int)v) - 1;
+}
+
+// block_sums of the sums in LIVE, written into a row of partials
+template <uint32_t LIVE>
+__device__ __forceinline__ void store_row(const double *v, double *lds, double *row) {
+  constexpr int N = __builtin_popcount(LIVE);
+  const int w = threadIdx.x >> 6;
+  int n = 0;
+#pragma unroll
+  for (int j = 0; j < SU2HIP_NSUMS; j++)
+    if ((LIVE >> j) & 1) {
+      const double t = wave_sum(v[j]);
+      if ((threadIdx.x & 63) == 0) lds[w * N + n] = t;
+      n++;
+    }
+  __syncthreads();
+  if (threadIdx.x < N) {
+    double r = 0.0;
+#pragma unroll
+    for (int i = 0; i < BLK / 64; i++) r += lds[i * N + threadIdx.x];
+    row[nth_sum(LIVE, (int)threadIdx.x)] = r;
+  }
+}
+
+// The sums of chunk s0 .. s0 + BLK of both parities into a row of partials.
 // Each thread measures site s of parity 0, then of parity 1, so every sum
 // of a thread is (0 + site0) + site1 in that order.  The loop is kept
-// rolled: interleaving the two sites doubles the live registers.
+// rolled: interleaving the two sites doubles the live registers.  Only the
+// model's own sums are reduced: the butterflies of all 24 were 288 cross-lane
+// reads per wavefront, 20 remain.
 template <typename T, int M>
-__global__ __launch_bounds__(BLK) void k_measure(const LatDesc *__restrict__ lats,
-                                                 const BlockMap *__restrict__ blk,
-                                                 double *__restrict__ partial) {
-  __shared__ double lds[BLK / 64 * SU2HIP_NSUMS];
-  const BlockMap bm = blk[blockIdx.x];
-  const LatDesc &L = lats[bm.lat];
-  if (!L.active) return;
-  int s = bm.s0 + (int)threadIdx.x;
+__device__ __forceinline__ void measure_chunk(const LatDesc &L, int s0, double *row, double *lds) {
+  const int s = s0 + (int)threadIdx.x;
   double acc[SU2HIP_NSUMS];
 #pragma unroll
   for (int j = 0; j < SU2HIP_NSUMS; j++) acc[j] = 0.0;
@@ -1897,25 +1981,11 @@ __global__ __launch_bounds__(BLK) void k_measure(const LatDesc *__restrict__ lat
 #pragma unroll 1
     for (int par = 0; par < 2; par++) measure_site<T, M>(L, par, s, acc);
   }
-  double t = block_sums<SU2HIP_NSUMS>(acc, lds);
-  if (threadIdx.x < SU2HIP_NSUMS)
-    partial[(size_t)(L.blk_base + bm.s0 / BLK) * SU2HIP_NSUMS + threadIdx.x] = t;
+  store_row<live_sums(M) & ~MAG_SUMS>(acc, lds, row);
 }
-
-// The two monopole sums of the adjoint model, written into the rows
-// k_measure has just filled (which hold 0 there): same threads, same sites,
-// same order, so each is bitwise what one fused kernel would give.  Kept
-// apart because the 24 projected links of a cube, in FP64, do not fit in
-// registers beside the other sums.
 template <typename T, int M>
-__global__ __launch_bounds__(BLK) void k_magcharge(const LatDesc *__restrict__ lats,
-                                                   const BlockMap *__restrict__ blk,
-                                                   double *__restrict__ partial) {
-  __shared__ double lds[BLK / 64 * 2];
-  const BlockMap bm = blk[blockIdx.x];
-  const LatDesc &L = lats[bm.lat];
-  if (!L.active) return;
-  int s = bm.s0 + (int)threadIdx.x;
+__device__ __forceinline__ void magcharge_chunk(const LatDesc &L, int s0, double *row, double *lds) {
+  const int s = s0 + (int)threadIdx.x;
   double acc[2] = {0.0, 0.0};
   if (s < L.Vh) {
 #pragma unroll 1
@@ -1926,31 +1996,78 @@ __global__ __launch_bounds__(BLK) void k_magcharge(const LatDesc *__restrict__ l
     }
   }
   double t = block_sums<2>(acc, lds);
-  if (threadIdx.x < 2)
-    partial[(size_t)(L.blk_base + bm.s0 / BLK) * SU2HIP_NSUMS + SU2HIP_SUM_MAGCHARGE + threadIdx.x] = t;
+  if (threadIdx.x < 2) row[SU2HIP_SUM_MAGCHARGE + threadIdx.x] = t;
 }
 
-__global__ __launch_bounds__(BLK) void k_measure_final(const LatDesc *__restrict__ lats,
-                                                       const double *__restrict__ partial,
-                                                       double *__restrict__ sums) {
+// The rows of one lattice added up, one workgroup of FIN threads: G groups of
+// threads take every G-th row, a thread one sum, and the groups are added in
+// a tree.  A row per thread and all its sums in a loop waited for 7 rows one
+// after another at 96^3 (17.1 us); this has every row in flight at once
+// (6.4 us).
+constexpr int FIN = 1024;
+__device__ __forceinline__ void sum_rows(const double *__restrict__ rows, int n, uint32_t live,
+                                         double *out, double *lds) {
+  const int N = __popc(live), G = FIN / N;
+  const int k = (int)threadIdx.x % N, g = (int)threadIdx.x / N;
+  const int j = nth_sum(live, k);
+  double v = 0.0;
+  if (g < G) {
+#pragma unroll 8
+    for (int i = g; i < n; i += G) v += rows[(size_t)i * SU2HIP_NSUMS + j];
+    lds[g * N + k] = v;
+  }
+  __syncthreads();
+  int top = 1;
+  while (top < G) top <<= 1;
+  for (int st = top >> 1; st > 0; st >>= 1) {
+    if (g < st && g + st < G) lds[g * N + k] += lds[(g + st) * N + k];
+    __syncthreads();
+  }
+  if (threadIdx.x < SU2HIP_NSUMS) {
+    const uint32_t b = sum_bit((int)threadIdx.x);
+    out[threadIdx.x] = (live & b) ? lds[__popc(live & (b - 1))] : 0.0;
+  }
+}
+
+template <typename T, int M>
+__global__ __launch_bounds__(BLK) void k_measure(const LatDesc *__restrict__ lats,
+                                                 const BlockMap *__restrict__ blk, int nblk, int one,
+                                                 double *__restrict__ partial) {
   __shared__ double lds[BLK / 64 * SU2HIP_NSUMS];
+  int idx;
+  const BlockMap bm = block_of(blk, nblk, one, BLK, 0, idx);
+  const LatDesc L = lats[bm.lat];
+  pin_desc<M, SU2HIP_K_MEASURE>(L);
+  if (!L.active) return;
+  measure_chunk<T, M>(L, bm.s0, partial + (size_t)(L.blk_base + bm.s0 / BLK) * SU2HIP_NSUMS, lds);
+}
+
+// The two monopole sums of the adjoint model, written into the rows of
+// k_measure: same threads, same sites, same order.  Kept apart because the
+// 24 projected links of a cube, in FP64, do not fit in registers beside the
+// other sums.
+template <typename T, int M>
+__global__ __launch_bounds__(BLK) void k_magcharge(const LatDesc *__restrict__ lats,
+                                                   const BlockMap *__restrict__ blk,
+                                                   double *__restrict__ partial) {
+  __shared__ double lds[BLK / 64 * 2];
+  const BlockMap bm = blk[blockIdx.x];
+  const LatDesc &L = lats[bm.lat];
+  if (!L.active) return;
+  magcharge_chunk<T, M>(L, bm.s0, partial + (size_t)(L.blk_base + bm.s0 / BLK) * SU2HIP_NSUMS, lds);
+}
+
+__global__ __launch_bounds__(FIN) void k_measure_final(const LatDesc *__restrict__ lats,
+                                                       const double *__restrict__ partial,
+                                                       uint32_t live, double *__restrict__ sums) {
+  __shared__ double lds[FIN];
   const LatDesc &L = lats[blockIdx.x];
   double *out = sums + (size_t)blockIdx.x * SU2HIP_NSUMS;
   if (!L.active) {
     if (threadIdx.x < SU2HIP_NSUMS) out[threadIdx.x] = 0.0;
     return;
   }
-  // each thread its rows in order, all sums of a row at once
-  double v[SU2HIP_NSUMS];
-#pragma unroll
-  for (int j = 0; j < SU2HIP_NSUMS; j++) v[j] = 0.0;
-  for (int i = threadIdx.x; i < L.nblk; i += BLK) {
-    const double *row = partial + (size_t)(L.blk_base + i) * SU2HIP_NSUMS;
-#pragma unroll
-    for (int j = 0; j < SU2HIP_NSUMS; j++) v[j] += row[j];
-  }
-  double t = block_sums<SU2HIP_NSUMS>(v, lds);
-  if (threadIdx.x < SU2HIP_NSUMS) out[threadIdx.x] = t;
+  sum_rows(partial + (size_t)L.blk_base * SU2HIP_NSUMS, L.nblk, live, out, lds);
 }
 
 // ------------------------------------------------------------------------
@@ -2664,7 +2781,7 @@ hipError_t launch_measure(const LaunchCtx &c) {
       return with_model_of<T>(c.model, [&](auto m) -> hipError_t {
         constexpr int M = decltype(m)::value;
         hipLaunchKernelGGL((k_measure<T, M>), dim3(c.nblk), dim3(BLK), 0, c.stream, c.desc, c.blk,
-                           c.partial);
+                           c.nblk, c.one, c.partial);
         if constexpr ((M & M_TR) != 0)
           hipLaunchKernelGGL((k_magcharge<T, M>), dim3(c.nblk), dim3(BLK), 0, c.stream, c.desc,
                              c.blk, c.partial);
@@ -2673,8 +2790,8 @@ hipError_t launch_measure(const LaunchCtx &c) {
     });
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k_measure_final, dim3(c.max_slots), dim3(BLK), 0, c.stream, c.desc,
-                     c.partial, c.sums);
+  hipLaunchKernelGGL(k_measure_final, dim3(c.max_slots), dim3(FIN), 0, c.stream, c.desc,
+                     c.partial, live_sums(c.model), c.sums);
   return hipGetLastError();
 }
 
@@ -2685,49 +2802,20 @@ hipError_t launch_measure(const LaunchCtx &c) {
 template <typename T, int M>
 __global__ __launch_bounds__(BLK) void k_measure_one(LatDesc L, double *__restrict__ partial) {
   __shared__ double lds[BLK / 64 * SU2HIP_NSUMS];
-  int s = (int)blockIdx.x * BLK + (int)threadIdx.x;
-  double acc[SU2HIP_NSUMS];
-#pragma unroll
-  for (int j = 0; j < SU2HIP_NSUMS; j++) acc[j] = 0.0;
-  if (s < L.Vh) {
-#pragma unroll 1
-    for (int par = 0; par < 2; par++) measure_site<T, M>(L, par, s, acc);
-  }
-  double t = block_sums<SU2HIP_NSUMS>(acc, lds);
-  if (threadIdx.x < SU2HIP_NSUMS) partial[(size_t)blockIdx.x * SU2HIP_NSUMS + threadIdx.x] = t;
+  measure_chunk<T, M>(L, (int)blockIdx.x * BLK, partial + (size_t)blockIdx.x * SU2HIP_NSUMS, lds);
 }
 
 template <typename T, int M>
 __global__ __launch_bounds__(BLK) void k_magcharge_one(LatDesc L, double *__restrict__ partial) {
   __shared__ double lds[BLK / 64 * 2];
-  int s = (int)blockIdx.x * BLK + (int)threadIdx.x;
-  double acc[2] = {0.0, 0.0};
-  if (s < L.Vh) {
-#pragma unroll 1
-    for (int par = 0; par < 2; par++) {
-      double ch = magcharge_site<T, M>(L, par, s);
-      acc[0] += ch;
-      acc[1] += ::fabs(ch);
-    }
-  }
-  double t = block_sums<2>(acc, lds);
-  if (threadIdx.x < 2)
-    partial[(size_t)blockIdx.x * SU2HIP_NSUMS + SU2HIP_SUM_MAGCHARGE + threadIdx.x] = t;
+  magcharge_chunk<T, M>(L, (int)blockIdx.x * BLK, partial + (size_t)blockIdx.x * SU2HIP_NSUMS, lds);
 }
 
-__global__ __launch_bounds__(BLK) void k_measure_one_final(const double *__restrict__ partial,
-                                                           int nblk, double *__restrict__ sums) {
-  __shared__ double lds[BLK / 64 * SU2HIP_NSUMS];
-  double v[SU2HIP_NSUMS];
-#pragma unroll
-  for (int j = 0; j < SU2HIP_NSUMS; j++) v[j] = 0.0;
-  for (int i = threadIdx.x; i < nblk; i += BLK) {
-    const double *row = partial + (size_t)i * SU2HIP_NSUMS;
-#pragma unroll
-    for (int j = 0; j < SU2HIP_NSUMS; j++) v[j] += row[j];
-  }
-  double t = block_sums<SU2HIP_NSUMS>(v, lds);
-  if (threadIdx.x < SU2HIP_NSUMS) sums[threadIdx.x] = t;
+__global__ __launch_bounds__(FIN) void k_measure_one_final(const double *__restrict__ partial,
+                                                           int nblk, uint32_t live,
+                                                           double *__restrict__ sums) {
+  __shared__ double lds[FIN];
+  sum_rows(partial, nblk, live, sums, lds);
 }
 
 hipError_t launch_measure_one(hipStream_t stream, int fp64, int model, const LatDesc &L,
@@ -2744,8 +2832,8 @@ hipError_t launch_measure_one(hipStream_t stream, int fp64, int model, const Lat
     });
   });
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_measure_one_final, dim3(1), dim3(BLK), 0, stream, (const double *)partial, nb,
-                     sums);
+  hipLaunchKernelGGL(k_measure_one_final, dim3(1), dim3(FIN), 0, stream, (const double *)partial, nb,
+                     live_sums(model), sums);
   return hipGetLastError();
 }
 
