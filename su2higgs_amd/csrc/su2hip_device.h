@@ -279,29 +279,35 @@ __device__ __forceinline__ gptr<T> gmem(T *p) {
   return reinterpret_cast<gptr<T>>(reinterpret_cast<unsigned long>(p));
 }
 
+// Four-component vectors of the Vh sites of one parity.  FP32: 16 bytes a
+// site.  FP64: the first two components of every site, then the last two, so
+// that each 16-byte load of a wavefront covers one contiguous 1 KiB; as 32
+// bytes a site, each of the two loads touched the lines of both and the L1s
+// were the FP64 link passes' second limit after the fabric (96^3 sweep 969 ->
+// 949 us, four 48^3 adjoint lattices 498 -> 484).  32-bit byte offsets from a uniform base (2^27 sites of 32 bytes).
 template <typename T>
-__device__ __forceinline__ Q<T> ld4(const T *p);
-template <>
-__device__ __forceinline__ Q<float> ld4<float>(const float *p) {
-  vf4 v = *gmem(reinterpret_cast<const vf4 *>(p));
-  return Q<float>{v.x, v.y, v.z, v.w};
-}
-template <>
-__device__ __forceinline__ Q<double> ld4<double>(const double *p) {
-  vd2 a = *gmem(reinterpret_cast<const vd2 *>(p));
-  vd2 b = *gmem(reinterpret_cast<const vd2 *>(p + 2));
-  return Q<double>{a.x, a.y, b.x, b.y};
+__device__ __forceinline__ Q<T> ld4(const T *run, int Vh, int s) {
+  const char *b = reinterpret_cast<const char *>(run);
+  const size_t o = (uint32_t)s * 16u;
+  if constexpr (sizeof(T) == 4) {
+    const vf4 v = *gmem(reinterpret_cast<const vf4 *>(b + o));
+    return Q<T>{v.x, v.y, v.z, v.w};
+  } else {
+    const vd2 v = *gmem(reinterpret_cast<const vd2 *>(b + o));
+    const vd2 w = *gmem(reinterpret_cast<const vd2 *>(b + (size_t)Vh * 16 + o));
+    return Q<T>{v.x, v.y, w.x, w.y};
+  }
 }
 template <typename T>
-__device__ __forceinline__ void st4(T *p, const Q<T> &q);
-template <>
-__device__ __forceinline__ void st4<float>(float *p, const Q<float> &q) {
-  *gmem(reinterpret_cast<vf4 *>(p)) = vf4{q.a, q.b, q.c, q.d};
-}
-template <>
-__device__ __forceinline__ void st4<double>(double *p, const Q<double> &q) {
-  *gmem(reinterpret_cast<vd2 *>(p)) = vd2{q.a, q.b};
-  *gmem(reinterpret_cast<vd2 *>(p + 2)) = vd2{q.c, q.d};
+__device__ __forceinline__ void st4(T *run, int Vh, int s, const Q<T> &q) {
+  char *b = reinterpret_cast<char *>(run);
+  const size_t o = (uint32_t)s * 16u;
+  if constexpr (sizeof(T) == 4) {
+    *gmem(reinterpret_cast<vf4 *>(b + o)) = vf4{q.a, q.b, q.c, q.d};
+  } else {
+    *gmem(reinterpret_cast<vd2 *>(b + o)) = vd2{q.a, q.b};
+    *gmem(reinterpret_cast<vd2 *>(b + (size_t)Vh * 16 + o)) = vd2{q.c, q.d};
+  }
 }
 
 // FP32 links are stored in 12 bytes instead of 16, by stereographic
@@ -378,7 +384,7 @@ __device__ __forceinline__ Q<T> ldU(const T *__restrict__ U, int Vh, int d, int 
     gptr<const float> p = gmem(U + ((size_t)(d * 2 + par) * Vh + s) * 3);
     return link_unpack(F3{p[0], p[1], p[2]});
   } else {
-    return ld4(U + ((size_t)(d * 2 + par) * Vh + s) * 4);
+    return ld4(U + (size_t)(d * 2 + par) * Vh * 4, Vh, s);
   }
 }
 template <int M, typename T>
@@ -395,16 +401,15 @@ __device__ __forceinline__ void stU(T *__restrict__ U, int Vh, int d, int par, i
     // per component
     const float dx = unit_excess(q);
     const float e = dx * __builtin_fmaf(0.375f, dx, -0.5f);
-    st4(U + ((size_t)(d * 2 + par) * Vh + s) * 4,
+    st4(U + (size_t)(d * 2 + par) * Vh * 4, Vh, s,
         Q<float>{__builtin_fmaf(q.a, e, q.a), __builtin_fmaf(q.b, e, q.b), __builtin_fmaf(q.c, e, q.c),
                  __builtin_fmaf(q.d, e, q.d)});
   } else {
-    st4(U + ((size_t)(d * 2 + par) * Vh + s) * 4, q);
+    st4(U + (size_t)(d * 2 + par) * Vh * 4, Vh, s, q);
   }
 }
-// The same with the (direction, parity) run of links as a uniform base and a
-// 32-bit byte offset (a run is at most 2^27 links of 32 bytes): one
-// instruction of address arithmetic per load instead of five.
+// The same from the (direction, parity) run of links, a uniform base: a 32-bit
+// byte offset is one instruction of address arithmetic instead of five.
 template <int M, typename T>
 __device__ __forceinline__ const T *link_run(const T *U, int Vh, int d, int par) {
   return U + (size_t)(d * 2 + par) * Vh * (packed_links<M, T>() ? 3 : 4);
@@ -421,22 +426,22 @@ struct LinkRaw {
   }
 };
 template <int M, typename T>
-__device__ __forceinline__ LinkRaw<M, T> ldL(const T *run, int s) {
-  const char *b = reinterpret_cast<const char *>(run);
+__device__ __forceinline__ LinkRaw<M, T> ldL(const T *run, int Vh, int s) {
   if constexpr (packed_links<M, T>()) {
+    const char *b = reinterpret_cast<const char *>(run);
     gptr<const float> p = gmem(reinterpret_cast<const float *>(b + (size_t)((uint32_t)s * 12u)));
     return LinkRaw<M, T>{F3{p[0], p[1], p[2]}};
   } else {
-    return LinkRaw<M, T>{ld4(reinterpret_cast<const T *>(b + (size_t)((uint32_t)s * (uint32_t)(4 * sizeof(T)))))};
+    return LinkRaw<M, T>{ld4(run, Vh, s)};
   }
 }
 template <typename T>
 __device__ __forceinline__ Q<T> ldF(const T *__restrict__ F, int Vh, int par, int s) {
-  return ld4(F + ((size_t)par * Vh + s) * 4);
+  return ld4(F + (size_t)par * Vh * 4, Vh, s);
 }
 template <typename T>
 __device__ __forceinline__ void stF(T *__restrict__ F, int Vh, int par, int s, const Q<T> &q) {
-  st4(F + ((size_t)par * Vh + s) * 4, q);
+  st4(F + (size_t)par * Vh * 4, Vh, s, q);
 }
 template <typename T>
 __device__ __forceinline__ V3<T> ldG(const T *__restrict__ G, int Vh, int par, int s) {

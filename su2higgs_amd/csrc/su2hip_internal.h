@@ -8,13 +8,14 @@
 //   links    U[d][p][s][c]   d<3, c<4    (24 Vh words; a 4-vector per link)
 //   doublet  F[p][s][c]      c<4         (8 Vh; a 4-vector per site)
 //   doublet2 F2[p][s][c]     c<4         (8 Vh; the second doublet, nhiggs = 2)
+//   (FP64 4-vectors in two halves, [c/2][s][c%2]: ld4)
 //   U(1)     A[d][p][s]                  (6 Vh)
 //   triplet  G[c][p][s]      c<3         (6 Vh)
 //   singlet  S[p][s]                     (2 Vh)
 //   backup   B: the doublet's or the triplet's layout
 // so the 64 lanes of a wavefront, which own 64 consecutive s of one parity,
-// read one contiguous 1 KiB (FP32) segment per link or doublet load and one
-// contiguous segment per component of the other fields.
+// read one contiguous 1 KiB segment per 16-byte load of a link or doublet and
+// one contiguous segment per component of the other fields.
 #pragma once
 
 #include <hip/hip_runtime.h>

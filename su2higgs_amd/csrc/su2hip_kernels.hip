@@ -97,12 +97,12 @@ struct StapleLinks {
     const T *mu_o = link_run<M>(U, L.Vh, MU, op);
     const T *nu_s = link_run<M>(U, L.Vh, NU, x.par), *nu_o = link_run<M>(U, L.Vh, NU, op);
     const Site sn = shift(L, x, NU, +1), sm = shift(L, x, NU, -1), spm = shift(L, sp, NU, -1);
-    xp = ldL<M>(nu_o, sp.s);
-    xn = ldL<M>(mu_o, sn.s);
-    x0 = ldL<M>(nu_s, x.s);
-    xpm = ldL<M>(nu_s, spm.s);
-    xm_mu = ldL<M>(mu_o, sm.s);
-    xm = ldL<M>(nu_o, sm.s);
+    xp = ldL<M>(nu_o, L.Vh, sp.s);
+    xn = ldL<M>(mu_o, L.Vh, sn.s);
+    x0 = ldL<M>(nu_s, L.Vh, x.s);
+    xpm = ldL<M>(nu_s, L.Vh, spm.s);
+    xm_mu = ldL<M>(mu_o, L.Vh, sm.s);
+    xm = ldL<M>(nu_o, L.Vh, sm.s);
   }
   __device__ __forceinline__ void add_to(Q<T> &W) const {
     // a stored four-component link enters conjugated by a sign, a packed one
@@ -171,7 +171,7 @@ __device__ __forceinline__ Q<T> link_staple(const LatDesc &L, const T *U, const 
     asm volatile("" : "+v"(W.a), "+v"(W.b), "+v"(W.c), "+v"(W.d) : : "memory");
   }
   s2.load(L, U, x, sp);
-  const auto o = ldL<M>(link_run<M>(U, L.Vh, MU, x.par), x.s);
+  const auto o = ldL<M>(link_run<M>(U, L.Vh, MU, x.par), L.Vh, x.s);
   // the cached hopping term, or the doublet it is formed from
   Q<T> h{(T)0, (T)0, (T)0, (T)0}, fp = h;
   T al = (T)0;
@@ -209,7 +209,7 @@ __device__ __forceinline__ Q<T> link_staple_rt(const LatDesc &L, const T *U, con
   old = ldU<M>(U, L.Vh, mu, x.par, x.s);
   Q<T> V = qscale(wilson_staple<T, M>(L, U, x, mu), (T)(-0.5 * L.beta));
   if constexpr (hop_cached<M>())
-    if (L.H) return qadd(V, ld4((const T *)L.H + ((size_t)(mu * 2 + x.par) * L.Vh + x.s) * 4));
+    if (L.H) return qadd(V, ld4((const T *)L.H + (size_t)(mu * 2 + x.par) * L.Vh * 4, L.Vh, x.s));
   if constexpr ((M & M_NH) != 0) V = qadd(V, hop_term<T, M>(L, A, F, x, mu));
   if constexpr ((M & M_H2) != 0) V = qadd(V, hop_term<T, M>(L, A, (const T *)L.F2, x, mu));
   return V;
@@ -721,7 +721,8 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
       if (n2 == (T)0) return 1;
       w = qconj(qscale(V, frsqrt(n2)));
     }
-    Q<T> nu = qmul(qmul(w, qconj(old)), w);
+    constexpr int V1 = packed_links<M, T>() && (M & M_TR) == 0 ? 1 : 2;
+    Q<T> nu = qmul_w<2>(qmul_w<2, 1, V1>(w, qconj(old)), w);
     (void)reunit;  // FP32 links are renormalised by their packed storage
     if constexpr ((M & M_TR) != 0) {
       V3<T> a1 = ldG(G, Vh, par, s), a2 = G_at(L, G, shift(L, x, mu, +1));
@@ -1243,7 +1244,7 @@ __global__ __launch_bounds__(BLK) void k_hop(const LatDesc *__restrict__ lats,
     const Site x = site_of(L, par, s);
 #pragma unroll
     for (int mu = 0; mu < 3; mu++)
-      st4(H + ((size_t)(mu * 2 + par) * L.Vh + s) * 4, hop_term<T, M>(L, A, F, x, mu));
+      st4(H + (size_t)(mu * 2 + par) * L.Vh * 4, L.Vh, s, hop_term<T, M>(L, A, F, x, mu));
   }
 }
 
@@ -1699,7 +1700,7 @@ __device__ void measure_site(const LatDesc &L, int par, int s, double *acc) {
   T a0[3], an[3][3];
 #pragma unroll
   for (int d = 0; d < 3; d++) {
-    u0[d] = ldL<M>(link_run<M>(U, L.Vh, d, par), s);
+    u0[d] = ldL<M>(link_run<M>(U, L.Vh, d, par), L.Vh, s);
     if constexpr ((M & M_U1) != 0) a0[d] = A_at(L, A, x, d);
   }
 #pragma unroll
@@ -1708,7 +1709,7 @@ __device__ void measure_site(const LatDesc &L, int par, int s, double *acc) {
 #pragma unroll
     for (int d = 0; d < 3; d++)
       if (d != n) {
-        un[d][n] = ldL<M>(link_run<M>(U, L.Vh, d, xn.par), xn.s);
+        un[d][n] = ldL<M>(link_run<M>(U, L.Vh, d, xn.par), L.Vh, xn.s);
         if constexpr ((M & M_U1) != 0) an[d][n] = A_at(L, A, xn, d);
       }
   }
@@ -2398,8 +2399,11 @@ __device__ __forceinline__ void *field_ptr(const LatDesc &L, int field) {
 
 // index of component k of a non-link field (links go through ldU / stU,
 // whose FP32 form is not one word per component)
+template <typename T>
 __device__ __forceinline__ size_t soa_index(int field, int Vh, int par, int s, int k) {
-  if (field == 2 || field == 5) return ((size_t)par * Vh + s) * 4 + k;
+  if (field == 2 || field == 5)  // ld4's layout
+    return sizeof(T) == 8 ? (size_t)par * Vh * 4 + ((size_t)(k >> 1) * Vh + s) * 2 + (k & 1)
+                          : ((size_t)par * Vh + s) * 4 + k;
   return (size_t)(k * 2 + par) * Vh + s;
 }
 
@@ -2421,13 +2425,13 @@ __global__ void k_to_device(LatDesc L, int field, const double *__restrict__ h) 
                  Q<T>{(T)(q[0] * n), (T)(q[1] * n), (T)(q[2] * n), (T)(q[3] * n)});
         } else {
           // four components: the values as given, rounded to T
-          st4((T *)dst + ((size_t)(d * 2 + par) * L.Vh + s) * 4,
+          st4((T *)dst + (size_t)(d * 2 + par) * L.Vh * 4, L.Vh, s,
               Q<T>{(T)q[0], (T)q[1], (T)q[2], (T)q[3]});
         }
       }
       continue;
     }
-    for (int k = 0; k < n; k++) ((T *)dst)[soa_index(field, L.Vh, par, s, k)] = (T)h[i * n + k];
+    for (int k = 0; k < n; k++) ((T *)dst)[soa_index<T>(field, L.Vh, par, s, k)] = (T)h[i * n + k];
   }
 }
 
@@ -2450,7 +2454,7 @@ __global__ void k_to_host(LatDesc L, int field, double *__restrict__ h) {
       }
       continue;
     }
-    for (int k = 0; k < n; k++) h[i * n + k] = (double)((const T *)src)[soa_index(field, L.Vh, par, s, k)];
+    for (int k = 0; k < n; k++) h[i * n + k] = (double)((const T *)src)[soa_index<T>(field, L.Vh, par, s, k)];
   }
 }
 
