@@ -368,6 +368,16 @@ __device__ __forceinline__ F3 link_pack(const Q<float> &q) {
   return v;
 }
 
+// The full FP32 form renormalises every link it stores: q (1 + e) with
+// e = 1/sqrt(1 + dx) - 1 to second order in the excess dx, one rounding per
+// component.
+__device__ __forceinline__ Q<float> link_unit(const Q<float> &q) {
+  const float dx = unit_excess(q);
+  const float e = dx * __builtin_fmaf(0.375f, dx, -0.5f);
+  return Q<float>{__builtin_fmaf(q.a, e, q.a), __builtin_fmaf(q.b, e, q.b), __builtin_fmaf(q.c, e, q.c),
+                  __builtin_fmaf(q.d, e, q.d)};
+}
+
 // Link loads and stores.  M carries the model bits of the kernel; with
 // M_PK an FP32 link is in the packed 12-byte form, otherwise (and always in
 // FP64) it is the four components.  There is no default: every caller says
@@ -396,14 +406,7 @@ __device__ __forceinline__ void stU(T *__restrict__ U, int Vh, int d, int par, i
     p[1] = v.y;
     p[2] = v.z;
   } else if constexpr (sizeof(T) == 4) {
-    // the full FP32 form renormalises every link it stores: q (1 + e) with
-    // e = 1/sqrt(1 + dx) - 1 to second order in the excess dx, one rounding
-    // per component
-    const float dx = unit_excess(q);
-    const float e = dx * __builtin_fmaf(0.375f, dx, -0.5f);
-    st4(U + (size_t)(d * 2 + par) * Vh * 4, Vh, s,
-        Q<float>{__builtin_fmaf(q.a, e, q.a), __builtin_fmaf(q.b, e, q.b), __builtin_fmaf(q.c, e, q.c),
-                 __builtin_fmaf(q.d, e, q.d)});
+    st4(U + (size_t)(d * 2 + par) * Vh * 4, Vh, s, link_unit(q));
   } else {
     st4(U + (size_t)(d * 2 + par) * Vh * 4, Vh, s, q);
   }
@@ -413,6 +416,11 @@ __device__ __forceinline__ void stU(T *__restrict__ U, int Vh, int d, int par, i
 template <int M, typename T>
 __device__ __forceinline__ const T *link_run(const T *U, int Vh, int d, int par) {
   return U + (size_t)(d * 2 + par) * Vh * (packed_links<M, T>() ? 3 : 4);
+}
+// the links of one parity from the base of their direction
+template <int M, typename T>
+__device__ __forceinline__ T *par_run(T *dir, int Vh, int par) {
+  return dir + (size_t)par * Vh * (packed_links<M, std::remove_const_t<T>>() ? 3 : 4);
 }
 // a link as it is stored, loaded now and rebuilt where it is used
 template <int M, typename T>
@@ -433,6 +441,28 @@ __device__ __forceinline__ LinkRaw<M, T> ldL(const T *run, int Vh, int s) {
     return LinkRaw<M, T>{F3{p[0], p[1], p[2]}};
   } else {
     return LinkRaw<M, T>{ld4(run, Vh, s)};
+  }
+}
+// what stU stores for q, and a link stored as it is
+template <int M, typename T>
+__device__ __forceinline__ LinkRaw<M, T> raw_link(const Q<T> &q) {
+  if constexpr (packed_links<M, T>())
+    return LinkRaw<M, T>{link_pack(q)};
+  else if constexpr (sizeof(T) == 4)
+    return LinkRaw<M, T>{link_unit(q)};
+  else
+    return LinkRaw<M, T>{q};
+}
+template <int M, typename T>
+__device__ __forceinline__ void stL(T *run, int Vh, int s, const LinkRaw<M, T> &r) {
+  if constexpr (packed_links<M, T>()) {
+    char *b = reinterpret_cast<char *>(run);
+    gptr<float> p = gmem(reinterpret_cast<float *>(b + (size_t)((uint32_t)s * 12u)));
+    p[0] = r.w.x;
+    p[1] = r.w.y;
+    p[2] = r.w.z;
+  } else {
+    st4(run, Vh, s, r.w);
   }
 }
 template <typename T>

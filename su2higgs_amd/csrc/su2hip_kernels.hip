@@ -92,17 +92,23 @@ __device__ __forceinline__ Q<T> wilson_staple(const LatDesc &L, const T *U, cons
 template <typename T, int M, int MU, int NU>
 struct StapleLinks {
   LinkRaw<M, T> xp, xn, x0, xpm, xm_mu, xm;
-  __device__ __forceinline__ void load(const LatDesc &L, const T *U, const Site &x, const Site &sp) {
-    const int op = x.par ^ 1;
-    const T *mu_o = link_run<M>(U, L.Vh, MU, op);
-    const T *nu_s = link_run<M>(U, L.Vh, NU, x.par), *nu_o = link_run<M>(U, L.Vh, NU, op);
-    const Site sn = shift(L, x, NU, +1), sm = shift(L, x, NU, -1), spm = shift(L, sp, NU, -1);
+  // Ub[d]: the links of direction d.  The transverse ones, and those of MU
+  // itself (a neighbour in the direction's other parity)
+  __device__ __forceinline__ void load_nu(const LatDesc &L, const T *const *Ub, const Site &x,
+                                          const Site &sp) {
+    const T *nu_s = par_run<M>(Ub[NU], L.Vh, x.par), *nu_o = par_run<M>(Ub[NU], L.Vh, x.par ^ 1);
+    const Site sm = shift(L, x, NU, -1), spm = shift(L, sp, NU, -1);
     xp = ldL<M>(nu_o, L.Vh, sp.s);
-    xn = ldL<M>(mu_o, L.Vh, sn.s);
     x0 = ldL<M>(nu_s, L.Vh, x.s);
     xpm = ldL<M>(nu_s, L.Vh, spm.s);
-    xm_mu = ldL<M>(mu_o, L.Vh, sm.s);
     xm = ldL<M>(nu_o, L.Vh, sm.s);
+  }
+  __device__ __forceinline__ void load(const LatDesc &L, const T *const *Ub, const Site &x,
+                                       const Site &sp) {
+    const T *mu_o = par_run<M>(Ub[MU], L.Vh, x.par ^ 1);
+    xn = ldL<M>(mu_o, L.Vh, shift(L, x, NU, +1).s);
+    xm_mu = ldL<M>(mu_o, L.Vh, shift(L, x, NU, -1).s);
+    load_nu(L, Ub, x, sp);
   }
   __device__ __forceinline__ void add_to(Q<T> &W) const {
     // a stored four-component link enters conjugated by a sign, a packed one
@@ -158,48 +164,70 @@ constexpr bool const_dir() {
 // an empty launch and 6.5 its 45 MB at the fabric's 7 TB/s); FP64 takes the transverse
 // directions one at a time, whose registers leave room for more wavefronts.
 template <typename T, int M, int MU>
-__device__ __forceinline__ Q<T> link_staple(const LatDesc &L, const T *U, const T *A, const T *F,
-                                            const Site &x, Q<T> &old) {
-  constexpr int N1 = MU == 0 ? 1 : 0, N2 = MU == 2 ? 1 : 2;
-  const Site sp = shift(L, x, MU, +1);
-  Q<T> W{(T)0, (T)0, (T)0, (T)0};
+struct SiteLinks {
+  static constexpr int N1 = MU == 0 ? 1 : 0, N2 = MU == 2 ? 1 : 2;
   StapleLinks<T, M, MU, N1> s1;
   StapleLinks<T, M, MU, N2> s2;
-  s1.load(L, U, x, sp);
-  if constexpr (sizeof(T) == 8) {
-    s1.add_to(W);
-    asm volatile("" : "+v"(W.a), "+v"(W.b), "+v"(W.c), "+v"(W.d) : : "memory");
-  }
-  s2.load(L, U, x, sp);
-  const auto o = ldL<M>(link_run<M>(U, L.Vh, MU, x.par), L.Vh, x.s);
-  // the cached hopping term, or the doublet it is formed from
-  Q<T> h{(T)0, (T)0, (T)0, (T)0}, fp = h;
-  T al = (T)0;
-  if constexpr ((M & M_NH) != 0) {
-    const bool cached = hop_cached<M>() && L.H;
-    h = ldF(cached ? (const T *)L.H + (size_t)MU * 8 * L.Vh : F, L.Vh, x.par, x.s);
-    if (!cached) {
-      fp = F_at(L, F, sp);
-      if constexpr ((M & M_U1) != 0) al = A_at(L, A, x, MU);
+  LinkRaw<M, T> o;
+  Q<T> h, fp;
+  T al;
+  // the link and its hopping term, cached or as the doublets it is formed from
+  __device__ __forceinline__ void load_own(const LatDesc &L, const T *const *Ub, const Site &x,
+                                           const Site &sp) {
+    o = ldL<M>(par_run<M>(Ub[MU], L.Vh, x.par), L.Vh, x.s);
+    if constexpr ((M & M_NH) != 0) {
+      const T *F = (const T *)L.F;
+      const bool cached = hop_cached<M>() && L.H;
+      h = ldF(cached ? (const T *)L.H + (size_t)MU * 8 * L.Vh : F, L.Vh, x.par, x.s);
+      if (!cached) {
+        fp = F_at(L, F, sp);
+        if constexpr ((M & M_U1) != 0) al = A_at(L, (const T *)L.A, x, MU);
+      }
     }
   }
+  // su2link_staple from the Wilson part W
+  __device__ __forceinline__ Q<T> staple(const LatDesc &L, const Q<T> &W, const Site &x) const {
+    const T k = (T)(-0.5 * L.beta);
+    if constexpr ((M & M_NH) == 0) {
+      return qscale(W, k);
+    } else {
+      Q<T> t = h;
+      if (!(hop_cached<M>() && L.H)) t = hop_of<T, M>(fp, al, h);
+      // -beta/2 W + the first doublet's term, one rounding
+      Q<T> V{ffma(W.a, k, t.a), ffma(W.b, k, t.b), ffma(W.c, k, t.c), ffma(W.d, k, t.d)};
+      // the second doublet's (the doublet loop of src/staples.c:150-190)
+      if constexpr ((M & M_H2) != 0)
+        V = qadd(V, hop_term<T, M>(L, (const T *)L.A, (const T *)L.F2, x, MU));
+      return V;
+    }
+  }
+};
+// W stays before the loads that follow it
+template <typename T>
+__device__ __forceinline__ void fence_q(Q<T> &W) {
+  asm volatile("" : "+v"(W.a), "+v"(W.b), "+v"(W.c), "+v"(W.d) : : "memory");
+}
+
+template <typename T, int M, int MU>
+__device__ __forceinline__ Q<T> link_staple(const LatDesc &L, const T *const *Ub, const Site &x,
+                                            Q<T> &old) {
+  const Site sp = shift(L, x, MU, +1);
+  Q<T> W{(T)0, (T)0, (T)0, (T)0};
+  SiteLinks<T, M, MU> k;
+  k.s1.load(L, Ub, x, sp);
+  if constexpr (sizeof(T) == 8) {
+    k.s1.add_to(W);
+    fence_q(W);
+  }
+  k.s2.load(L, Ub, x, sp);
+  k.load_own(L, Ub, x, sp);
   if constexpr (sizeof(T) == 4) {
     __builtin_amdgcn_sched_barrier(0);
-    s1.add_to(W);
+    k.s1.add_to(W);
   }
-  s2.add_to(W);
-  old = o.get();
-  const T k = (T)(-0.5 * L.beta);
-  if constexpr ((M & M_NH) == 0) {
-    return qscale(W, k);
-  } else {
-    if (!(hop_cached<M>() && L.H)) h = hop_of<T, M>(fp, al, h);
-    // -beta/2 W + the first doublet's term, one rounding
-    Q<T> V{ffma(W.a, k, h.a), ffma(W.b, k, h.b), ffma(W.c, k, h.c), ffma(W.d, k, h.d)};
-    // the second doublet's (the doublet loop of src/staples.c:150-190)
-    if constexpr ((M & M_H2) != 0) V = qadd(V, hop_term<T, M>(L, A, (const T *)L.F2, x, MU));
-    return V;
-  }
+  k.s2.add_to(W);
+  old = k.o.get();
+  return k.staple(L, W, x);
 }
 
 // the same with the direction at run time
@@ -280,8 +308,9 @@ __device__ __forceinline__ V3<T> triplet_staple(const LatDesc &L, const T *U, co
 // hopping_triplet_forward (src/su2u1.c:605-617) with link u
 template <typename T>
 __device__ __forceinline__ T hop_triplet(const Q<T> &u, const V3<T> &a, const V3<T> &b) {
-  V3<T> r = rotate(u, b);
-  return -(a.x * r.x + a.y * r.y + a.z * r.z);
+  // rotate(u, b) and the product with the roundings pinned (sum2)
+  const Q<T> t = qmul_w<2, 1, 2>(qmul_w<2>(u, Q<T>{(T)0, b.x, b.y, b.z}), qconj(u));
+  return -vdot_w<1>(a, V3<T>{t.b, t.c, t.d});
 }
 
 // polysolve3 (src/overrelax.c:14-34): real root by Cardano's formula for a
@@ -562,35 +591,18 @@ struct Fields {
   void *U, *A, *F, *G, *S, *B;
 };
 
-// MU: the direction of an SU(2) link kind (-1 for the others, which take it
-// or the doublet from mu)
-template <typename T, int M, int KIND, int MU>
-__device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int par, int s, int mu_in,
-                                           Rng &r, int reunit) {
-  const int mu = MU >= 0 ? MU : mu_in;
-  T *U = (T *)L.U;
-  T *A = (T *)L.A;
-  T *F = (T *)L.F;
-  T *G = (T *)L.G;
-  T *S = (T *)L.S;
-  const int Vh = L.Vh;
-
+// The move of an SU(2) link kind from the link `old` and its staple V (a1,
+// a2: the triplets at its ends): 1 with the new link in nu, 0 rejected, 2
+// counted as accepted and unchanged.  Lanes with `on` false only keep a full
+// wavefront together (the FP64 heatbath's shared tries).
+template <typename T, int M, int KIND>
+__device__ __forceinline__ int link_move(const LatDesc &L, Q<T> V, const Q<T> &old, const V3<T> &a1,
+                                         const V3<T> &a2, Rng &r, bool on, Q<T> &nu) {
+  constexpr int WV = staple_norm_w<T, M>();
   if constexpr (KIND == SU2HIP_K_LINK_HEATBATH) {
     // heatbath_su2link (src/heatbath.c:15-124), Kennedy-Pendleton
-    Q<T> old;
     T oldact = 0;
-    V3<T> a1{}, a2{};
-    if constexpr ((M & M_TR) != 0) {
-      a1 = ldG(G, Vh, par, s);
-      a2 = G_at(L, G, shift(L, x, mu, +1));
-    }
-    Q<T> V;
-    if constexpr (MU >= 0)
-      V = link_staple<T, M, MU>(L, U, A, F, x, old);
-    else
-      V = link_staple_rt<T, M>(L, U, A, F, x, mu, old);
     if constexpr ((M & M_TR) != 0) oldact = hop_triplet(old, a1, a2);
-    constexpr int WV = staple_norm_w<T, M>();
     T r1, r2, r3, d, a0;
     int loop = 1;
     // a full wavefront shares the FP64 direction's rejection tries
@@ -608,7 +620,7 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
         d = r1 * r3 + r2;
         r3 = (T)1 - uni<T>(r);
         loop++;
-      } while (r3 * r3 > (T)1 - (T)0.5 * d && loop <= 200);
+      } while (on && r3 * r3 > (T)1 - (T)0.5 * d && loop <= 200);
     } else {
       // the same Kennedy-Pendleton loop on the hardware log/cos
       T ia = frsqrt(qdot_w<WV>(V, V));
@@ -622,23 +634,22 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
         d = r1 * r3 + r2;
         r3 = (T)1 - uni<T>(r);
         loop++;
-      } while (r3 * r3 > (T)1 - (T)0.5 * d && loop <= 200);
+      } while (on && r3 * r3 > (T)1 - (T)0.5 * d && loop <= 200);
     }
     a0 = (loop > 200) ? (T)1e-9 : (T)1 - d;
     T rad = (T)1 - a0 * a0;
-    Q<T> nu;
     if constexpr (sizeof(T) == 8) {
       // isotropic direction by cube rejection, the reference's draw order
       // (src/heatbath.c:82-93)
       if (wave) {
         // every lane stays in the wavefront's rounds, as a worker at least
         int tries;
-        hb_dir_wave(r, !(rad < (T)0), r1, r2, r3, d, tries);
-        if (rad < (T)0) return 0;
+        hb_dir_wave(r, on && !(rad < (T)0), r1, r2, r3, d, tries);
+        if (!on || rad < (T)0) return 0;
         r.k += 3u * (uint32_t)tries;
         r.blk = 0xFFFFFFFFu;
       } else {
-        if (rad < (T)0) return 0;
+        if (!on || rad < (T)0) return 0;
         d = (T)2;
         while (d > (T)1 || d == (T)0) {
           r1 = (T)2 * uni<T>(r) - (T)1;
@@ -651,7 +662,7 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
       d = ::sqrt(d);
       nu = Q<T>{a0, r1 * (rad / d), r2 * (rad / d), r3 * (rad / d)};
     } else {
-      if (rad < (T)0) return 0;
+      if (!on || rad < (T)0) return 0;
       // FP32: the same uniform direction on S^2 without rejection
       // (cos(theta) uniform in [-1,1], phi uniform), so a wavefront does
       // not wait for its slowest lane
@@ -667,17 +678,11 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
       T diff = oldact - hop_triplet(nu, a1, a2);
       if (!(uni<T>(r) < sexp(diff))) return 0;
     }
-    stU<M>(U, Vh, mu, par, s, nu);
     return 1;
   } else if constexpr (KIND == SU2HIP_K_LINK_METROPOLIS) {
     // metro_su2link (src/metropolis.c:15-41), random_su2link (src/init.c:43-58);
     // Delta S = 2 Re[(U'-U) V]_0 + Delta(triplet hop), from the staple
-    Q<T> old;
-    Q<T> V;
-    if constexpr (MU >= 0)
-      V = link_staple<T, M, MU>(L, U, A, F, x, old);
-    else
-      V = link_staple_rt<T, M>(L, U, A, F, x, mu, old);
+    if (!on) return 0;
     Q<T> R;
     R.a = (T)10 * (uni<T>(r) - (T)0.5);
     R.b = (T)1 * (uni<T>(r) - (T)0.5);
@@ -689,48 +694,68 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
     } else {
       R = qscale(R, frsqrt(qdot(R, R)));
     }
-    Q<T> nu = qmul_w<2>(old, R);
-    (void)reunit;  // FP32 links are renormalised by their packed storage
+    nu = qmul_w<2>(old, R);
     Q<T> du{nu.a - old.a, nu.b - old.b, nu.c - old.c, nu.d - old.d};
     T diff = (T)2 * qmul(du, V).a;
-    if constexpr ((M & M_TR) != 0) {
-      V3<T> a1 = ldG(G, Vh, par, s), a2 = G_at(L, G, shift(L, x, mu, +1));
+    if constexpr ((M & M_TR) != 0)
       diff += hop_triplet(nu, a1, a2) - hop_triplet(old, a1, a2);
-    }
     if (!metro_accept(diff, r)) return 0;
-    stU<M>(U, Vh, mu, par, s, nu);
     return 1;
   } else if constexpr (KIND == SU2HIP_K_LINK_OVERRELAX) {
     // SU(2) link overrelaxation, U' = W^+ U^+ W^+ with W = staple/|staple|
     // (no reference counterpart); with a triplet a Metropolis test on its
     // hopping term as in src/heatbath.c:107-120
-    Q<T> old;
-    Q<T> V;
-    if constexpr (MU >= 0)
-      V = link_staple<T, M, MU>(L, U, A, F, x, old);
-    else
-      V = link_staple_rt<T, M>(L, U, A, F, x, mu, old);
-    constexpr int WV = staple_norm_w<T, M>();
+    if (!on) return 0;
     Q<T> w;
     if constexpr (sizeof(T) == 8) {
       T a = ::sqrt(qdot_w<WV>(V, V));
-      if (a == (T)0) return 1;
+      if (a == (T)0) return 2;
       w = qconj(Q<T>{V.a / a, V.b / a, V.c / a, V.d / a});
     } else {
       T n2 = qdot_w<WV>(V, V);
-      if (n2 == (T)0) return 1;
+      if (n2 == (T)0) return 2;
       w = qconj(qscale(V, frsqrt(n2)));
     }
     constexpr int V1 = packed_links<M, T>() && (M & M_TR) == 0 ? 1 : 2;
-    Q<T> nu = qmul_w<2>(qmul_w<2, 1, V1>(w, qconj(old)), w);
-    (void)reunit;  // FP32 links are renormalised by their packed storage
+    nu = qmul_w<2>(qmul_w<2, 1, V1>(w, qconj(old)), w);
     if constexpr ((M & M_TR) != 0) {
-      V3<T> a1 = ldG(G, Vh, par, s), a2 = G_at(L, G, shift(L, x, mu, +1));
       T diff = hop_triplet(old, a1, a2) - hop_triplet(nu, a1, a2);
       if (!(uni<T>(r) < sexp(diff))) return 0;
     }
-    stU<M>(U, Vh, mu, par, s, nu);
     return 1;
+  }
+  return 0;
+}
+
+// MU: the direction of an SU(2) link kind (-1 for the others, which take it
+// or the doublet from mu)
+template <typename T, int M, int KIND, int MU>
+__device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int par, int s, int mu_in,
+                                           Rng &r, int reunit) {
+  const int mu = MU >= 0 ? MU : mu_in;
+  T *U = (T *)L.U;
+  T *A = (T *)L.A;
+  T *F = (T *)L.F;
+  T *G = (T *)L.G;
+  T *S = (T *)L.S;
+  const int Vh = L.Vh;
+
+  if constexpr (KIND <= SU2HIP_K_LINK_OVERRELAX) {
+    V3<T> a1{}, a2{};
+    if constexpr ((M & M_TR) != 0) {
+      a1 = ldG(G, Vh, par, s);
+      a2 = G_at(L, G, shift(L, x, mu, +1));
+    }
+    Q<T> V, old, nu;
+    if constexpr (MU >= 0) {
+      const T *Ub[3] = {link_run<M>(U, Vh, 0, 0), link_run<M>(U, Vh, 1, 0), link_run<M>(U, Vh, 2, 0)};
+      V = link_staple<T, M, MU>(L, Ub, x, old);
+    } else {
+      V = link_staple_rt<T, M>(L, U, A, F, x, mu, old);
+    }
+    const int res = link_move<T, M, KIND>(L, V, old, a1, a2, r, true, nu);
+    if (res == 1) stU<M>(U, Vh, mu, par, s, nu);
+    return res != 0;
   } else if constexpr (KIND == SU2HIP_K_U1_METROPOLIS) {
     // metro_u1link (src/metropolis.c:48-70) with localact_u1link
     // (src/su2u1.c:336-354) evaluated as a difference
