@@ -77,7 +77,7 @@ struct Step {
 };
 
 struct Ev {
-  int kind;
+  int kind, passes;
   hipEvent_t a, b;
 };
 
@@ -90,6 +90,19 @@ struct AltMap {
   int nblk = 0, cap = 0;
   std::vector<BlockMap> h;
 };
+
+// Tiles of the paired link passes, one table per direction in one device
+// array, and their counters [6 kinds][2][n] (fold_pairs).
+struct PairMap {
+  PairTile *d = nullptr;
+  long long *d_cnt = nullptr;
+  void *mem = nullptr;  // the lattices' second link buffers (LatDesc::Ualt)
+  size_t bytes = 0;
+  int n = 0, cap = 0;
+  int first[3] = {}, count[3] = {}, threads[3] = {};
+  std::vector<PairTile> h;
+};
+constexpr int PAIR_KINDS = 6;
 
 constexpr int NCHUNK = 3;
 constexpr int CHUNKS[NCHUNK] = {64, 128, 256};
@@ -128,6 +141,11 @@ struct su2hip_batch {
   double kms[SU2HIP_NKINDS] = {};
   long long kcount[SU2HIP_NKINDS] = {};
   AltMap alt[2];                  // chunks 64 and 128; 256 is the main table
+  PairMap pair;                   // paired link passes
+  bool pair_on = false;           // sweeps take them
+  // tables whose counters may be nonzero (1 << k), of the launches made and of
+  // the captured sweep: 0 the main table, 1 and 2 alt, 3 pair
+  unsigned touched = 0, graph_touched = 0;
   hipStream_t flow_stream = nullptr;  // asynchronous flows (su2hip_flow_start)
   int tune[SU2HIP_NKINDS] = {};   // chunk per pass kind, 0 = chosen by size
   int waves[SU2HIP_NKINDS] = {};  // occupancy target per pass kind (su2hip_set_waves)
@@ -274,7 +292,9 @@ static LaunchCtx ctx_for(su2hip_batch *b, int kind) {
       c.nblk = b->alt[k].nblk;
       c.cnt = b->alt[k].d_cnt;
       c.block = ch;
+      b->touched |= 2u << k;
     }
+  if (c.block == BLK) b->touched |= 1;
   return c;
 }
 
@@ -296,6 +316,7 @@ static void fill_desc(Slot &s) {
   L.G = p.triplet ? take(6 * Vh) : nullptr;
   L.S = p.singlet ? take(2 * Vh) : nullptr;
   L.H = s.hop_mem;
+  L.Ualt = nullptr;  // build_pairs
   L.B = s.bu_mem;
   L.L0 = p.L[0];
   L.L1 = p.L[1];
@@ -450,9 +471,29 @@ static int fold_table(su2hip_batch *b, long long *d_cnt, int nblk, const std::ve
   return SU2HIP_OK;
 }
 
+static int fold_pairs(su2hip_batch *b) {
+  PairMap &m = b->pair;
+  if (!m.d_cnt || m.n == 0) return SU2HIP_OK;
+  size_t n = (size_t)PAIR_KINDS * 2 * m.n;
+  std::vector<long long> h(n);
+  HIPTRY(hipMemcpyAsync(h.data(), m.d_cnt, n * sizeof(long long), hipMemcpyDeviceToHost, b->stream));
+  HIPTRY(hipMemsetAsync(m.d_cnt, 0, n * sizeof(long long), b->stream));
+  HIPTRY(hipStreamSynchronize(b->stream));
+  for (int k = 0; k < PAIR_KINDS; k++)
+    for (int i = 0; i < m.n; i++) {
+      long long a = h[(size_t)(k * 2) * m.n + i], t = h[(size_t)(k * 2 + 1) * m.n + i];
+      if (a || t) add_counts(b->slots[m.h[i].lat].cnt, k, a, t);
+    }
+  return SU2HIP_OK;
+}
+
 static int fold_counts(su2hip_batch *b) {
-  int rc = fold_table(b, b->d_cnt, b->nblk, b->h_blk);
-  for (int k = 0; k < 2 && !rc; k++) rc = fold_table(b, b->alt[k].d_cnt, b->alt[k].nblk, b->alt[k].h);
+  int rc = SU2HIP_OK;
+  if (b->touched & 1) rc = fold_table(b, b->d_cnt, b->nblk, b->h_blk);
+  for (int k = 0; k < 2 && !rc; k++)
+    if (b->touched & (2u << k)) rc = fold_table(b, b->alt[k].d_cnt, b->alt[k].nblk, b->alt[k].h);
+  if (!rc && (b->touched & 8)) rc = fold_pairs(b);
+  if (!rc) b->touched = 0;
   return rc;
 }
 
@@ -498,6 +539,179 @@ static int build_alt(su2hip_batch *b, AltMap &m, int chunk) {
                           b->stream));
     HIPTRY(hipMemsetAsync(m.d_cnt, 0, sizeof(long long) * NCOUNT * 2 * n, b->stream));
   }
+  return SU2HIP_OK;
+}
+
+// Paired link passes up to these many sites of a handle.  A sweep with five
+// link rounds, single -> paired passes: FP32 32^3 132 -> 114 us, 40^3 142 ->
+// 127, 48^3 147 -> 139, but 52^3 157 -> 161; FP64 with U(1) 32^3 218 -> 200,
+// 40^3 240 -> 231, sixteen of 16^3 222 -> 201, but 44^3 245 -> 270.
+constexpr uint64_t PAIR_SITES_FP32 = 120000, PAIR_SITES_FP64 = 65536;
+
+// Tiles of link direction dir in one lattice: whole rows in x and n1 of them
+// in the other transverse direction, or for direction 0 boxes of at most nx by
+// n1 by n2.
+struct PairShape {
+  int n[3], halo[3], count[3];
+  int tiles() const { return count[0] * count[1] * count[2]; }
+  int threads() const { return n[0] * (n[1] + 2 * halo[1]) * (n[2] + 2 * halo[2]); }
+};
+
+static PairShape pair_shape(const LatDesc &L, int dir, int nx, int n1, int n2) {
+  const int ext[3] = {L.h0, L.L1, L.L2};
+  PairShape p{{L.h0, 1, 1}, {0, 0, 0}, {}};
+  if (dir == 0) {
+    // the boxes of a row equally wide
+    const int k = (L.h0 + nx - 1) / nx;
+    p.n[0] = (L.h0 + k - 1) / k;
+    p.n[1] = n1;
+    p.n[2] = n2;
+  } else {
+    p.n[3 - dir] = n1;
+  }
+  for (int d = 0; d < 3; d++) {
+    if (d && d != dir) {
+      p.halo[d] = p.n[d] + 2 < ext[d];
+      if (!p.halo[d]) p.n[d] = ext[d];
+    }
+    p.count[d] = (ext[d] + p.n[d] - 1) / p.n[d];
+  }
+  return p;
+}
+
+static void pair_tiles(int lat, const LatDesc &L, const PairShape &p, std::vector<PairTile> &v) {
+  for (int z = 0; z < L.L2; z += p.n[2])
+    for (int y = 0; y < L.L1; y += p.n[1])
+      for (int x = 0; x < L.h0; x += p.n[0]) {
+        PairTile t;
+        t.lat = lat;
+        t.xh0 = x;
+        t.nx = std::min(p.n[0], L.h0 - x);
+        t.y0 = y;
+        t.ny = std::min(p.n[1], L.L1 - y);
+        t.z0 = z;
+        t.nz = std::min(p.n[2], L.L2 - z);
+        t.hy = p.halo[1];
+        t.hz = p.halo[2];
+        t.dx = make_fastdiv((uint32_t)t.nx);
+        t.dy0 = make_fastdiv((uint32_t)(t.ny + 2 * t.hy));
+        t.dy1 = make_fastdiv((uint32_t)t.ny);
+        v.push_back(t);
+      }
+}
+
+// The shape for all lattices of the handle: of those that fit a workgroup the
+// one with the fewest waves of the first phase on the busiest of 256 CUs,
+// then the fewest waves of both phases in all, then the smaller tile.  A
+// round of three pairs in FP32: 32^3 12.3-12.4 us with 256 tiles of 3 + 1
+// waves, 12.6-12.8 with 4 + 2 on fewer CUs, 17 with 256 tiles' work on 128;
+// 48^3 15.7-16.0 at 6 waves a CU, 16.5-17.2 at 8-10.  False if none fits.
+static bool pair_choose(const su2hip_batch *b, int dir, int sel[3], int &threads) {
+  long best = -1;
+  for (int nx = 32; nx >= (dir ? 32 : 4); nx -= 4)
+    for (int n1 = 8; n1 >= 2; n1--)
+      for (int n2 = dir ? 1 : n1; n2 >= (dir ? 1 : 2); n2--) {
+        long tiles = 0;
+        int thr = 1, core = 1;
+        for (int i = 0; i < b->max_slots; i++) {
+          if (!b->slots[i].used) continue;
+          const PairShape p = pair_shape(b->slots[i].hd, dir, nx, n1, n2);
+          tiles += p.tiles();
+          thr = std::max(thr, p.threads());
+          core = std::max(core, p.n[0] * p.n[1] * p.n[2]);
+        }
+        if (thr > PAIR_THREADS) continue;
+        const long w0 = (thr + 63) / 64, w1 = (core + 63) / 64;
+        const long cost = ((tiles + 255) / 256 * w0 << 32) + tiles * (w0 + w1);
+        if (best >= 0 && cost > best) continue;
+        best = cost;
+        sel[0] = nx;
+        sel[1] = n1;
+        sel[2] = n2;
+        threads = (thr + 63) / 64 * 64;
+      }
+  return best >= 0;
+}
+
+static void pair_drop(su2hip_batch *b) {
+  PairMap &m = b->pair;
+  if (b->pair_on) b->graph_valid = false;
+  b->pair_on = false;
+  if (m.mem) {
+    (void)hipStreamSynchronize(b->stream);
+    (void)hipFree(m.mem);
+  }
+  m.mem = nullptr;
+  m.bytes = 0;
+}
+
+// Paired link passes for the lattices of the handle, where they gain
+// (k_pair_link) and their buffers fit the HBM budget; else single passes.
+static int build_pairs(su2hip_batch *b) {
+  PairMap &m = b->pair;
+  uint64_t sites = 0;
+  size_t bytes = 0;
+  bool ok = b->tmpl.nhiggs < 2;
+  for (int i = 0; i < b->max_slots; i++) {
+    Slot &s = b->slots[i];
+    s.hd.Ualt = nullptr;
+    if (!s.used) continue;
+    sites += 2 * (uint64_t)s.hd.Vh;
+    bytes += align256(link_words(s.p) * wsize(s.p));
+    ok = ok && s.hd.h0 <= PAIR_THREADS / 4;
+  }
+  ok = ok && sites && sites <= (b->fp64 ? PAIR_SITES_FP64 : PAIR_SITES_FP32);
+  if (ok && bytes > m.bytes) {
+    pair_drop(b);
+    if ((b->hbm_budget && b->used + bytes > b->hbm_budget) || hipMalloc(&m.mem, bytes) != hipSuccess) {
+      m.mem = nullptr;
+      ok = false;
+    } else {
+      m.bytes = bytes;
+    }
+  }
+  if (!ok) {
+    pair_drop(b);
+    m.n = 0;
+    return SU2HIP_OK;
+  }
+  char *q = (char *)m.mem;
+  for (int i = 0; i < b->max_slots; i++) {
+    Slot &s = b->slots[i];
+    if (!s.used) continue;
+    s.hd.Ualt = q;
+    q += align256(link_words(s.p) * wsize(s.p));
+  }
+  m.h.clear();
+  for (int dir = 0; dir < 3; dir++) {
+    int sel[3];
+    if (!pair_choose(b, dir, sel, m.threads[dir])) {
+      pair_drop(b);
+      m.n = 0;
+      return SU2HIP_OK;
+    }
+    m.first[dir] = (int)m.h.size();
+    for (int i = 0; i < b->max_slots; i++)
+      if (b->slots[i].used)
+        pair_tiles(i, b->slots[i].hd, pair_shape(b->slots[i].hd, dir, sel[0], sel[1], sel[2]), m.h);
+    m.count[dir] = (int)m.h.size() - m.first[dir];
+  }
+  m.n = (int)m.h.size();
+  if (m.n > m.cap) {
+    if (m.d) HIPTRY(hipFree(m.d));
+    if (m.d_cnt) HIPTRY(hipFree(m.d_cnt));
+    m.d = nullptr;
+    m.d_cnt = nullptr;
+    m.cap = 0;
+    if (hipMalloc(&m.d, sizeof(PairTile) * m.n) != hipSuccess ||
+        hipMalloc(&m.d_cnt, sizeof(long long) * PAIR_KINDS * 2 * m.n) != hipSuccess)
+      return fail(SU2HIP_ENOMEM, "tile table allocation failed");
+    m.cap = m.n;
+  }
+  HIPTRY(hipMemcpyAsync(m.d, m.h.data(), sizeof(PairTile) * m.n, hipMemcpyHostToDevice, b->stream));
+  HIPTRY(hipMemsetAsync(m.d_cnt, 0, sizeof(long long) * PAIR_KINDS * 2 * m.n, b->stream));
+  HIPTRY(hipStreamSynchronize(b->stream));
+  b->pair_on = true;
   return SU2HIP_OK;
 }
 
@@ -552,6 +766,7 @@ static int rebuild_map(su2hip_batch *b) {
     HIPTRY(hipMemsetAsync(b->d_cnt, 0, sizeof(long long) * NCOUNT * 2 * n, b->stream));
   }
   for (int k = 0; k < 2 && !rc; k++) rc = build_alt(b, b->alt[k], CHUNKS[k]);
+  if (!rc) rc = build_pairs(b);
   if (rc) return rc;
   rc = push_desc(b);
   if (rc) return rc;
@@ -663,9 +878,9 @@ static hipEvent_t ev_get(su2hip_batch *b) {
   return e;
 }
 
-// run fn() bracketed by timing events when timing is on
+// run fn() bracketed by timing events when timing is on, as passes launches
 template <typename Fn>
-static hipError_t timed(su2hip_batch *b, int kind, Fn &&fn) {
+static hipError_t timed(su2hip_batch *b, int kind, int passes, Fn &&fn) {
   if (!b->timing) return fn();
   hipEvent_t a = ev_get(b), e = ev_get(b);
   if (!a || !e) return hipErrorOutOfMemory;
@@ -674,14 +889,15 @@ static hipError_t timed(su2hip_batch *b, int kind, Fn &&fn) {
   r = fn();
   if (r != hipSuccess) return r;
   r = hipEventRecord(e, b->stream);
-  b->pending.push_back(Ev{kind, a, e});
+  b->pending.push_back(Ev{kind, passes, a, e});
   return r;
 }
 
 // in_sweep: the step is part of a compound sweep, whose random pass order
 // (when on) replaces the step's parity and link direction
-static hipError_t enqueue_step(su2hip_batch *b, const Step &st, bool in_sweep = true) {
+static hipError_t enqueue_step(su2hip_batch *b, const Step &st, int alt, bool in_sweep = true) {
   LaunchCtx c = ctx_of(b);
+  c.alt = alt;
   if (in_sweep && b->random_order) {
     c.order = b->d_order;
     c.npass = b->passes;
@@ -689,19 +905,21 @@ static hipError_t enqueue_step(su2hip_batch *b, const Step &st, bool in_sweep = 
   int reunit = b->tmpl.reunitarize && !b->fp64;
   if (!st.muca) {
     LaunchCtx ct = ctx_for(b, st.kind);
+    ct.alt = alt;
     ct.order = c.order;
     ct.npass = c.npass;
-    return timed(b, st.kind, [&] {
+    return timed(b, st.kind, 1, [&] {
       return launch_pass(ct, st.kind, st.parity, st.dir, st.pass_off, -1, reunit);
     });
   }
   c.waves = b->waves[st.kind];  // multicanonical steps keep the 256-site table
+  b->touched |= 1;
   for (int k = 0; k < b->muca_steps; k++) {
-    hipError_t e = timed(b, st.kind, [&] {
+    hipError_t e = timed(b, st.kind, 1, [&] {
       return launch_pass(c, st.kind, st.parity, st.dir, st.pass_off, k, reunit);
     });
     if (e != hipSuccess) return e;
-    e = timed(b, SU2HIP_K_MUCA,
+    e = timed(b, SU2HIP_K_MUCA, 1,
               [&] { return launch_muca_accept(c, st.kind, st.dir, st.parity, st.pass_off, k); });
     if (e != hipSuccess) return e;
   }
@@ -714,11 +932,21 @@ static bool su2_link_kind(int kind) {
          kind == SU2HIP_K_LINK_OVERRELAX;
 }
 
+// steps i and i + 1 of the schedule are the two parities of one link
+// direction, of a kind that k_pair_link takes
+static bool pairable(const su2hip_batch *b, size_t i) {
+  if (!b->pair_on || b->random_order || i + 1 >= b->sched.size()) return false;
+  const Step &s = b->sched[i], &n = b->sched[i + 1];
+  return (s.kind == SU2HIP_K_LINK_HEATBATH || s.kind == SU2HIP_K_LINK_OVERRELAX) &&
+         n.kind == s.kind && n.dir == s.dir && s.parity == 0 && n.parity == 1 &&
+         n.pass_off == s.pass_off + 1;
+}
+
 static hipError_t enqueue_sweep(su2hip_batch *b) {
   if (b->random_order) {
     const su2hip_params &p = b->tmpl;
     LaunchCtx c = ctx_of(b);
-    hipError_t e = timed(b, SU2HIP_K_AUX, [&] {
+    hipError_t e = timed(b, SU2HIP_K_AUX, 1, [&] {
       return launch_order(c, b->d_order, b->d_info, b->passes, p.update_links, p.scalar_sweeps + 1);
     });
     if (e != hipSuccess) return e;
@@ -727,18 +955,39 @@ static hipError_t enqueue_sweep(su2hip_batch *b) {
   // doublet and the U(1) links change only in the passes between rounds
   bool hop_fresh = false;
   LaunchCtx c = ctx_of(b);
-  for (const Step &st : b->sched) {
+  for (size_t i = 0; i < b->sched.size(); i++) {
+    const Step &st = b->sched[i];
     hipError_t e = hipSuccess;
     if (!su2_link_kind(st.kind))
       hop_fresh = false;
     else if (!hop_fresh && b->hop_on) {
-      e = timed(b, SU2HIP_K_AUX, [&] { return launch_hop(c); });
+      e = timed(b, SU2HIP_K_AUX, 1, [&] { return launch_hop(c); });
       hop_fresh = true;
     }
-    if (e == hipSuccess) e = enqueue_step(b, st);
+    if (e == hipSuccess && pairable(b, i)) {
+      // SU(2) link passes come in rounds of all three directions, so the
+      // passes of other kinds find c.alt 0 or ALT_LINKS
+      const PairMap &m = b->pair;
+      const int d = st.dir;
+      e = timed(b, st.kind, 2, [&] {
+        return launch_pair_link(c, m.d + m.first[d], m.count[d], m.threads[d], st.kind, d, st.pass_off,
+                                m.d_cnt + m.first[d], m.n);
+      });
+      b->touched |= 8;
+      c.alt ^= 1 << d;
+      i++;
+    } else if (e == hipSuccess) {
+      e = enqueue_step(b, st, c.alt);
+    }
     if (e != hipSuccess) return e;
   }
-  return timed(b, SU2HIP_K_AUX, [&] { return launch_end_sweep(c, b->passes); });
+  // between sweeps every field is in its first buffer
+  if (c.alt) {
+    hipError_t e = timed(b, SU2HIP_K_AUX, 1, [&] { return launch_pair_close(c); });
+    if (e != hipSuccess) return e;
+    c.alt = 0;
+  }
+  return timed(b, SU2HIP_K_AUX, 1, [&] { return launch_end_sweep(c, b->passes); });
 }
 
 // device tables of the random pass order for the current schedule
@@ -811,12 +1060,20 @@ static int resolve_links(int n, const su2hip_params *params) {
   return bytes > SU2HIP_LINKS_PACKED_ABOVE ? SU2HIP_LINKS_PACKED : SU2HIP_LINKS_FULL;
 }
 
+// whether bytes more would exceed the handle's HBM budget; the second link
+// buffers of paired passes give way to any other use
+static bool over_budget(su2hip_batch *b, size_t bytes) {
+  if (!b->hbm_budget) return false;
+  if (b->used + b->pair.bytes + bytes > b->hbm_budget) pair_drop(b);
+  return b->used + bytes > b->hbm_budget;
+}
+
 // the slot's hopping-term cache, inside the handle's HBM budget
 static int hop_alloc(su2hip_batch *b, int i) {
   Slot &s = b->slots[i];
   size_t bytes = hop_cache_bytes(s.p);
   if (s.hop_mem || bytes == 0) return SU2HIP_OK;
-  if (b->hbm_budget && b->used + bytes > b->hbm_budget)
+  if (over_budget(b, bytes))
     return fail(SU2HIP_ENOMEM, "HBM budget: %llu + %zu bytes of hopping-term cache exceeds %llu",
                 (unsigned long long)b->used, bytes, (unsigned long long)b->hbm_budget);
   if (hipMalloc(&s.hop_mem, bytes) != hipSuccess) {
@@ -860,7 +1117,7 @@ static int alloc_slot(su2hip_batch *b, int i, const su2hip_params &p_in) {
   su2hip_params p = p_in;
   p.link_format = b->tmpl.link_format;  // the handle's resolved storage
   size_t bytes = slot_bytes(p);
-  if (b->hbm_budget && b->used + bytes > b->hbm_budget)
+  if (over_budget(b, bytes))
     return fail(SU2HIP_ENOMEM, "HBM budget: %llu + %zu bytes exceeds %llu",
                 (unsigned long long)b->used, bytes, (unsigned long long)b->hbm_budget);
   Slot &s = b->slots[i];
@@ -1092,6 +1349,9 @@ int su2hip_destroy(su2hip_batch_t *b) {
     if (m.d_blk) (void)hipFree(m.d_blk);
     if (m.d_cnt) (void)hipFree(m.d_cnt);
   }
+  if (b->pair.mem) (void)hipFree(b->pair.mem);
+  if (b->pair.d) (void)hipFree(b->pair.d);
+  if (b->pair.d_cnt) (void)hipFree(b->pair.d_cnt);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   if (b->flow_stream) (void)hipStreamDestroy(b->flow_stream);
   delete b;
@@ -1292,7 +1552,11 @@ int su2hip_update(su2hip_batch_t *b, int n_sweeps) {
       b->gexec = nullptr;
       hipGraph_t g = nullptr;
       HIPTRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+      const unsigned before = b->touched;
+      b->touched = 0;
       hipError_t e = enqueue_sweep(b);
+      b->graph_touched = b->touched;
+      b->touched = before;
       hipError_t e2 = hipStreamEndCapture(b->stream, &g);
       if (e != hipSuccess || e2 != hipSuccess) {
         if (g) (void)hipGraphDestroy(g);
@@ -1304,6 +1568,7 @@ int su2hip_update(su2hip_batch_t *b, int n_sweeps) {
       if (e != hipSuccess) return fail(SU2HIP_EDEVICE, "graph instantiate: %s", hipGetErrorString(e));
       b->graph_valid = true;
     }
+    b->touched |= b->graph_touched;
     for (int i = 0; i < n_sweeps; i++) HIPTRY(hipGraphLaunch(b->gexec, b->stream));
     return SU2HIP_OK;
   }
@@ -1353,7 +1618,7 @@ int su2hip_pass(su2hip_batch_t *b, int kind, int parity, int dir) {
   for (auto &s : b->slots)
     if (s.used && field && muca_on_field(s.hm, field)) muca = true;
   hipError_t e = b->hop_on && su2_link_kind(kind) ? launch_hop(ctx_of(b)) : hipSuccess;
-  if (e == hipSuccess) e = enqueue_step(b, Step{kind, parity, dir, 0, muca, 0}, false);
+  if (e == hipSuccess) e = enqueue_step(b, Step{kind, parity, dir, 0, muca, 0}, 0, false);
   if (e == hipErrorInvalidValue)
     return fail(SU2HIP_EINVAL, "kind %d is not part of this model", kind);
   if (e != hipSuccess) return fail(SU2HIP_EDEVICE, "pass launch: %s", hipGetErrorString(e));
@@ -1514,7 +1779,7 @@ int su2hip_measure_all(su2hip_batch_t *b, double *sums) {
   int rc = prepare(b);
   if (rc) return rc;
   LaunchCtx c = ctx_of(b);
-  hipError_t e = timed(b, SU2HIP_K_MEASURE, [&] { return launch_measure(c); });
+  hipError_t e = timed(b, SU2HIP_K_MEASURE, 1, [&] { return launch_measure(c); });
   if (e != hipSuccess) return fail(SU2HIP_EDEVICE, "measure: %s", hipGetErrorString(e));
   HIPTRY(hipMemcpyAsync(sums, b->d_sums, sizeof(double) * SU2HIP_NSUMS * b->max_slots,
                         hipMemcpyDeviceToHost, b->stream));
@@ -1629,7 +1894,7 @@ int su2hip_muca_set(su2hip_batch_t *b, int slot, const su2hip_muca *m, const dou
     size_t Vh = (size_t)vol_of(s.p) / 2;
     bub = align256((s.p.nhiggs ? 8 : 6) * Vh * wsize(s.p));
     if (!s.bu_mem) {
-      if (b->hbm_budget && b->used + bub > b->hbm_budget)
+      if (over_budget(b, bub))
         return fail(SU2HIP_ENOMEM, "HBM budget exceeded by the multicanonical backup");
       if (hipMalloc(&newbu, bub) != hipSuccess) return fail(SU2HIP_ENOMEM, "backup allocation");
     }
@@ -2042,7 +2307,7 @@ static int flow_enqueue(su2hip_batch *b, int slot, int scheme, double dt, double
   size_t Vh = (size_t)vol_of(p) / 2, w = wsize(p);
   if (!s.flow_mem) {
     size_t fb = align256(flow_words(p) * w) + 4096;
-    if (b->hbm_budget && b->used + fb > b->hbm_budget)
+    if (over_budget(b, fb))
       return fail(SU2HIP_ENOMEM, "HBM budget exceeded by the flow buffers");
     if (hipMalloc(&s.flow_mem, fb) != hipSuccess) return fail(SU2HIP_ENOMEM, "flow buffers");
     s.flow_bytes = fb;
@@ -2134,7 +2399,7 @@ static int flow_enqueue(su2hip_batch *b, int slot, int scheme, double dt, double
   };
   auto row = [&]() -> hipError_t {
     LaunchCtx c = ctx();
-    hipError_t x = use_timing ? timed(b, SU2HIP_K_MEASURE, [&] { return launch_measure(c); })
+    hipError_t x = use_timing ? timed(b, SU2HIP_K_MEASURE, 1, [&] { return launch_measure(c); })
                               : launch_measure(c);
     if (x == hipSuccess)
       x = hipMemcpyAsync(j.d_rows + r * SU2HIP_NSUMS, j.d_sums + (size_t)slot * SU2HIP_NSUMS,
@@ -2153,7 +2418,7 @@ static int flow_enqueue(su2hip_batch *b, int slot, int scheme, double dt, double
         return launch_flow_stage(c, slot, Ub[cur], Ub[1 - cur], Gb[cur], Gb[1 - cur], Z, ZG, h,
                                  msq_t, stage);
       };
-      e = use_timing ? timed(b, SU2HIP_K_FLOW, go) : go();
+      e = use_timing ? timed(b, SU2HIP_K_FLOW, 1, go) : go();
       cur = 1 - cur;
     }
     if (e == hipSuccess && steps[k].second) e = row();
@@ -2269,7 +2534,7 @@ static int resolve_events(su2hip_batch *b) {
     float ms = 0.f;
     HIPTRY(hipEventElapsedTime(&ms, ev.a, ev.b));
     b->kms[ev.kind] += ms;
-    b->kcount[ev.kind]++;
+    b->kcount[ev.kind] += ev.passes;
     b->pool.push_back(ev.a);
     b->pool.push_back(ev.b);
   }

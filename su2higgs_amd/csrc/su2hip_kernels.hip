@@ -1138,7 +1138,7 @@ __device__ __forceinline__ void pin_desc(const LatDesc &L) {
 template <typename T, int M, int KIND>
 __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
                                           const MucaDev *__restrict__ mucas,
-                                          const BlockMap *__restrict__ blk, int one, int chunk,
+                                          const BlockMap *__restrict__ blk, int one, int chunk, int alt,
                                           int par_in, int mu_in, int pass_off, int step, int reunit,
                                           long long *__restrict__ cnt, int nblk,
                                           double *__restrict__ partial,
@@ -1146,8 +1146,9 @@ __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
                                           double *lds) {
   int idx;
   const BlockMap bm = block_of(blk, nblk, one, chunk, pass_off & 1, idx);
-  const LatDesc L = lats[bm.lat];
+  LatDesc L = lats[bm.lat];
   pin_desc<M, KIND>(L);
+  if (alt) L.U = L.Ualt;
   if (!L.active || L.budget == 0) return;
   int par = par_in, mu = mu_in;
   if (order) {
@@ -1222,14 +1223,14 @@ __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
 
 #define K_PASS_ARGS                                                                          \
   const LatDesc *__restrict__ lats, const MucaDev *__restrict__ mucas,                       \
-      const BlockMap *__restrict__ blk, int one, int chunk, int par_in, int mu_in,           \
+      const BlockMap *__restrict__ blk, int one, int chunk, int alt, int par_in, int mu_in,  \
       int pass_off, int step, int reunit, long long *__restrict__ cnt, int nblk, double *__restrict__ partial,       \
       const uint8_t *__restrict__ order, int npass
 
 template <typename T, int M, int KIND>
 __global__ __launch_bounds__(BLK) void k_pass(K_PASS_ARGS) {
   __shared__ double lds[BLK / 64];
-  pass_body<T, M, KIND>(lats, mucas, blk, one, chunk, par_in, mu_in, pass_off, step, reunit, cnt, nblk,
+  pass_body<T, M, KIND>(lats, mucas, blk, one, chunk, alt, par_in, mu_in, pass_off, step, reunit, cnt, nblk,
                         partial, order, npass, lds);
 }
 
@@ -1242,8 +1243,204 @@ template <typename T, int M, int KIND>
 __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(5))) void k_pass_w5(
     K_PASS_ARGS) {
   __shared__ double lds[BLK / 64];
-  pass_body<T, M, KIND>(lats, mucas, blk, one, chunk, par_in, mu_in, pass_off, step, reunit, cnt, nblk,
+  pass_body<T, M, KIND>(lats, mucas, blk, one, chunk, alt, par_in, mu_in, pass_off, step, reunit, cnt, nblk,
                         partial, order, npass, lds);
+}
+
+// ------------------------------------------------------------------------
+// both parities of a link direction in one launch
+//
+// Below some 10^5 sites a sweep is its launches: an empty one takes 1.8 us in
+// a replayed graph and a pass of 32^3 2.8 us.  Here a workgroup updates the
+// first parity in its tile and, where a second-parity link's staple reaches
+// out of the tile, in one more row on each side, keeps those links in LDS,
+// and then updates the second parity.  The staple of direction mu reaches
+// links of mu only in the plane across mu, so a tile needs no margin along
+// mu, and none in x where it holds whole rows.  Margin links are computed by
+// two workgroups from the same inputs and draws, so to the same bits; all are
+// read from one buffer and written to the other, so no workgroup reads what
+// another has already replaced.  Each thread takes at most one site of each
+// parity, and the loads of both are in flight before the first is updated
+// (FP32), or those of the second's first half before the barrier (FP64).
+// Overrelaxation of both parities in a replayed graph, two passes -> one: FP32
+// 8^3 5.3 -> 4.2 us, 32^3 5.6 -> 4.1, FP64 8^3 6.3 -> 5.1, 32^3 6.6 -> 5.1.
+// It is bound by its chain: launch, tile and descriptor, loads, two updates.
+// Larger lattices lose, where the margin's arithmetic and loads cost more than
+// the launch that is saved.
+
+// the links of direction d where `second` says; by the buffers' distance, as
+// a choice between the two members would put the descriptor into scratch
+template <int M, typename T>
+__device__ __forceinline__ T *link_base(const LatDesc &L, int d, int second) {
+  const ptrdiff_t off = second ? (char *)L.Ualt - (char *)L.U : 0;
+  return const_cast<T *>(link_run<M>((const T *)((char *)L.U + off), L.Vh, d, 0));
+}
+
+// the site of a tile at row (ly, lz) counted from its margin's first
+__device__ __forceinline__ Site tile_site(const LatDesc &L, const PairTile &t, int xl, int ly, int lz,
+                                          int par) {
+  Site x;
+  x.y = t.y0 - t.hy + ly;
+  x.y = x.y < 0 ? x.y + L.L1 : (x.y >= L.L1 ? x.y - L.L1 : x.y);
+  x.z = t.z0 - t.hz + lz;
+  x.z = x.z < 0 ? x.z + L.L2 : (x.z >= L.L2 ? x.z - L.L2 : x.z);
+  const int xh = t.xh0 + xl;
+  x.x = 2 * xh + ((par + x.y + x.z) & 1);
+  x.par = par;
+  x.s = xh + L.h0 * (x.y + L.L1 * x.z);
+  return x;
+}
+
+template <typename T, int M, int KIND, int MU>
+__global__ __launch_bounds__(PAIR_THREADS) void k_pair_link(const LatDesc *__restrict__ lats,
+                                                            const PairTile *__restrict__ tiles,
+                                                            int ntiles, int pass_off, int alt,
+                                                            long long *__restrict__ cnt, int ncnt) {
+  __shared__ LinkRaw<M, T> fresh[PAIR_THREADS];
+  // XCD j gets a contiguous run of tiles
+  const int j = (int)(blockIdx.x % NXCD), q = ntiles / (int)NXCD, rem = ntiles % (int)NXCD;
+  const int ti = j * q + (j < rem ? j : rem) + (int)(blockIdx.x / NXCD);
+  const PairTile t = tiles[ti];
+  asm volatile("" ::"s"(t.xh0), "s"(t.nx), "s"(t.y0), "s"(t.ny), "s"(t.z0), "s"(t.nz), "s"(t.hy),
+               "s"(t.hz), "s"(t.dx.m), "s"(t.dy0.m), "s"(t.dy1.m));
+  const LatDesc L = lats[t.lat];
+  pin_desc<M, KIND>(L);
+  asm volatile("" ::"s"(L.Ualt));
+  if (!L.active || L.budget == 0) return;
+  const T *Ub[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) Ub[d] = link_base<M, T>(L, d, (alt >> d) & 1);
+  T *Uo = link_base<M, T>(L, MU, !((alt >> MU) & 1));
+  const T *G = (const T *)L.G;
+  constexpr int N1 = SiteLinks<T, M, MU>::N1, N2 = SiteLinks<T, M, MU>::N2;
+  const int my = t.ny + 2 * t.hy, mz = t.nz + 2 * t.hz;
+  const int i = (int)threadIdx.x, row = (int)fdiv((uint32_t)i, t.dx), xl = i - row * t.nx;
+  // first parity: the tile and its margin rows (but not the margin's corners)
+  const int lz0 = (int)fdiv((uint32_t)row, t.dy0), ly0 = row - lz0 * my;
+  const bool ey = t.hy && (ly0 == 0 || ly0 == my - 1), ez = t.hz && (lz0 == 0 || lz0 == mz - 1);
+  const bool on0 = row < my * mz && !(ey && ez), core0 = on0 && !(ey || ez);
+  // second parity: the tile
+  const int lz1 = (int)fdiv((uint32_t)row, t.dy1) + t.hz, ly1 = row - (lz1 - t.hz) * t.ny + t.hy;
+  const bool on1 = row < t.ny * t.nz;
+  Site x0{}, x1{};
+  SiteLinks<T, M, MU> k0{}, k1{};
+  V3<T> g0a{}, g0b{}, g1a{}, g1b{};
+  Q<T> W{(T)0, (T)0, (T)0, (T)0}, V{(T)1, (T)0, (T)0, (T)0}, old{}, nu;
+  if (on0) {
+    x0 = tile_site(L, t, xl, ly0, lz0, 0);
+    const Site sp = shift(L, x0, MU, +1);
+    k0.s1.load(L, Ub, x0, sp);
+    if constexpr (sizeof(T) == 8) {
+      k0.s1.add_to(W);
+      fence_q(W);
+    }
+    k0.s2.load(L, Ub, x0, sp);
+    k0.load_own(L, Ub, x0, sp);
+    if constexpr ((M & M_TR) != 0) {
+      g0a = G_at(L, G, x0);
+      g0b = G_at(L, G, sp);
+    }
+  }
+  if (on1) x1 = tile_site(L, t, xl, ly1, lz1, 1);
+  const Site sp1 = shift(L, x1, MU, +1);
+  if constexpr (sizeof(T) == 4) {
+    if (on1) {
+      k1.s1.load_nu(L, Ub, x1, sp1);
+      k1.s2.load_nu(L, Ub, x1, sp1);
+      k1.load_own(L, Ub, x1, sp1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  Rng r;
+  rng_init(r, L.key0, L.key1, L.pass + (uint64_t)pass_off, (uint32_t)x0.s);
+  if (on0) {
+    if constexpr (sizeof(T) == 4) k0.s1.add_to(W);
+    k0.s2.add_to(W);
+    old = k0.o.get();
+    V = k0.staple(L, W, x0);
+  }
+  int res = link_move<T, M, KIND>(L, V, old, g0a, g0b, r, on0, nu);
+  if (on0) {
+    const LinkRaw<M, T> w = res == 1 ? raw_link<M, T>(nu) : k0.o;
+    fresh[i] = w;
+    if (core0) stL<M>(par_run<M>(Uo, L.Vh, 0), L.Vh, x0.s, w);
+  }
+  uint64_t am = __ballot(core0 && res != 0), tm = __ballot(core0);
+  int nacc = __popcll(am), ntot = __popcll(tm);
+  if constexpr (sizeof(T) == 8) {
+    if (on1) k1.s1.load_nu(L, Ub, x1, sp1);
+  }
+  __syncthreads();
+  V = Q<T>{(T)1, (T)0, (T)0, (T)0};
+  if (on1) {
+    // the neighbours of the second parity among the fresh links
+    const int l = xl + t.nx * (ly1 + my * lz1);
+    auto near = [&](int d, int &p, int &m) {
+      if (d == 0) {  // whole rows
+        p = l - xl + (shift(L, x1, 0, +1).x >> 1);
+        m = l - xl + (shift(L, x1, 0, -1).x >> 1);
+      } else if (d == 1) {
+        p = l + t.nx * (t.hy || ly1 + 1 < my ? 1 : 1 - my);
+        m = l - t.nx * (t.hy || ly1 > 0 ? 1 : 1 - my);
+      } else {
+        p = l + t.nx * my * (t.hz || lz1 + 1 < mz ? 1 : 1 - mz);
+        m = l - t.nx * my * (t.hz || lz1 > 0 ? 1 : 1 - mz);
+      }
+    };
+    W = Q<T>{(T)0, (T)0, (T)0, (T)0};
+    int p, m;
+    near(N1, p, m);
+    k1.s1.xn = fresh[p];
+    k1.s1.xm_mu = fresh[m];
+    k1.s1.add_to(W);
+    if constexpr (sizeof(T) == 8) {
+      fence_q(W);
+      k1.s2.load_nu(L, Ub, x1, sp1);
+      k1.load_own(L, Ub, x1, sp1);
+    }
+    if constexpr ((M & M_TR) != 0) {
+      g1a = G_at(L, G, x1);
+      g1b = G_at(L, G, sp1);
+    }
+    near(N2, p, m);
+    k1.s2.xn = fresh[p];
+    k1.s2.xm_mu = fresh[m];
+    k1.s2.add_to(W);
+    old = k1.o.get();
+    V = k1.staple(L, W, x1);
+  }
+  rng_init(r, L.key0, L.key1, L.pass + (uint64_t)(pass_off + 1), (uint32_t)(L.Vh + x1.s));
+  res = link_move<T, M, KIND>(L, V, old, g1a, g1b, r, on1, nu);
+  if (on1) stL<M>(par_run<M>(Uo, L.Vh, 1), L.Vh, x1.s, res == 1 ? raw_link<M, T>(nu) : k1.o);
+  am = __ballot(on1 && res != 0);
+  tm = __ballot(on1);
+  nacc += __popcll(am);
+  ntot += __popcll(tm);
+  if ((threadIdx.x & 63) == 0 && ntot) {
+    count_up(&cnt[(size_t)(KIND * 2 + 0) * ncnt + ti], nacc);
+    count_up(&cnt[(size_t)(KIND * 2 + 1) * ncnt + ti], ntot);
+  }
+}
+
+// links in the second buffer back to the first, at the end of a sweep that
+// paired an odd number of rounds
+template <typename T, int M>
+__global__ __launch_bounds__(BLK) void k_pair_close(const LatDesc *__restrict__ lats,
+                                                    const BlockMap *__restrict__ blk, int nblk, int one,
+                                                    int alt) {
+  int idx;
+  const BlockMap bm = block_of(blk, nblk, one, BLK, 0, idx);
+  const LatDesc L = lats[bm.lat];
+  if (!L.active || L.budget == 0) return;
+  const int s = bm.s0 + (int)threadIdx.x;
+  if (s >= L.Vh) return;
+#pragma unroll
+  for (int d = 0; d < 3; d++)
+    if ((alt >> d) & 1)
+#pragma unroll
+      for (int par = 0; par < 2; par++)
+        stL<M>((T *)link_run<M>((const T *)L.U, L.Vh, d, par), L.Vh, s,
+               ldL<M>(link_run<M>((const T *)L.Ualt, L.Vh, d, par), L.Vh, s));
 }
 
 // The hopping-term cache of one doublet: for every link, the doublet part
@@ -2690,15 +2887,16 @@ static hipError_t pass_one(const LaunchCtx &c, int parity, int dir, int pass_off
     // multicanonical steps use the 256-site table: their order-parameter
     // partials are indexed by 256-site chunk
     if (step >= 0 && c.block != BLK) return hipErrorInvalidValue;
+    if (c.alt != 0 && c.alt != ALT_LINKS) return hipErrorInvalidValue;
     if constexpr (KIND == SU2HIP_K_LINK_OVERRELAX) {
       if (c.waves == 5) {
         if (c.ev_start || c.ev_stop) {
           hipExtLaunchKernelGGL((k_pass_w5<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream,
-                                c.ev_start, c.ev_stop, 0, c.desc, c.muca, c.blk, c.one, c.block, parity, dir,
+                                c.ev_start, c.ev_stop, 0, c.desc, c.muca, c.blk, c.one, c.block, c.alt, parity, dir,
                                 pass_off, step, reunit, c.cnt, c.nblk, c.partial, c.order, c.npass);
         } else {
           hipLaunchKernelGGL((k_pass_w5<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream,
-                             c.desc, c.muca, c.blk, c.one, c.block, parity, dir, pass_off, step, reunit, c.cnt,
+                             c.desc, c.muca, c.blk, c.one, c.block, c.alt, parity, dir, pass_off, step, reunit, c.cnt,
                              c.nblk, c.partial, c.order, c.npass);
         }
         return hipGetLastError();
@@ -2706,11 +2904,11 @@ static hipError_t pass_one(const LaunchCtx &c, int parity, int dir, int pass_off
     }
     if (c.ev_start || c.ev_stop) {
       hipExtLaunchKernelGGL((k_pass<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream,
-                            c.ev_start, c.ev_stop, 0, c.desc, c.muca, c.blk, c.one, c.block, parity, dir, pass_off,
+                            c.ev_start, c.ev_stop, 0, c.desc, c.muca, c.blk, c.one, c.block, c.alt, parity, dir, pass_off,
                             step, reunit, c.cnt, c.nblk, c.partial, c.order, c.npass);
     } else {
       hipLaunchKernelGGL((k_pass<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream, c.desc,
-                         c.muca, c.blk, c.one, c.block, parity, dir, pass_off, step, reunit, c.cnt, c.nblk,
+                         c.muca, c.blk, c.one, c.block, c.alt, parity, dir, pass_off, step, reunit, c.cnt, c.nblk,
                          c.partial, c.order, c.npass);
     }
     return hipGetLastError();
@@ -2738,6 +2936,52 @@ hipError_t launch_pass(const LaunchCtx &c, int kind, int parity, int dir, int pa
         case SU2HIP_K_SINGLET_METROPOLIS: return pass_one<T, M, SU2HIP_K_SINGLET_METROPOLIS>(c, parity, dir, pass_off, muca_step, reunit);
       }
       return hipErrorInvalidValue;
+    });
+  });
+}
+
+template <typename T, int M, int KIND>
+static hipError_t pair_one(const LaunchCtx &c, const PairTile *tiles, int ntiles, int threads, int dir,
+                           int pass_off, long long *cnt, int ncnt) {
+  auto go = [&](auto mu) {
+    hipLaunchKernelGGL((k_pair_link<T, M, KIND, decltype(mu)::value>), dim3(ntiles), dim3(threads), 0,
+                       c.stream, c.desc, tiles, ntiles, pass_off, c.alt, cnt, ncnt);
+    return hipGetLastError();
+  };
+  if (dir == 0) return go(std::integral_constant<int, 0>{});
+  if (dir == 1) return go(std::integral_constant<int, 1>{});
+  return go(std::integral_constant<int, 2>{});
+}
+
+hipError_t launch_pair_link(const LaunchCtx &c, const PairTile *tiles, int ntiles, int threads,
+                            int kind, int dir, int pass_off, long long *cnt, int ncnt) {
+  if (ntiles == 0) return hipSuccess;
+  if (threads < 1 || threads > PAIR_THREADS || threads % 64 || dir < 0 || dir > 2)
+    return hipErrorInvalidValue;
+  return with_prec(c.fp64, [&](auto t) {
+    using T = decltype(t);
+    return with_model_of<T>(c.model, [&](auto m) -> hipError_t {
+      constexpr int M = decltype(m)::value;
+      if constexpr ((M & M_H2) == 0) {
+        if (kind == SU2HIP_K_LINK_HEATBATH)
+          return pair_one<T, M, SU2HIP_K_LINK_HEATBATH>(c, tiles, ntiles, threads, dir, pass_off, cnt, ncnt);
+        if (kind == SU2HIP_K_LINK_OVERRELAX)
+          return pair_one<T, M, SU2HIP_K_LINK_OVERRELAX>(c, tiles, ntiles, threads, dir, pass_off, cnt, ncnt);
+      }
+      return hipErrorInvalidValue;
+    });
+  });
+}
+
+hipError_t launch_pair_close(const LaunchCtx &c) {
+  if (c.nblk == 0 || c.alt == 0) return hipSuccess;
+  return with_prec(c.fp64, [&](auto t) {
+    using T = decltype(t);
+    return with_model_of<T>(c.model, [&](auto m) -> hipError_t {
+      constexpr int M = decltype(m)::value;
+      hipLaunchKernelGGL((k_pair_close<T, M>), dim3(c.nblk), dim3(BLK), 0, c.stream, c.desc, c.blk,
+                         c.nblk, c.one, c.alt);
+      return hipGetLastError();
     });
   });
 }
