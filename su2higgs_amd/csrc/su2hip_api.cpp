@@ -91,18 +91,26 @@ struct AltMap {
   std::vector<BlockMap> h;
 };
 
-// Tiles of the paired link passes, one table per direction in one device
-// array, and their counters [6 kinds][2][n] (fold_pairs).
+// Tiles of the paired passes, in one device array one table per direction of
+// the links and one of the scalars, and their counters: of each table [kinds]
+// [2][its tiles], for the kinds that use it.
+constexpr int PAIR_TABLES = 4, PAIR_SCALARS = 3;
 struct PairMap {
   PairTile *d = nullptr;
   long long *d_cnt = nullptr;
-  void *mem = nullptr;  // the lattices' second link buffers (LatDesc::Ualt)
+  void *mem = nullptr;  // the lattices' second buffers (LatDesc::Ualt ...)
   size_t bytes = 0;
-  int n = 0, cap = 0;
-  int first[3] = {}, count[3] = {}, threads[3] = {};
+  int n = 0;
+  size_t cap = 0, cnt_cap = 0, ncnt = 0;
+  int first[PAIR_TABLES] = {}, count[PAIR_TABLES] = {}, threads[PAIR_TABLES] = {};
+  size_t cnt0[PAIR_TABLES] = {};
   std::vector<PairTile> h;
 };
-constexpr int PAIR_KINDS = 6;
+constexpr int pair_table(int kind, int dir) { return kind <= SU2HIP_K_U1_METROPOLIS ? dir : PAIR_SCALARS; }
+constexpr int pair_kind0(int table) { return table == PAIR_SCALARS ? SU2HIP_K_U1_METROPOLIS + 1 : 0; }
+constexpr int PAIR_KIND_ROWS[PAIR_TABLES] = {SU2HIP_K_U1_METROPOLIS + 1, SU2HIP_K_U1_METROPOLIS + 1,
+                                             SU2HIP_K_U1_METROPOLIS + 1,
+                                             SU2HIP_K_SINGLET_METROPOLIS - SU2HIP_K_U1_METROPOLIS};
 
 constexpr int NCHUNK = 3;
 constexpr int CHUNKS[NCHUNK] = {64, 128, 256};
@@ -142,7 +150,8 @@ struct su2hip_batch {
   long long kcount[SU2HIP_NKINDS] = {};
   AltMap alt[2];                  // chunks 64 and 128; 256 is the main table
   PairMap pair;                   // paired link passes
-  bool pair_on = false;           // sweeps take them
+  bool pair_on = false;           // sweeps take them,
+  bool pair_fields = false;       // of U(1) links and scalars too
   // tables whose counters may be nonzero (1 << k), of the launches made and of
   // the captured sweep: 0 the main table, 1 and 2 alt, 3 pair
   unsigned touched = 0, graph_touched = 0;
@@ -316,7 +325,6 @@ static void fill_desc(Slot &s) {
   L.G = p.triplet ? take(6 * Vh) : nullptr;
   L.S = p.singlet ? take(2 * Vh) : nullptr;
   L.H = s.hop_mem;
-  L.Ualt = nullptr;  // build_pairs
   L.B = s.bu_mem;
   L.L0 = p.L[0];
   L.L1 = p.L[1];
@@ -473,16 +481,17 @@ static int fold_table(su2hip_batch *b, long long *d_cnt, int nblk, const std::ve
 
 static int fold_pairs(su2hip_batch *b) {
   PairMap &m = b->pair;
-  if (!m.d_cnt || m.n == 0) return SU2HIP_OK;
-  size_t n = (size_t)PAIR_KINDS * 2 * m.n;
-  std::vector<long long> h(n);
-  HIPTRY(hipMemcpyAsync(h.data(), m.d_cnt, n * sizeof(long long), hipMemcpyDeviceToHost, b->stream));
-  HIPTRY(hipMemsetAsync(m.d_cnt, 0, n * sizeof(long long), b->stream));
+  if (!m.d_cnt || m.ncnt == 0) return SU2HIP_OK;
+  std::vector<long long> h(m.ncnt);
+  HIPTRY(hipMemcpyAsync(h.data(), m.d_cnt, m.ncnt * sizeof(long long), hipMemcpyDeviceToHost, b->stream));
+  HIPTRY(hipMemsetAsync(m.d_cnt, 0, m.ncnt * sizeof(long long), b->stream));
   HIPTRY(hipStreamSynchronize(b->stream));
-  for (int k = 0; k < PAIR_KINDS; k++)
-    for (int i = 0; i < m.n; i++) {
-      long long a = h[(size_t)(k * 2) * m.n + i], t = h[(size_t)(k * 2 + 1) * m.n + i];
-      if (a || t) add_counts(b->slots[m.h[i].lat].cnt, k, a, t);
+  for (int t = 0; t < PAIR_TABLES; t++)
+    for (int k = 0; k < PAIR_KIND_ROWS[t]; k++) {
+      const long long *q = h.data() + m.cnt0[t] + (size_t)k * 2 * m.count[t];
+      for (int i = 0; i < m.count[t]; i++)
+        if (q[i] || q[m.count[t] + i])
+          add_counts(b->slots[m.h[m.first[t] + i].lat].cnt, pair_kind0(t) + k, q[i], q[m.count[t] + i]);
     }
   return SU2HIP_OK;
 }
@@ -547,20 +556,24 @@ static int build_alt(su2hip_batch *b, AltMap &m, int chunk) {
 // 127, 48^3 147 -> 139, but 52^3 157 -> 161; FP64 with U(1) 32^3 218 -> 200,
 // 40^3 240 -> 231, sixteen of 16^3 222 -> 201, but 44^3 245 -> 270.
 constexpr uint64_t PAIR_SITES_FP32 = 120000, PAIR_SITES_FP64 = 65536;
+// and those of the other kinds: sweeps with five link rounds, links paired ->
+// all: FP32 24^3 113.8 -> 110.6 us, 32^3 113.7 -> 113.3, 48^3 139 -> 146; FP64
+// triplet 24^3 166 -> 158
+constexpr uint64_t PAIR_SITES_FIELDS = 36000;
 
 // Tiles of link direction dir in one lattice: whole rows in x and n1 of them
-// in the other transverse direction, or for direction 0 boxes of at most nx by
-// n1 by n2.
+// in the other transverse direction, or for direction 0 and the scalars
+// (PAIR_SCALARS) boxes of at most nx by n1 by n2.
 struct PairShape {
   int n[3], halo[3], count[3];
   int tiles() const { return count[0] * count[1] * count[2]; }
-  int threads() const { return n[0] * (n[1] + 2 * halo[1]) * (n[2] + 2 * halo[2]); }
+  int threads() const { return (n[0] + halo[0]) * (n[1] + 2 * halo[1]) * (n[2] + 2 * halo[2]); }
 };
 
 static PairShape pair_shape(const LatDesc &L, int dir, int nx, int n1, int n2) {
   const int ext[3] = {L.h0, L.L1, L.L2};
   PairShape p{{L.h0, 1, 1}, {0, 0, 0}, {}};
-  if (dir == 0) {
+  if (dir == 0 || dir == PAIR_SCALARS) {
     // the boxes of a row equally wide
     const int k = (L.h0 + nx - 1) / nx;
     p.n[0] = (L.h0 + k - 1) / k;
@@ -570,7 +583,9 @@ static PairShape pair_shape(const LatDesc &L, int dir, int nx, int n1, int n2) {
     p.n[3 - dir] = n1;
   }
   for (int d = 0; d < 3; d++) {
-    if (d && d != dir) {
+    if (d == 0) {
+      p.halo[0] = dir == PAIR_SCALARS && p.n[0] < L.h0;
+    } else if (d != dir) {
       p.halo[d] = p.n[d] + 2 < ext[d];
       if (!p.halo[d]) p.n[d] = ext[d];
     }
@@ -591,9 +606,10 @@ static void pair_tiles(int lat, const LatDesc &L, const PairShape &p, std::vecto
         t.ny = std::min(p.n[1], L.L1 - y);
         t.z0 = z;
         t.nz = std::min(p.n[2], L.L2 - z);
+        t.hx = p.halo[0];
         t.hy = p.halo[1];
         t.hz = p.halo[2];
-        t.dx = make_fastdiv((uint32_t)t.nx);
+        t.dx = make_fastdiv((uint32_t)(t.nx + t.hx));
         t.dy0 = make_fastdiv((uint32_t)(t.ny + 2 * t.hy));
         t.dy1 = make_fastdiv((uint32_t)t.ny);
         v.push_back(t);
@@ -608,9 +624,10 @@ static void pair_tiles(int lat, const LatDesc &L, const PairShape &p, std::vecto
 // 48^3 15.7-16.0 at 6 waves a CU, 16.5-17.2 at 8-10.  False if none fits.
 static bool pair_choose(const su2hip_batch *b, int dir, int sel[3], int &threads) {
   long best = -1;
-  for (int nx = 32; nx >= (dir ? 32 : 4); nx -= 4)
+  const bool box = dir == 0 || dir == PAIR_SCALARS;
+  for (int nx = 32; nx >= (box ? 4 : 32); nx -= 4)
     for (int n1 = 8; n1 >= 2; n1--)
-      for (int n2 = dir ? 1 : n1; n2 >= (dir ? 1 : 2); n2--) {
+      for (int n2 = box ? n1 : 1; n2 >= (box ? 2 : 1); n2--) {
         long tiles = 0;
         int thr = 1, core = 1;
         for (int i = 0; i < b->max_slots; i++) {
@@ -654,10 +671,10 @@ static int build_pairs(su2hip_batch *b) {
   bool ok = b->tmpl.nhiggs < 2;
   for (int i = 0; i < b->max_slots; i++) {
     Slot &s = b->slots[i];
-    s.hd.Ualt = nullptr;
+    s.hd.Ualt = s.hd.Aalt = s.hd.Falt = s.hd.Galt = s.hd.Salt = nullptr;
     if (!s.used) continue;
     sites += 2 * (uint64_t)s.hd.Vh;
-    bytes += align256(link_words(s.p) * wsize(s.p));
+    bytes += s.bytes;
     ok = ok && s.hd.h0 <= PAIR_THREADS / 4;
   }
   ok = ok && sites && sites <= (b->fp64 ? PAIR_SITES_FP64 : PAIR_SITES_FP32);
@@ -673,21 +690,31 @@ static int build_pairs(su2hip_batch *b) {
   if (!ok) {
     pair_drop(b);
     m.n = 0;
+    m.ncnt = 0;
     return SU2HIP_OK;
   }
   char *q = (char *)m.mem;
   for (int i = 0; i < b->max_slots; i++) {
     Slot &s = b->slots[i];
     if (!s.used) continue;
-    s.hd.Ualt = q;
-    q += align256(link_words(s.p) * wsize(s.p));
+    // laid out as the slot's own
+    const ptrdiff_t off = q - (char *)s.mem;
+    auto alt = [&](void *p) { return p ? (void *)((char *)p + off) : nullptr; };
+    s.hd.Ualt = alt(s.hd.U);
+    s.hd.Aalt = alt(s.hd.A);
+    s.hd.Falt = alt(s.hd.F);
+    s.hd.Galt = alt(s.hd.G);
+    s.hd.Salt = alt(s.hd.S);
+    q += s.bytes;
   }
   m.h.clear();
-  for (int dir = 0; dir < 3; dir++) {
+  m.ncnt = 0;
+  for (int dir = 0; dir < PAIR_TABLES; dir++) {
     int sel[3];
     if (!pair_choose(b, dir, sel, m.threads[dir])) {
       pair_drop(b);
       m.n = 0;
+      m.ncnt = 0;
       return SU2HIP_OK;
     }
     m.first[dir] = (int)m.h.size();
@@ -695,23 +722,27 @@ static int build_pairs(su2hip_batch *b) {
       if (b->slots[i].used)
         pair_tiles(i, b->slots[i].hd, pair_shape(b->slots[i].hd, dir, sel[0], sel[1], sel[2]), m.h);
     m.count[dir] = (int)m.h.size() - m.first[dir];
+    m.cnt0[dir] = m.ncnt;
+    m.ncnt += (size_t)PAIR_KIND_ROWS[dir] * 2 * m.count[dir];
   }
   m.n = (int)m.h.size();
-  if (m.n > m.cap) {
+  if ((size_t)m.n > m.cap || m.ncnt > m.cnt_cap) {
     if (m.d) HIPTRY(hipFree(m.d));
     if (m.d_cnt) HIPTRY(hipFree(m.d_cnt));
     m.d = nullptr;
     m.d_cnt = nullptr;
-    m.cap = 0;
+    m.cap = m.cnt_cap = 0;
     if (hipMalloc(&m.d, sizeof(PairTile) * m.n) != hipSuccess ||
-        hipMalloc(&m.d_cnt, sizeof(long long) * PAIR_KINDS * 2 * m.n) != hipSuccess)
+        hipMalloc(&m.d_cnt, sizeof(long long) * m.ncnt) != hipSuccess)
       return fail(SU2HIP_ENOMEM, "tile table allocation failed");
     m.cap = m.n;
+    m.cnt_cap = m.ncnt;
   }
   HIPTRY(hipMemcpyAsync(m.d, m.h.data(), sizeof(PairTile) * m.n, hipMemcpyHostToDevice, b->stream));
-  HIPTRY(hipMemsetAsync(m.d_cnt, 0, sizeof(long long) * PAIR_KINDS * 2 * m.n, b->stream));
+  HIPTRY(hipMemsetAsync(m.d_cnt, 0, sizeof(long long) * m.ncnt, b->stream));
   HIPTRY(hipStreamSynchronize(b->stream));
   b->pair_on = true;
+  b->pair_fields = sites <= PAIR_SITES_FIELDS;
   return SU2HIP_OK;
 }
 
@@ -932,14 +963,14 @@ static bool su2_link_kind(int kind) {
          kind == SU2HIP_K_LINK_OVERRELAX;
 }
 
-// steps i and i + 1 of the schedule are the two parities of one link
-// direction, of a kind that k_pair_link takes
+// steps i and i + 1 of the schedule are the two parities of one pass, of a
+// kind that launch_pair takes
 static bool pairable(const su2hip_batch *b, size_t i) {
   if (!b->pair_on || b->random_order || i + 1 >= b->sched.size()) return false;
   const Step &s = b->sched[i], &n = b->sched[i + 1];
-  return (s.kind == SU2HIP_K_LINK_HEATBATH || s.kind == SU2HIP_K_LINK_OVERRELAX) &&
-         n.kind == s.kind && n.dir == s.dir && s.parity == 0 && n.parity == 1 &&
-         n.pass_off == s.pass_off + 1;
+  if (s.kind >= SU2HIP_K_U1_METROPOLIS && !b->pair_fields) return false;
+  return pair_kind(s.kind, b->model, b->fp64) && !s.muca && !n.muca && n.kind == s.kind && n.dir == s.dir &&
+         s.parity == 0 && n.parity == 1 && n.pass_off == s.pass_off + 1;
 }
 
 static hipError_t enqueue_sweep(su2hip_batch *b) {
@@ -965,16 +996,17 @@ static hipError_t enqueue_sweep(su2hip_batch *b) {
       hop_fresh = true;
     }
     if (e == hipSuccess && pairable(b, i)) {
-      // SU(2) link passes come in rounds of all three directions, so the
-      // passes of other kinds find c.alt 0 or ALT_LINKS
+      // link passes come in rounds of all three directions, so the passes of
+      // other kinds find the bits of a link field all set or all clear
       const PairMap &m = b->pair;
-      const int d = st.dir;
+      const int t = pair_table(st.kind, st.dir);
       e = timed(b, st.kind, 2, [&] {
-        return launch_pair_link(c, m.d + m.first[d], m.count[d], m.threads[d], st.kind, d, st.pass_off,
-                                m.d_cnt + m.first[d], m.n);
+        return launch_pair(c, m.d + m.first[t], m.count[t], m.threads[t], st.kind, st.dir, st.pass_off,
+                           m.d_cnt + m.cnt0[t] + (size_t)(st.kind - pair_kind0(t)) * 2 * m.count[t],
+                           m.count[t]);
       });
       b->touched |= 8;
-      c.alt ^= 1 << d;
+      c.alt ^= pair_bit(st.kind, st.dir);
       i++;
     } else if (e == hipSuccess) {
       e = enqueue_step(b, st, c.alt);

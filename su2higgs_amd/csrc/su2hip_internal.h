@@ -87,7 +87,8 @@ struct LatDesc {
   // term of every link staple, H_mu(x) (k_hop), 4 values per link in the
   // link layout; else null
   void *H;
-  void *Ualt;                   // second link buffer of paired passes, else null
+  // second buffers of paired passes, else null
+  void *Ualt, *Aalt, *Falt, *Galt, *Salt;
   int L0, L1, L2, h0;           // extents, h0 = L0/2
   int Vh, vol;                  // sites per parity, volume
   FastDiv div_h0, div_L1;
@@ -126,21 +127,24 @@ struct BlockMap {
   int s0;
 };
 
-// Buffers of a paired pass (k_pair_link): bit d set while the links of
-// direction d are in the lattice's second buffer
-constexpr int ALT_LINKS = 7;
+// The fields that are in a lattice's second buffers between the paired passes
+// of a sweep: bits of the link directions, the U(1) link directions, the
+// doublet, the triplet and the singlet
+constexpr int ALT_LINKS = 7, ALT_U1_SHIFT = 3, ALT_U1 = 7 << ALT_U1_SHIFT, ALT_F = 64, ALT_G = 128,
+              ALT_S = 256;
 // threads of a paired pass's workgroup, one per site of its tile in a parity
 constexpr int PAIR_THREADS = 256;
 
 // One tile of a paired pass: the sites with x >> 1 in [xh0, xh0 + nx), y in
-// [y0, y0 + ny), z in [z0, z0 + nz).  hy, hz: 1 where the tile does not span
-// that extent (transverse to the link direction), so the first parity is
-// updated in one more row on each side too.
+// [y0, y0 + ny), z in [z0, z0 + nz).  hx, hy, hz: 1 where the second parity's
+// neighbours of the first lie outside the tile in that direction, so that the
+// first parity is updated in one more row on each side too (in x in one more
+// site of each row).
 struct PairTile {
   int lat;
   int xh0, nx, y0, ny, z0, nz;
-  int hy, hz;
-  FastDiv dx, dy0, dy1;  // by nx, by ny + 2 hy and by ny
+  int hx, hy, hz;
+  FastDiv dx, dy0, dy1;  // by nx + hx, by ny + 2 hy and by ny
 };
 
 // ---- launch interface (implemented in su2hip_kernels.hip) ----
@@ -171,7 +175,8 @@ struct LaunchCtx {
   // ([max_slots][npass]); null = the launch's parity and direction
   const uint8_t *order = nullptr;
   int npass = 0;
-  // where the links are (ALT_LINKS bits; single passes need all or none)
+  // where the fields are (ALT_ bits; the directions of a field all or none,
+  // but for the passes that pair them)
   int alt = 0;
 };
 
@@ -180,13 +185,17 @@ struct LaunchCtx {
 // `muca_step` of a multicanonical parity sweep.
 hipError_t launch_pass(const LaunchCtx &c, int kind, int parity, int dir,
                        int pass_off, int muca_step, int reunit);
-// Both parities of one direction of a link kind (the pass at pass_off and the
-// one after it) in one launch over the tiles of a table, from the buffers
-// c.alt names into the other buffer of direction dir.  cnt: counters
-// [6 kinds][2][ncnt] of the tiles, the table's first at entry 0.
-hipError_t launch_pair_link(const LaunchCtx &c, const PairTile *tiles, int ntiles, int threads,
-                            int kind, int dir, int pass_off, long long *cnt, int ncnt);
-// copy every link in the second buffer (c.alt) back to the first
+// whether launch_pair takes a pass kind of a model
+bool pair_kind(int kind, int model, int fp64);
+// the bit of LaunchCtx::alt that a paired pass changes
+int pair_bit(int kind, int dir);
+// Both parities of a pass kind (and link direction; the pass at pass_off and
+// the one after it) in one launch over the tiles of a table, from the buffers
+// c.alt names into the other buffer of the field.  cnt, ncnt: the kind's two
+// counter rows of the tiles, ncnt apart.
+hipError_t launch_pair(const LaunchCtx &c, const PairTile *tiles, int ntiles, int threads, int kind,
+                       int dir, int pass_off, long long *cnt, int ncnt);
+// copy every field in a second buffer (c.alt) back to its first
 hipError_t launch_pair_close(const LaunchCtx &c);
 // the doublet's hopping term of every link staple (one doublet; a no-op
 // otherwise), read by the link passes that follow until the doublet or the

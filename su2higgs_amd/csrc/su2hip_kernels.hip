@@ -249,37 +249,44 @@ constexpr int staple_norm_w() {
   return (M & M_H2) != 0 && (sizeof(T) == 4 || (M & M_U1) != 0) ? 2 : 1;
 }
 
-// staple_doublet (src/staples.c:243-302)
-template <typename T, int M>
-__device__ __forceinline__ void doublet_hops(const LatDesc &L, const T *U, const T *A, const T *F,
-                                             const Site &x, int d, Q<T> &s) {
-  Site xp = shift(L, x, d, +1), xm = shift(L, x, d, -1);
-  Q<T> t = qmul(U_at<M>(L, U, x, d), F_at(L, F, xp));
+// on a lambda: inlined before the compiler orders and contracts floating-point
+// operations, as the text at the place of its call would be
+#define SU2_INLINE __attribute__((always_inline))
+
+// staple_doublet (src/staples.c:243-302); nb(nb.at(d, sign)): Phi at the
+// neighbour
+template <typename T, int M, class NB>
+__device__ __forceinline__ void doublet_hops(const LatDesc &L, const T *U, const T *A,
+                                             const Site &x, int d, Q<T> &s, NB &&nb) {
+  const auto tp = nb.at(d, +1), tm = nb.at(d, -1);
+  Site xm = shift(L, x, d, -1);
+  Q<T> t = qmul(U_at<M>(L, U, x, d), nb(tp));
   if constexpr ((M & M_U1) != 0) t = qmul_u1(t, u1twist<T>(A_at(L, A, x, d)));
   s = qadd(s, qscale(t, (T)-1));
-  Q<T> t2 = qmul(qconj(U_at<M>(L, U, xm, d)), F_at(L, F, xm));
+  Q<T> t2 = qmul(qconj(U_at<M>(L, U, xm, d)), nb(tm));
   if constexpr ((M & M_U1) != 0) t2 = qmul_u1(t2, qconj(u1twist<T>(A_at(L, A, xm, d))));
   s = qadd(s, qscale(t2, (T)-1));
 }
 
-template <typename T, int M>
-__device__ __forceinline__ Q<T> doublet_staple(const LatDesc &L, const T *U, const T *A, const T *F,
-                                               const Site &x) {
+template <typename T, int M, class NB>
+__device__ __forceinline__ Q<T> doublet_staple(const LatDesc &L, const T *U, const T *A,
+                                               const Site &x, NB &&nb) {
   Q<T> s{(T)0, (T)0, (T)0, (T)0};
   if constexpr ((M & M_U1) != 0 && sizeof(T) == 8) {
     // one direction at a time: six inlined FP64 sincos side by side would
     // hold 170 VGPRs (2 waves per SIMD)
 #pragma unroll 1
-    for (int d = 0; d < 3; d++) doublet_hops<T, M>(L, U, A, F, x, d, s);
+    for (int d = 0; d < 3; d++) doublet_hops<T, M>(L, U, A, x, d, s, nb);
     return s;
   }
 #pragma unroll
   for (int d = 0; d < 3; d++) {
-    Site xp = shift(L, x, d, +1), xm = shift(L, x, d, -1);
-    Q<T> t = qmul(U_at<M>(L, U, x, d), F_at(L, F, xp));
+    const auto tp = nb.at(d, +1), tm = nb.at(d, -1);
+    Site xm = shift(L, x, d, -1);
+    Q<T> t = qmul(U_at<M>(L, U, x, d), nb(tp));
     if constexpr ((M & M_U1) != 0) t = qmul_u1(t, u1twist<T>(A_at(L, A, x, d)));
     s = qadd(s, qscale(t, (T)-1));
-    Q<T> t2 = qmul(qconj(U_at<M>(L, U, xm, d)), F_at(L, F, xm));
+    Q<T> t2 = qmul(qconj(U_at<M>(L, U, xm, d)), nb(tm));
     if constexpr ((M & M_U1) != 0) t2 = qmul_u1(t2, qconj(u1twist<T>(A_at(L, A, xm, d))));
     s = qadd(s, qscale(t2, (T)-1));
   }
@@ -287,17 +294,18 @@ __device__ __forceinline__ Q<T> doublet_staple(const LatDesc &L, const T *U, con
 }
 
 // hopping staple of the triplet (src/overrelax.c:143-180)
-template <typename T, int M>
-__device__ __forceinline__ V3<T> triplet_staple(const LatDesc &L, const T *U, const T *G, const Site &x) {
+template <typename T, int M, class NB>
+__device__ __forceinline__ V3<T> triplet_staple(const LatDesc &L, const T *U, const Site &x, NB &&nb) {
   V3<T> s{(T)0, (T)0, (T)0};
 #pragma unroll
   for (int d = 0; d < 3; d++) {
-    Site xp = shift(L, x, d, +1), xm = shift(L, x, d, -1);
-    V3<T> r = rotate(U_at<M>(L, U, x, d), G_at(L, G, xp));
+    const auto tp = nb.at(d, +1), tm = nb.at(d, -1);
+    Site xm = shift(L, x, d, -1);
+    V3<T> r = rotate(U_at<M>(L, U, x, d), nb(tp));
     s.x -= r.x;
     s.y -= r.y;
     s.z -= r.z;
-    r = rotate(qconj(U_at<M>(L, U, xm, d)), G_at(L, G, xm));
+    r = rotate(qconj(U_at<M>(L, U, xm, d)), nb(tm));
     s.x -= r.x;
     s.y -= r.y;
     s.z -= r.z;
@@ -727,11 +735,71 @@ __device__ __forceinline__ int link_move(const LatDesc &L, Q<T> V, const Q<T> &o
   return 0;
 }
 
+// The field that a pass of kind KIND other than an SU(2) link kind updates
+// (of two doublets the first; A of one direction)
+template <typename T, int KIND>
+struct FieldOf {
+  using type = std::conditional_t<
+      KIND == SU2HIP_K_DOUBLET_OVERRELAX || KIND == SU2HIP_K_DOUBLET_METROPOLIS, Q<T>,
+      std::conditional_t<KIND == SU2HIP_K_TRIPLET_OVERRELAX || KIND == SU2HIP_K_TRIPLET_METROPOLIS,
+                         V3<T>, T>>;
+};
+template <typename T, int KIND>
+__device__ __forceinline__ typename FieldOf<T, KIND>::type field_at(const T *p, int Vh, int mu, int par,
+                                                                     int s) {
+  if constexpr (KIND == SU2HIP_K_U1_METROPOLIS)
+    return ldA(p, Vh, mu, par, s);
+  else if constexpr (std::is_same_v<typename FieldOf<T, KIND>::type, Q<T>>)
+    return ldF(p, Vh, par, s);
+  else if constexpr (std::is_same_v<typename FieldOf<T, KIND>::type, V3<T>>)
+    return ldG(p, Vh, par, s);
+  else
+    return ldS(p, Vh, par, s);
+}
+template <typename T, int KIND>
+__device__ __forceinline__ void field_set(T *p, int Vh, int mu, int par, int s,
+                                          const typename FieldOf<T, KIND>::type &v) {
+  if constexpr (KIND == SU2HIP_K_U1_METROPOLIS)
+    *gmem(p + (size_t)(mu * 2 + par) * Vh + s) = v;
+  else if constexpr (std::is_same_v<typename FieldOf<T, KIND>::type, Q<T>>)
+    stF(p, Vh, par, s, v);
+  else if constexpr (std::is_same_v<typename FieldOf<T, KIND>::type, V3<T>>)
+    stG(p, Vh, par, s, v);
+  else
+    *gmem(p + (size_t)par * Vh + s) = v;
+}
+template <typename T, int KIND>
+__device__ __forceinline__ T *field_of(const LatDesc &L) {
+  if constexpr (KIND == SU2HIP_K_U1_METROPOLIS)
+    return (T *)L.A;
+  else if constexpr (std::is_same_v<typename FieldOf<T, KIND>::type, Q<T>>)
+    return (T *)L.F;
+  else if constexpr (std::is_same_v<typename FieldOf<T, KIND>::type, V3<T>>)
+    return (T *)L.G;
+  else
+    return (T *)L.S;
+}
+
+// its value at the neighbours of x in the lattice's buffer p
+template <typename T, int KIND>
+struct Near {
+  const LatDesc &L;
+  const Site &x;
+  const T *p;
+  int mu;
+  __device__ __forceinline__ Site at(int d, int sg) const { return shift(L, x, d, sg); }
+  __device__ __forceinline__ typename FieldOf<T, KIND>::type operator()(const Site &c) const {
+    return field_at<T, KIND>(p, L.Vh, mu, c.par, c.s);
+  }
+};
+
 // MU: the direction of an SU(2) link kind (-1 for the others, which take it
-// or the doublet from mu)
-template <typename T, int M, int KIND, int MU>
-__device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int par, int s, int mu_in,
-                                           Rng &r, int reunit) {
+// or the doublet from mu).  For the other kinds nb(nb.at(d, sign)) is the
+// updated field at the neighbour and put(v) takes the new value where there is one;
+// Ab: the U(1) links by direction, or null where they are all at L.A.
+template <typename T, int M, int KIND, int MU, class NB, class PUT>
+__device__ __forceinline__ int site_update(const LatDesc &L, const T *const *Ab, const Site &x, int par,
+                                           int s, int mu_in, Rng &r, NB &&nb, PUT &&put) {
   const int mu = MU >= 0 ? MU : mu_in;
   T *U = (T *)L.U;
   T *A = (T *)L.A;
@@ -759,7 +827,10 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
   } else if constexpr (KIND == SU2HIP_K_U1_METROPOLIS) {
     // metro_u1link (src/metropolis.c:48-70) with localact_u1link
     // (src/su2u1.c:336-354) evaluated as a difference
-    T al = ldA(A, Vh, mu, par, s);
+    auto Ad = [&](int d, const Site &c) SU2_INLINE {
+      return Ab ? ldA(Ab[d], Vh, 0, c.par, c.s) : A_at(L, (const T *)A, c, d);
+    };
+    const T al = Ad(mu, x);
     T na = al + (T)0.95 * (uni<T>(r) - (T)0.5);
     if constexpr (sizeof(T) == 4) {
       // FP32: keep the angle in [-pi, pi] so it keeps its precision; the
@@ -780,9 +851,10 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
 #pragma unroll
       for (int nu = 0; nu < 3; nu++) {
         if (nu == mu) continue;
-        Site xn = shift(L, x, nu, +1), xm = shift(L, x, nu, -1), xpm = shift(L, xp, nu, -1);
-        T rest_up = A_at(L, A, xp, nu) - A_at(L, A, xn, mu) - A_at(L, A, x, nu);
-        T rest_dn = A_at(L, A, xm, mu) + A_at(L, A, xpm, nu) - A_at(L, A, xm, nu);
+        const auto tn = nb.at(nu, +1), tm = nb.at(nu, -1);
+        Site xm = shift(L, x, nu, -1), xpm = shift(L, xp, nu, -1);
+        T rest_up = Ad(nu, xp) - nb(tn) - Ad(nu, x);
+        T rest_dn = nb(tm) + Ad(nu, xpm) - Ad(nu, xm);
         sum += ::sin(rr * (m + rest_up)) - ::sin(rr * (rest_dn - m));
       }
       dS = (T)2 * (T)L.betau1 * ::sin(rr * h) * sum;
@@ -806,9 +878,10 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
 #pragma unroll
       for (int nu = 0; nu < 3; nu++) {
         if (nu == mu) continue;
-        Site xn = shift(L, x, nu, +1), xm = shift(L, x, nu, -1), xpm = shift(L, xp, nu, -1);
-        T rest_up = A_at(L, A, xp, nu) - A_at(L, A, xn, mu) - A_at(L, A, x, nu);
-        T rest_dn = A_at(L, A, xm, mu) + A_at(L, A, xpm, nu) - A_at(L, A, xm, nu);
+        const auto tn = nb.at(nu, +1), tm = nb.at(nu, -1);
+        Site xm = shift(L, x, nu, -1), xpm = shift(L, xp, nu, -1);
+        T rest_up = Ad(nu, xp) - nb(tn) - Ad(nu, x);
+        T rest_dn = nb(tm) + Ad(nu, xpm) - Ad(nu, xm);
         sum += fsin(rr * (m + rest_up)) - fsin(rr * (rest_dn - m));
       }
       dS = (T)2 * (T)L.betau1 * fsin(rr * h) * sum;
@@ -823,7 +896,7 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
       }
     }
     if (!metro_accept(dS, r)) return 0;
-    *gmem(A + (size_t)(mu * 2 + par) * Vh + s) = na;
+    put(na);
     return 1;
   } else if constexpr ((KIND == SU2HIP_K_DOUBLET_OVERRELAX ||
                         KIND == SU2HIP_K_DOUBLET_METROPOLIS) && (M & M_H2) != 0) {
@@ -832,7 +905,8 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
     const T *Fo = mu ? (const T *)F : (const T *)L.F2;
     Q<T> ft = ldF(Fh, Vh, par, s);
     Q<double> f = qd(ft), H = qd(ldF(Fo, Vh, par, s));
-    Q<double> st = qd(doublet_staple<T, M>(L, U, A, Fh, x));
+    Q<double> st = qd(doublet_staple<T, M>(
+        L, U, A, x, Near<T, KIND>{L, x, Fh, 0}));
     Q<T> nf;
     if constexpr (KIND == SU2HIP_K_DOUBLET_OVERRELAX) {
       // overrelax_higgs2 (src/overrelax.c:295-417) in FP64 for both
@@ -863,7 +937,7 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
   } else if constexpr (KIND == SU2HIP_K_DOUBLET_OVERRELAX ||
                        KIND == SU2HIP_K_DOUBLET_METROPOLIS) {
     Q<T> f = ldF(F, Vh, par, s);
-    Q<T> st = doublet_staple<T, M>(L, U, A, F, x);
+    Q<T> st = doublet_staple<T, M>(L, U, A, x, nb);
     double B0 = 0.5 * L.msq + 1.0 * 3;
     if constexpr ((M & M_TR) != 0) {
       V3<T> g = ldG(G, Vh, par, s);
@@ -877,8 +951,8 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
     Q<T> nf;
     int acc;
     if constexpr (KIND == SU2HIP_K_DOUBLET_OVERRELAX && sizeof(T) == 4) {
-      // overrelax_doublet in FP32
-      T n2 = qdot(st, st);
+      // overrelax_doublet in FP32; the first sum's rounding pinned (sum2)
+      T n2 = qdot_w<packed_links<M, T>() || (M & M_U1) == 0 ? 2 : 1>(st, st);
       T iF = frsqrt(n2);
       T Fn = n2 * iF;
       Q<T> e = qscale(st, iF);
@@ -915,12 +989,12 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
                (T)B0 * (n2 - o2) + (T)C * (n2 * n2 - o2 * o2);
       if (!metro_accept(diff, r)) return 0;
     }
-    stF(F, Vh, par, s, nf);
+    put(nf);
     return 1;
   } else if constexpr (KIND == SU2HIP_K_TRIPLET_OVERRELAX ||
                        KIND == SU2HIP_K_TRIPLET_METROPOLIS) {
     V3<T> g = ldG(G, Vh, par, s);
-    V3<T> st = triplet_staple<T, M>(L, U, G, x);
+    V3<T> st = triplet_staple<T, M>(L, U, x, nb);
     double C = 0.25 * L.b4;
     V3<T> ng;
     if constexpr (KIND == SU2HIP_K_TRIPLET_OVERRELAX && sizeof(T) == 4) {
@@ -967,15 +1041,15 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
                (T)B0 * (n2 - o2) + (T)C * (n2 * n2 - o2 * o2);
       if (!metro_accept(diff, r)) return 0;
     }
-    stG(G, Vh, par, s, ng);
+    put(ng);
     return 1;
   } else if constexpr (KIND == SU2HIP_K_SINGLET_OVERRELAX ||
                        KIND == SU2HIP_K_SINGLET_METROPOLIS) {
     double Sx = ldS(S, Vh, par, s);
-    double nb = 0.0;
+    double ns = 0.0;
 #pragma unroll
     for (int d = 0; d < 3; d++)
-      nb += (double)S_at(L, S, shift(L, x, d, +1)) + (double)S_at(L, S, shift(L, x, d, -1));
+      ns += (double)nb(nb.at(d, +1)) + (double)nb(nb.at(d, -1));
     double ph = 0.0;
     if constexpr ((M & M_NH) != 0) {
       Q<T> f = ldF(F, Vh, par, s);
@@ -984,7 +1058,7 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
     double nS;
     if constexpr (KIND == SU2HIP_K_SINGLET_OVERRELAX) {
       // overrelax_singlet (src/overrelax.c:243-285)
-      double c1 = L.b1_s - nb;
+      double c1 = L.b1_s - ns;
       double c2 = 3 + 0.5 * L.msq_s;
       double c3 = 1.0 / 3.0 * L.b3_s;
       double c4 = 0.25 * L.b4_s;
@@ -1011,10 +1085,10 @@ __device__ __forceinline__ int site_update(const LatDesc &L, const Site &x, int 
         if constexpr ((M & M_NH) != 0) pv += 0.5 * L.a1_s * v * ph + 0.5 * L.a2_s * v * v * ph;
         return pv;
       };
-      double diff = 3.0 * (nS * nS - Sx * Sx) - (nS - Sx) * nb + (pot(nS) - pot(Sx));
+      double diff = 3.0 * (nS * nS - Sx * Sx) - (nS - Sx) * ns + (pot(nS) - pot(Sx));
       if (!metro_accept((T)diff, r)) return 0;
     }
-    *gmem(S + (size_t)par * Vh + s) = (T)nS;
+    put((T)nS);
     return 1;
   }
   return 0;
@@ -1135,6 +1209,24 @@ __device__ __forceinline__ void pin_desc(const LatDesc &L) {
   if constexpr (KIND <= SU2HIP_K_LINK_OVERRELAX) asm volatile("" ::"s"(L.beta));
 }
 
+// the fields where LaunchCtx::alt has them
+template <int M>
+__device__ __forceinline__ void use_alt(LatDesc &L, int alt) {
+  if (alt & ALT_LINKS) L.U = L.Ualt;
+  if constexpr ((M & M_U1) != 0) {
+    if (alt & ALT_U1) L.A = L.Aalt;
+  }
+  if constexpr ((M & M_NH) != 0) {
+    if (alt & ALT_F) L.F = L.Falt;
+  }
+  if constexpr ((M & M_TR) != 0) {
+    if (alt & ALT_G) L.G = L.Galt;
+  }
+  if constexpr ((M & M_SG) != 0) {
+    if (alt & ALT_S) L.S = L.Salt;
+  }
+}
+
 template <typename T, int M, int KIND>
 __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
                                           const MucaDev *__restrict__ mucas,
@@ -1148,7 +1240,7 @@ __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
   const BlockMap bm = block_of(blk, nblk, one, chunk, pass_off & 1, idx);
   LatDesc L = lats[bm.lat];
   pin_desc<M, KIND>(L);
-  if (alt) L.U = L.Ualt;
+  if constexpr ((M & M_H2) == 0) use_alt<M>(L, alt);
   if (!L.active || L.budget == 0) return;
   int par = par_in, mu = mu_in;
   if (order) {
@@ -1186,6 +1278,19 @@ __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
     Site x = site_of(L, par, s);
     Rng r;
     rng_init(r, L.key0, L.key1, L.pass + (uint64_t)pass_off, (uint32_t)(par * L.Vh + s));
+    auto go = [&](auto dir, int m) SU2_INLINE {
+      constexpr int MU = decltype(dir)::value;
+      if constexpr (KIND <= SU2HIP_K_LINK_OVERRELAX) {
+        acc = site_update<T, M, KIND, MU>(L, nullptr, x, par, s, m, r, 0, 0);
+      } else {
+        T *p = field_of<T, KIND>(L);
+        acc = site_update<T, M, KIND, MU>(
+            L, nullptr, x, par, s, m, r,
+            Near<T, KIND>{L, x, p, m},
+            [&](const typename FieldOf<T, KIND>::type &v)
+                SU2_INLINE { field_set<T, KIND>(p, L.Vh, m, par, s, v); });
+      }
+    };
     if constexpr ((KIND <= SU2HIP_K_LINK_OVERRELAX && const_dir<T, M>()) ||
                   (KIND == SU2HIP_K_U1_METROPOLIS && sizeof(T) == 4)) {
       // one inlined copy per link direction: the neighbour offsets and the
@@ -1193,13 +1298,13 @@ __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
       // together instead of one direction at a time (U(1), 96^3: 6.8 ->
       // 6.4 us).  The FP64 U(1) kind loses more to the extra registers.
       if (mu == 0)
-        acc = site_update<T, M, KIND, 0>(L, x, par, s, 0, r, reunit);
+        go(std::integral_constant<int, 0>{}, 0);
       else if (mu == 1)
-        acc = site_update<T, M, KIND, 1>(L, x, par, s, 1, r, reunit);
+        go(std::integral_constant<int, 1>{}, 1);
       else
-        acc = site_update<T, M, KIND, 2>(L, x, par, s, 2, r, reunit);
+        go(std::integral_constant<int, 2>{}, 2);
     } else {
-      acc = site_update<T, M, KIND, -1>(L, x, par, s, mu, r, reunit);
+      go(std::integral_constant<int, -1>{}, mu);
     }
   }
   // counted wavefront by wavefront with atomics that return nothing: no
@@ -1276,7 +1381,18 @@ __device__ __forceinline__ T *link_base(const LatDesc &L, int d, int second) {
   return const_cast<T *>(link_run<M>((const T *)((char *)L.U + off), L.Vh, d, 0));
 }
 
-// the site of a tile at row (ly, lz) counted from its margin's first
+// a workgroup's tile: XCD j gets a contiguous run of them
+__device__ __forceinline__ PairTile tile_of(const PairTile *tiles, int ntiles, int &ti) {
+  const int j = (int)(blockIdx.x % NXCD), q = ntiles / (int)NXCD, rem = ntiles % (int)NXCD;
+  ti = j * q + (j < rem ? j : rem) + (int)(blockIdx.x / NXCD);
+  const PairTile t = tiles[ti];
+  asm volatile("" ::"s"(t.xh0), "s"(t.nx), "s"(t.y0), "s"(t.ny), "s"(t.z0), "s"(t.nz), "s"(t.hx),
+               "s"(t.hy), "s"(t.hz), "s"(t.dx.m), "s"(t.dy0.m), "s"(t.dy1.m));
+  return t;
+}
+
+// the site of a tile at column xl from the tile's first and row (ly, lz) from
+// its margin's first
 __device__ __forceinline__ Site tile_site(const LatDesc &L, const PairTile &t, int xl, int ly, int lz,
                                           int par) {
   Site x;
@@ -1284,7 +1400,8 @@ __device__ __forceinline__ Site tile_site(const LatDesc &L, const PairTile &t, i
   x.y = x.y < 0 ? x.y + L.L1 : (x.y >= L.L1 ? x.y - L.L1 : x.y);
   x.z = t.z0 - t.hz + lz;
   x.z = x.z < 0 ? x.z + L.L2 : (x.z >= L.L2 ? x.z - L.L2 : x.z);
-  const int xh = t.xh0 + xl;
+  int xh = t.xh0 + xl;
+  xh = xh < 0 ? xh + L.h0 : (xh >= L.h0 ? xh - L.h0 : xh);
   x.x = 2 * xh + ((par + x.y + x.z) & 1);
   x.par = par;
   x.s = xh + L.h0 * (x.y + L.L1 * x.z);
@@ -1297,13 +1414,9 @@ __global__ __launch_bounds__(PAIR_THREADS) void k_pair_link(const LatDesc *__res
                                                             int ntiles, int pass_off, int alt,
                                                             long long *__restrict__ cnt, int ncnt) {
   __shared__ LinkRaw<M, T> fresh[PAIR_THREADS];
-  // XCD j gets a contiguous run of tiles
-  const int j = (int)(blockIdx.x % NXCD), q = ntiles / (int)NXCD, rem = ntiles % (int)NXCD;
-  const int ti = j * q + (j < rem ? j : rem) + (int)(blockIdx.x / NXCD);
-  const PairTile t = tiles[ti];
-  asm volatile("" ::"s"(t.xh0), "s"(t.nx), "s"(t.y0), "s"(t.ny), "s"(t.z0), "s"(t.nz), "s"(t.hy),
-               "s"(t.hz), "s"(t.dx.m), "s"(t.dy0.m), "s"(t.dy1.m));
-  const LatDesc L = lats[t.lat];
+  int ti;
+  const PairTile t = tile_of(tiles, ntiles, ti);
+  LatDesc L = lats[t.lat];
   pin_desc<M, KIND>(L);
   asm volatile("" ::"s"(L.Ualt));
   if (!L.active || L.budget == 0) return;
@@ -1311,9 +1424,10 @@ __global__ __launch_bounds__(PAIR_THREADS) void k_pair_link(const LatDesc *__res
 #pragma unroll
   for (int d = 0; d < 3; d++) Ub[d] = link_base<M, T>(L, d, (alt >> d) & 1);
   T *Uo = link_base<M, T>(L, MU, !((alt >> MU) & 1));
+  use_alt<M>(L, alt & ~ALT_LINKS);
   const T *G = (const T *)L.G;
   constexpr int N1 = SiteLinks<T, M, MU>::N1, N2 = SiteLinks<T, M, MU>::N2;
-  const int my = t.ny + 2 * t.hy, mz = t.nz + 2 * t.hz;
+  const int my = t.ny + 2 * t.hy, mz = t.nz + 2 * t.hz;  // t.hx is 0
   const int i = (int)threadIdx.x, row = (int)fdiv((uint32_t)i, t.dx), xl = i - row * t.nx;
   // first parity: the tile and its margin rows (but not the margin's corners)
   const int lz0 = (int)fdiv((uint32_t)row, t.dy0), ly0 = row - lz0 * my;
@@ -1417,13 +1531,132 @@ __global__ __launch_bounds__(PAIR_THREADS) void k_pair_link(const LatDesc *__res
   nacc += __popcll(am);
   ntot += __popcll(tm);
   if ((threadIdx.x & 63) == 0 && ntot) {
-    count_up(&cnt[(size_t)(KIND * 2 + 0) * ncnt + ti], nacc);
-    count_up(&cnt[(size_t)(KIND * 2 + 1) * ncnt + ti], ntot);
+    count_up(&cnt[ti], nacc);
+    count_up(&cnt[ncnt + ti], ntot);
   }
 }
 
-// links in the second buffer back to the first, at the end of a sweep that
-// paired an odd number of rounds
+// the updated field at the tile's fresh entry at(d, sign)
+template <class V, class AT>
+struct NearTile {
+  const AT &at;
+  const V *v;
+  __device__ __forceinline__ V operator()(int i) const { return v[i]; }
+};
+
+// The same for the other kinds: U(1) links of one direction, whose staple
+// reaches its own direction like an SU(2) link's, and the scalars, whose
+// margin is one site all round.  In x that is one site of the first parity
+// per row of the tile (to the right of it or the left, by the row's parity),
+// and its margin rows need none.  Bound by its chain like k_pair_link, with the
+// update's arithmetic twice over as the longest part: loading the second
+// parity's links ahead gained nothing (FP32 32^3 doublet 5.6 -> 5.9 us).  Two
+// passes -> one, overrelaxation of the doublet in a replayed graph: FP32 8^3 5.7
+// -> 5.2 us, 24^3 6.1 -> 5.4, FP64 8^3 7.3 -> 6.6; traced, a box of 18 x 14 x 26
+// in FP64: U(1) 10.0 -> 7.3, singlet 9.3 -> 5.0.
+template <typename T, int M, int KIND, int MU>
+__global__ __launch_bounds__(PAIR_THREADS) void k_pair_field(const LatDesc *__restrict__ lats,
+                                                             const PairTile *__restrict__ tiles,
+                                                             int ntiles, int pass_off, int alt,
+                                                             long long *__restrict__ cnt, int ncnt) {
+  using V = typename FieldOf<T, KIND>::type;
+  __shared__ V fresh[PAIR_THREADS];
+  int ti;
+  const PairTile t = tile_of(tiles, ntiles, ti);
+  LatDesc L = lats[t.lat];
+  pin_desc<M, KIND>(L);
+  if (!L.active || L.budget == 0) return;
+  // the field where it is and where it goes; the others where they are
+  const T *Ab[3] = {nullptr, nullptr, nullptr}, *in;
+  T *out;
+  constexpr int m = MU >= 0 ? MU : 0;
+  if constexpr (KIND == SU2HIP_K_U1_METROPOLIS) {
+    const ptrdiff_t d2 = (char *)L.Aalt - (char *)L.A;
+    auto at = [&](int d, int second) {
+      return (T *)((char *)L.A + (second ? d2 : 0)) + (size_t)d * 2 * L.Vh;
+    };
+#pragma unroll
+    for (int d = 0; d < 3; d++) Ab[d] = at(d, (alt >> (ALT_U1_SHIFT + d)) & 1);
+    in = Ab[m];
+    out = at(m, !((alt >> (ALT_U1_SHIFT + m)) & 1));
+    use_alt<M>(L, alt & ~ALT_U1);
+  } else {
+    LatDesc O = L;
+    use_alt<M>(L, alt);
+    use_alt<M>(O, ~alt & (ALT_F | ALT_G | ALT_S));
+    in = field_of<T, KIND>(L);
+    out = field_of<T, KIND>(O);
+  }
+  const int w = t.nx + t.hx, my = t.ny + 2 * t.hy, mz = t.nz + 2 * t.hz;
+  const int i = (int)threadIdx.x, row = (int)fdiv((uint32_t)i, t.dx), xl = i - row * w;
+  // whether the first parity's entries of tile row (ly, lz) start a site to
+  // the left of the tile
+  auto left = [&](int ly, int lz) SU2_INLINE {
+    const bool core = !(t.hy && (ly == 0 || ly == my - 1)) && !(t.hz && (lz == 0 || lz == mz - 1));
+    return t.hx && core && ((t.y0 - t.hy + ly + t.z0 - t.hz + lz) & 1) ? 1 : 0;
+  };
+  Site x{};
+  Rng r;
+  V cur{}, nu{};
+  int acc = 0;
+  const int lz0 = (int)fdiv((uint32_t)row, t.dy0), ly0 = row - lz0 * my;
+  const bool ey = t.hy && (ly0 == 0 || ly0 == my - 1), ez = t.hz && (lz0 == 0 || lz0 == mz - 1);
+  const bool on0 = row < my * mz && !(ey && ez) && (xl < t.nx || !(ey || ez));
+  const int xr = xl - left(ly0, lz0);  // from the tile's first column
+  const bool core0 = on0 && !(ey || ez) && xr >= 0 && xr < t.nx;
+  auto update = [&](int pass, auto &&nb) SU2_INLINE {
+    rng_init(r, L.key0, L.key1, L.pass + (uint64_t)pass, (uint32_t)(x.par * L.Vh + x.s));
+    nu = cur;
+    acc = site_update<T, M, KIND, MU>(L, KIND == SU2HIP_K_U1_METROPOLIS ? Ab : nullptr, x, x.par, x.s,
+                                      m, r, nb, [&](const V &v) SU2_INLINE { nu = v; });
+  };
+  if (on0) {
+    x = tile_site(L, t, xr, ly0, lz0, 0);
+    cur = field_at<T, KIND>(in, L.Vh, 0, 0, x.s);
+    update(pass_off, Near<T, KIND>{L, x, in, 0});
+    fresh[i] = nu;
+    if (core0) field_set<T, KIND>(out, L.Vh, 0, 0, x.s, nu);
+  }
+  uint64_t am = __ballot(core0 && acc), tm = __ballot(core0);
+  int nacc = __popcll(am), ntot = __popcll(tm);
+  const int lz1 = (int)fdiv((uint32_t)row, t.dy1) + t.hz, ly1 = row - (lz1 - t.hz) * t.ny + t.hy;
+  const bool on1 = row < t.ny * t.nz && xl < t.nx;
+  acc = 0;
+  if (on1) {
+    x = tile_site(L, t, xl, ly1, lz1, 1);
+    cur = field_at<T, KIND>(in, L.Vh, 0, 1, x.s);
+  }
+  __syncthreads();
+  if (on1) {
+    auto at = [&](int d, int sg) SU2_INLINE {
+      int ly = ly1, lz = lz1, xx = xl;
+      if (d == 0) {
+        xx += ((x.x & 1) ? (sg > 0) : -(sg < 0));
+        if (!t.hx) xx = xx < 0 ? t.nx - 1 : (xx >= t.nx ? 0 : xx);
+      } else if (d == 1) {
+        ly += sg;
+        if (!t.hy) ly = ly < 0 ? my - 1 : (ly >= my ? 0 : ly);
+      } else {
+        lz += sg;
+        if (!t.hz) lz = lz < 0 ? mz - 1 : (lz >= mz ? 0 : lz);
+      }
+      return xx + left(ly, lz) + w * (ly + my * lz);
+    };
+    update(pass_off + 1, NearTile<V, decltype(at)>{at, fresh});
+    field_set<T, KIND>(out, L.Vh, 0, 1, x.s, nu);
+  }
+  am = __ballot(on1 && acc);
+  tm = __ballot(on1);
+  nacc += __popcll(am);
+  ntot += __popcll(tm);
+  if ((threadIdx.x & 63) == 0 && ntot) {
+    count_up(&cnt[ti], nacc);
+    count_up(&cnt[ncnt + ti], ntot);
+  }
+}
+
+// fields in second buffers back to the first ones, at the end of a sweep that
+// paired an odd number of rounds of them
 template <typename T, int M>
 __global__ __launch_bounds__(BLK) void k_pair_close(const LatDesc *__restrict__ lats,
                                                     const BlockMap *__restrict__ blk, int nblk, int one,
@@ -1432,15 +1665,30 @@ __global__ __launch_bounds__(BLK) void k_pair_close(const LatDesc *__restrict__ 
   const BlockMap bm = block_of(blk, nblk, one, BLK, 0, idx);
   const LatDesc L = lats[bm.lat];
   if (!L.active || L.budget == 0) return;
-  const int s = bm.s0 + (int)threadIdx.x;
-  if (s >= L.Vh) return;
+  const int s = bm.s0 + (int)threadIdx.x, Vh = L.Vh;
+  if (s >= Vh) return;
 #pragma unroll
-  for (int d = 0; d < 3; d++)
-    if ((alt >> d) & 1)
+  for (int par = 0; par < 2; par++) {
 #pragma unroll
-      for (int par = 0; par < 2; par++)
-        stL<M>((T *)link_run<M>((const T *)L.U, L.Vh, d, par), L.Vh, s,
-               ldL<M>(link_run<M>((const T *)L.Ualt, L.Vh, d, par), L.Vh, s));
+    for (int d = 0; d < 3; d++) {
+      if ((alt >> d) & 1)
+        stL<M>((T *)link_run<M>((const T *)L.U, Vh, d, par), Vh, s,
+               ldL<M>(link_run<M>((const T *)L.Ualt, Vh, d, par), Vh, s));
+      if constexpr ((M & M_U1) != 0) {
+        if ((alt >> (ALT_U1_SHIFT + d)) & 1)
+          *gmem((T *)L.A + (size_t)(d * 2 + par) * Vh + s) = ldA((const T *)L.Aalt, Vh, d, par, s);
+      }
+    }
+    if constexpr ((M & M_NH) != 0) {
+      if (alt & ALT_F) stF((T *)L.F, Vh, par, s, ldF((const T *)L.Falt, Vh, par, s));
+    }
+    if constexpr ((M & M_TR) != 0) {
+      if (alt & ALT_G) stG((T *)L.G, Vh, par, s, ldG((const T *)L.Galt, Vh, par, s));
+    }
+    if constexpr ((M & M_SG) != 0) {
+      if (alt & ALT_S) *gmem((T *)L.S + (size_t)par * Vh + s) = ldS((const T *)L.Salt, Vh, par, s);
+    }
+  }
 }
 
 // The hopping-term cache of one doublet: for every link, the doublet part
@@ -1451,11 +1699,13 @@ __global__ __launch_bounds__(BLK) void k_pair_close(const LatDesc *__restrict__ 
 // sincos once per round instead of once per pass.
 template <typename T, int M>
 __global__ __launch_bounds__(BLK) void k_hop(const LatDesc *__restrict__ lats,
-                                             const BlockMap *__restrict__ blk, int nblk, int one) {
+                                             const BlockMap *__restrict__ blk, int nblk, int one,
+                                             int alt) {
   int idx;
   const BlockMap bm = block_of(blk, nblk, one, BLK, 1, idx);
-  const LatDesc L = lats[bm.lat];
+  LatDesc L = lats[bm.lat];
   pin_desc<M, SU2HIP_K_AUX>(L);
+  use_alt<M>(L, alt);
   if (!L.active || L.budget == 0 || !L.H) return;
   const int s = bm.s0 + (int)threadIdx.x;
   if (s >= L.Vh) return;
@@ -2711,7 +2961,7 @@ __device__ __forceinline__ V3<T> link_force(const LatDesc &L, const T *U, const 
 template <typename T, int M>
 __device__ __forceinline__ V3<T> triplet_force(const LatDesc &L, const T *U, const T *F, const T *G,
                                               const Site &x, double msq_t) {
-  V3<T> res = triplet_staple<T, M>(L, U, G, x);
+  V3<T> res = triplet_staple<T, M>(L, U, x, Near<T, SU2HIP_K_TRIPLET_OVERRELAX>{L, x, G, 0});
   V3<T> g = G_at(L, G, x);
   T tsq = (T)0.5 * (g.x * g.x + g.y * g.y + g.z * g.z);
   T k = (T)(2.0 * 3 + msq_t) + (T)2 * (T)L.b4 * tsq;
@@ -2887,7 +3137,8 @@ static hipError_t pass_one(const LaunchCtx &c, int parity, int dir, int pass_off
     // multicanonical steps use the 256-site table: their order-parameter
     // partials are indexed by 256-site chunk
     if (step >= 0 && c.block != BLK) return hipErrorInvalidValue;
-    if (c.alt != 0 && c.alt != ALT_LINKS) return hipErrorInvalidValue;
+    const int la = c.alt & ALT_LINKS, ua = c.alt & ALT_U1;
+    if ((la && la != ALT_LINKS) || (ua && ua != ALT_U1)) return hipErrorInvalidValue;
     if constexpr (KIND == SU2HIP_K_LINK_OVERRELAX) {
       if (c.waves == 5) {
         if (c.ev_start || c.ev_stop) {
@@ -2940,21 +3191,58 @@ hipError_t launch_pass(const LaunchCtx &c, int kind, int parity, int dir, int pa
   });
 }
 
+// FP64 doublet passes with U(1) links stay single: their chain of three
+// directions' sines twice over is as long as the launch saved (a box of 18 x 14
+// x 26: 11.5 us a pair, 5.9 a pass, traced)
+template <typename T, int M>
+constexpr bool pair_doublet() {
+  return (M & M_NH) != 0 && ((M & M_U1) == 0 || sizeof(T) == 4);
+}
+
+bool pair_kind(int kind, int model, int fp64) {
+  switch (kind) {
+    case SU2HIP_K_DOUBLET_OVERRELAX:
+    case SU2HIP_K_DOUBLET_METROPOLIS: return !(fp64 && (model & M_U1));
+    case SU2HIP_K_LINK_HEATBATH:
+    case SU2HIP_K_LINK_OVERRELAX:
+    case SU2HIP_K_U1_METROPOLIS:
+    case SU2HIP_K_TRIPLET_OVERRELAX:
+    case SU2HIP_K_TRIPLET_METROPOLIS:
+    case SU2HIP_K_SINGLET_OVERRELAX:
+    case SU2HIP_K_SINGLET_METROPOLIS: return true;
+  }
+  return false;
+}
+
+int pair_bit(int kind, int dir) {
+  if (kind <= SU2HIP_K_LINK_OVERRELAX) return 1 << dir;
+  if (kind == SU2HIP_K_U1_METROPOLIS) return 1 << (ALT_U1_SHIFT + dir);
+  if (kind == SU2HIP_K_DOUBLET_OVERRELAX || kind == SU2HIP_K_DOUBLET_METROPOLIS) return ALT_F;
+  if (kind == SU2HIP_K_TRIPLET_OVERRELAX || kind == SU2HIP_K_TRIPLET_METROPOLIS) return ALT_G;
+  return ALT_S;
+}
+
 template <typename T, int M, int KIND>
 static hipError_t pair_one(const LaunchCtx &c, const PairTile *tiles, int ntiles, int threads, int dir,
                            int pass_off, long long *cnt, int ncnt) {
   auto go = [&](auto mu) {
-    hipLaunchKernelGGL((k_pair_link<T, M, KIND, decltype(mu)::value>), dim3(ntiles), dim3(threads), 0,
-                       c.stream, c.desc, tiles, ntiles, pass_off, c.alt, cnt, ncnt);
+    constexpr int MU = decltype(mu)::value;
+    if constexpr (KIND <= SU2HIP_K_LINK_OVERRELAX)
+      hipLaunchKernelGGL((k_pair_link<T, M, KIND, MU>), dim3(ntiles), dim3(threads), 0, c.stream,
+                         c.desc, tiles, ntiles, pass_off, c.alt, cnt, ncnt);
+    else
+      hipLaunchKernelGGL((k_pair_field<T, M, KIND, MU>), dim3(ntiles), dim3(threads), 0, c.stream,
+                         c.desc, tiles, ntiles, pass_off, c.alt, cnt, ncnt);
     return hipGetLastError();
   };
-  if (dir == 0) return go(std::integral_constant<int, 0>{});
-  if (dir == 1) return go(std::integral_constant<int, 1>{});
-  return go(std::integral_constant<int, 2>{});
+  if constexpr (KIND > SU2HIP_K_U1_METROPOLIS) return go(std::integral_constant<int, -1>{});
+  else if (dir == 0) return go(std::integral_constant<int, 0>{});
+  else if (dir == 1) return go(std::integral_constant<int, 1>{});
+  else return go(std::integral_constant<int, 2>{});
 }
 
-hipError_t launch_pair_link(const LaunchCtx &c, const PairTile *tiles, int ntiles, int threads,
-                            int kind, int dir, int pass_off, long long *cnt, int ncnt) {
+hipError_t launch_pair(const LaunchCtx &c, const PairTile *tiles, int ntiles, int threads, int kind,
+                       int dir, int pass_off, long long *cnt, int ncnt) {
   if (ntiles == 0) return hipSuccess;
   if (threads < 1 || threads > PAIR_THREADS || threads % 64 || dir < 0 || dir > 2)
     return hipErrorInvalidValue;
@@ -2962,12 +3250,29 @@ hipError_t launch_pair_link(const LaunchCtx &c, const PairTile *tiles, int ntile
     using T = decltype(t);
     return with_model_of<T>(c.model, [&](auto m) -> hipError_t {
       constexpr int M = decltype(m)::value;
+      auto go = [&](auto k) {
+        return pair_one<T, M, decltype(k)::value>(c, tiles, ntiles, threads, dir, pass_off, cnt, ncnt);
+      };
+#define SU2_PAIR(K) \
+  if (kind == K) return go(std::integral_constant<int, K>{})
       if constexpr ((M & M_H2) == 0) {
-        if (kind == SU2HIP_K_LINK_HEATBATH)
-          return pair_one<T, M, SU2HIP_K_LINK_HEATBATH>(c, tiles, ntiles, threads, dir, pass_off, cnt, ncnt);
-        if (kind == SU2HIP_K_LINK_OVERRELAX)
-          return pair_one<T, M, SU2HIP_K_LINK_OVERRELAX>(c, tiles, ntiles, threads, dir, pass_off, cnt, ncnt);
+        SU2_PAIR(SU2HIP_K_LINK_HEATBATH);
+        SU2_PAIR(SU2HIP_K_LINK_OVERRELAX);
+        if constexpr ((M & M_U1) != 0) SU2_PAIR(SU2HIP_K_U1_METROPOLIS);
+        if constexpr (pair_doublet<T, M>()) {
+          SU2_PAIR(SU2HIP_K_DOUBLET_OVERRELAX);
+          SU2_PAIR(SU2HIP_K_DOUBLET_METROPOLIS);
+        }
+        if constexpr ((M & M_TR) != 0) {
+          SU2_PAIR(SU2HIP_K_TRIPLET_OVERRELAX);
+          SU2_PAIR(SU2HIP_K_TRIPLET_METROPOLIS);
+        }
+        if constexpr ((M & M_SG) != 0) {
+          SU2_PAIR(SU2HIP_K_SINGLET_OVERRELAX);
+          SU2_PAIR(SU2HIP_K_SINGLET_METROPOLIS);
+        }
       }
+#undef SU2_PAIR
       return hipErrorInvalidValue;
     });
   });
@@ -2994,7 +3299,7 @@ hipError_t launch_hop(const LaunchCtx &c) {
       constexpr int M = decltype(m)::value;
       if constexpr (hop_cached<M>()) {
         hipLaunchKernelGGL((k_hop<T, M>), dim3(c.nblk), dim3(BLK), 0, c.stream, c.desc, c.blk,
-                           c.nblk, c.one);
+                           c.nblk, c.one, c.alt);
         return hipGetLastError();
       }
       return hipSuccess;
