@@ -224,8 +224,10 @@ hipError_t launch_cold(const LaunchCtx &c, int slot, double phi0, double sigma0,
 hipError_t launch_hot(const LaunchCtx &c, int slot);
 hipError_t launch_to_device_layout(const LaunchCtx &c, int slot, int field,
                                    const double *host_layout_dev);
-hipError_t launch_to_host_layout(const LaunchCtx &c, int slot, int field,
+hipError_t launch_to_host_layout(const LaunchCtx &c, int slot, int Vh, int field,
                                  double *host_layout_dev);
+// bytes (a multiple of 16) between 16-byte aligned places that the GPU sees
+hipError_t launch_copy(const void *src, void *dst, size_t bytes, hipStream_t s);
 hipError_t launch_copy_probe(const double *src, double *dst, size_t n,
                              hipStream_t s);
 // gradient flow on one lattice (slot) whose descriptor in c.desc points at

@@ -10,6 +10,7 @@
 // is a dense contraction, so MFMA is not used and the kernels are bound by
 // HBM traffic and FP math.
 #include <hip/hip_ext.h>
+#include <algorithm>
 #include <type_traits>
 
 #include "su2hip_device.h"
@@ -2908,7 +2909,9 @@ __global__ void k_to_device(LatDesc L, int field, const double *__restrict__ h) 
 }
 
 template <typename T, int M>
-__global__ void k_to_host(LatDesc L, int field, double *__restrict__ h) {
+__global__ void k_to_host(const LatDesc *__restrict__ lats, int slot, int field,
+                          double *__restrict__ h) {
+  const LatDesc &L = lats[slot];
   int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= L.Vh) return;
   const void *src = field_ptr(L, field);
@@ -3530,19 +3533,23 @@ hipError_t launch_to_device_layout(const LaunchCtx &c, int slot, int field, cons
   });
 }
 
-hipError_t launch_to_host_layout(const LaunchCtx &c, int slot, int field, double *h) {
-  hipError_t e;
-  LatDesc L = host_desc_of(c, slot, e);
-  if (e != hipSuccess) return e;
-  int nb = (L.Vh + BLK - 1) / BLK;
+hipError_t launch_to_host_layout(const LaunchCtx &c, int slot, int Vh, int field, double *h) {
+  const int nb = (Vh + BLK - 1) / BLK;
   return with_prec(c.fp64, [&](auto t) {
     using T = decltype(t);
     return with_model_of<T>(c.model, [&](auto m) -> hipError_t {
       constexpr int M = decltype(m)::value;
-      hipLaunchKernelGGL((k_to_host<T, M>), dim3(nb), dim3(BLK), 0, c.stream, L, field, h);
+      hipLaunchKernelGGL((k_to_host<T, M>), dim3(nb), dim3(BLK), 0, c.stream, c.desc, slot, field, h);
       return hipGetLastError();
     });
   });
+}
+
+hipError_t launch_copy(const void *src, void *dst, size_t bytes, hipStream_t s) {
+  const size_t n2 = bytes / sizeof(double2);
+  const int nb = (int)std::min<size_t>(256 * 4, (n2 + 255) / 256);
+  hipLaunchKernelGGL(k_copy, dim3(nb), dim3(256), 0, s, (const double2 *)src, (double2 *)dst, n2);
+  return hipGetLastError();
 }
 
 hipError_t launch_copy_probe(const double *src, double *dst, size_t n, hipStream_t s) {
