@@ -428,7 +428,8 @@ int su2hip_flow_force(su2hip_batch_t *b, int slot, double *force);
 /* ---- timing ----------------------------------------------------------------
  * With timing on, every launch is bracketed by HIP events on the handle's
  * stream; su2hip_kernel_times() returns the summed milliseconds and the
- * launch count per SU2HIP_K_* kind since the last reset. */
+ * launch count per SU2HIP_K_* kind since the last reset (a launch that makes
+ * both parities' passes of a small lattice counts as those two). */
 int su2hip_set_timing(su2hip_batch_t *b, int enable);
 int su2hip_kernel_times(su2hip_batch_t *b, double *ms, int64_t *launches);
 int su2hip_reset_timing(su2hip_batch_t *b);
