@@ -744,7 +744,6 @@ static int build_pairs(su2hip_batch *b) {
   }
   HIPTRY(hipMemcpyAsync(m.d, m.h.data(), sizeof(PairTile) * m.n, hipMemcpyHostToDevice, b->stream));
   HIPTRY(hipMemsetAsync(m.d_cnt, 0, sizeof(long long) * m.ncnt, b->stream));
-  HIPTRY(hipStreamSynchronize(b->stream));
   b->pair_on = true;
   b->pair_fields = sites <= PAIR_SITES_FIELDS;
   return SU2HIP_OK;
@@ -1076,9 +1075,10 @@ static int ensure_stage(su2hip_batch *b, size_t doubles) {
 // engine each time, and is staged by the runtime at 17.7 GB/s.  Here a kernel
 // writes the pieces into pinned slots of the handle while threads move the
 // pieces before them on; what fits one slot goes at once for all fields.
-// Pageable -> this: 8^3 130 -> 25 us, 24^3 130 -> 105, 40^3 (7.7 MB) 490 -> 280,
-// 96^3 (134 MB) 7.6 -> 4.9 ms, 144^3 25.6 -> 17.0.  8 threads or pieces of 4 MB
-// measure the same, copies by the DMA engine instead 100 us more for the small.
+// Pageable -> this: 8^3 130 -> 25 us, 24^3 130 -> 108, 40^3 (7.7 MB) 490 -> 275,
+// 96^3 (134 MB, 47 GB/s) 7.6 -> 2.85 ms, 144^3 25.6 -> 9.4.  Six threads measure
+// the same, pieces of 1 MB 3.1 ms; copies by the DMA engine take 100 us more for
+// the small.
 constexpr size_t DOWN_PIECE = 2u << 20;
 constexpr int DOWN_SLOTS = 8, DOWN_THREADS = 4;
 
@@ -1142,26 +1142,30 @@ static hipError_t download(su2hip_batch *b, const std::vector<DownPiece> &v, Sta
       moved[t].store(i + 1, std::memory_order_release);
     }
   };
-  for (int i = 0; i < n + slots && e == hipSuccess; i++) {
-    if (i >= slots) {
-      // the oldest piece in flight, then its slot's reader
-      const int k = i - slots;
-      if (k >= n) break;
-      e = hipEventSynchronize(ev[k % slots]);
-      if (e != hipSuccess) break;
-      ready.store(k + 1, std::memory_order_release);
-      finish(k);
-      if (i < n)
-        while (moved[k % nthreads].load(std::memory_order_acquire) <= k) std::this_thread::yield();
+  // the next piece in flight has arrived: handed on
+  int arrived = 0;
+  auto arrive = [&] {
+    e = hipEventSynchronize(ev[arrived % slots]);
+    if (e != hipSuccess) return;
+    ready.store(arrived + 1, std::memory_order_release);
+    finish(arrived++);
+  };
+  for (int i = 0; i < n && e == hipSuccess; i++) {
+    // the slot's last piece moved on; meanwhile the ones behind it arrive
+    while (i >= slots && e == hipSuccess &&
+           moved[(i - slots) % nthreads].load(std::memory_order_acquire) <= i - slots) {
+      if (arrived < i)
+        arrive();
+      else
+        std::this_thread::yield();
     }
-    if (i < n) {
-      e = stage(i);
-      if (e == hipSuccess)
-        e = launch_copy((char *)b->d_stage + v[i].off, b->pin + (size_t)(i % slots) * DOWN_PIECE, v[i].n,
-                        b->stream);
-      if (e == hipSuccess) e = hipEventRecord(ev[i % slots], b->stream);
-    }
+    if (e == hipSuccess) e = stage(i);
+    if (e == hipSuccess)
+      e = launch_copy((char *)b->d_stage + v[i].off, b->pin + (size_t)(i % slots) * DOWN_PIECE, v[i].n,
+                      b->stream);
+    if (e == hipSuccess) e = hipEventRecord(ev[i % slots], b->stream);
   }
+  while (arrived < n && e == hipSuccess) arrive();
   if (e != hipSuccess) stop.store(true);
   for (int t = 0; t < started; t++) th[t].join();
   if (e != hipSuccess) (void)hipStreamSynchronize(b->stream);
