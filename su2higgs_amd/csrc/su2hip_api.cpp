@@ -40,6 +40,19 @@ static int fail(int code, const char *fmt, ...) {
       return fail(SU2HIP_EDEVICE, "%s failed: %s", #x, hipGetErrorString(e_));       \
   } while (0)
 
+// Device memory.  A refusal leaves no error behind: the handle may go on
+// without the memory or the caller after SU2HIP_ENOMEM, and every launch
+// reports what hipGetLastError() finds, an earlier call's failure too.
+template <typename T>
+static hipError_t dev_alloc(T **p, size_t bytes) {
+  hipError_t e = hipMalloc((void **)p, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    *p = nullptr;
+  }
+  return e;
+}
+
 namespace {
 
 // A gradient flow in flight: device descriptors, private measurement
@@ -540,8 +553,8 @@ static int build_alt(su2hip_batch *b, AltMap &m, int chunk) {
     m.d_blk = nullptr;
     m.d_cnt = nullptr;
     int cap = std::max(n, 256);
-    if (hipMalloc(&m.d_blk, sizeof(BlockMap) * cap) != hipSuccess ||
-        hipMalloc(&m.d_cnt, sizeof(long long) * NCOUNT * 2 * cap) != hipSuccess)
+    if (dev_alloc(&m.d_blk, sizeof(BlockMap) * cap) != hipSuccess ||
+        dev_alloc(&m.d_cnt, sizeof(long long) * NCOUNT * 2 * cap) != hipSuccess)
       return fail(SU2HIP_ENOMEM, "block table allocation failed");
     m.cap = cap;
   }
@@ -684,7 +697,7 @@ static int build_pairs(su2hip_batch *b) {
   ok = ok && sites && sites <= (b->fp64 ? PAIR_SITES_FP64 : PAIR_SITES_FP32);
   if (ok && bytes > m.bytes) {
     pair_drop(b);
-    if ((b->hbm_budget && b->used + bytes > b->hbm_budget) || hipMalloc(&m.mem, bytes) != hipSuccess) {
+    if ((b->hbm_budget && b->used + bytes > b->hbm_budget) || dev_alloc(&m.mem, bytes) != hipSuccess) {
       m.mem = nullptr;
       ok = false;
     } else {
@@ -736,8 +749,8 @@ static int build_pairs(su2hip_batch *b) {
     m.d = nullptr;
     m.d_cnt = nullptr;
     m.cap = m.cnt_cap = 0;
-    if (hipMalloc(&m.d, sizeof(PairTile) * m.n) != hipSuccess ||
-        hipMalloc(&m.d_cnt, sizeof(long long) * m.ncnt) != hipSuccess)
+    if (dev_alloc(&m.d, sizeof(PairTile) * m.n) != hipSuccess ||
+        dev_alloc(&m.d_cnt, sizeof(long long) * m.ncnt) != hipSuccess)
       return fail(SU2HIP_ENOMEM, "tile table allocation failed");
     m.cap = m.n;
     m.cnt_cap = m.ncnt;
@@ -775,8 +788,8 @@ static int rebuild_map(su2hip_batch *b) {
     b->d_blk = nullptr;
     b->d_cnt = nullptr;
     int cap = std::max(n, 64);
-    if (hipMalloc(&b->d_blk, sizeof(BlockMap) * cap) != hipSuccess ||
-        hipMalloc(&b->d_cnt, sizeof(long long) * NCOUNT * 2 * cap) != hipSuccess)
+    if (dev_alloc(&b->d_blk, sizeof(BlockMap) * cap) != hipSuccess ||
+        dev_alloc(&b->d_cnt, sizeof(long long) * NCOUNT * 2 * cap) != hipSuccess)
       return fail(SU2HIP_ENOMEM, "block table allocation failed");
     b->nblk_cap = cap;
   }
@@ -784,7 +797,7 @@ static int rebuild_map(su2hip_batch *b) {
   if (need > b->partial_cap) {
     if (b->d_partial) HIPTRY(hipFree(b->d_partial));
     b->d_partial = nullptr;
-    if (hipMalloc(&b->d_partial, need * sizeof(double)) != hipSuccess)
+    if (dev_alloc(&b->d_partial, need * sizeof(double)) != hipSuccess)
       return fail(SU2HIP_ENOMEM, "partial-sum buffer allocation failed");
     b->partial_cap = need;
   }
@@ -1033,14 +1046,14 @@ static int ensure_order(su2hip_batch *b) {
     if (b->d_order) HIPTRY(hipFree(b->d_order));
     b->d_order = nullptr;
     b->order_cap = 0;
-    if (hipMalloc(&b->d_order, no) != hipSuccess) return fail(SU2HIP_ENOMEM, "order table");
+    if (dev_alloc(&b->d_order, no) != hipSuccess) return fail(SU2HIP_ENOMEM, "order table");
     b->order_cap = no;
   }
   if (ni > b->info_cap) {
     if (b->d_info) HIPTRY(hipFree(b->d_info));
     b->d_info = nullptr;
     b->info_cap = 0;
-    if (hipMalloc(&b->d_info, ni * sizeof(uint16_t)) != hipSuccess)
+    if (dev_alloc(&b->d_info, ni * sizeof(uint16_t)) != hipSuccess)
       return fail(SU2HIP_ENOMEM, "order table");
     b->info_cap = ni;
   }
@@ -1064,7 +1077,7 @@ static int ensure_stage(su2hip_batch *b, size_t doubles) {
   if (doubles <= b->stage_cap) return SU2HIP_OK;
   if (b->d_stage) HIPTRY(hipFree(b->d_stage));
   b->d_stage = nullptr;
-  if (hipMalloc(&b->d_stage, doubles * sizeof(double)) != hipSuccess)
+  if (dev_alloc(&b->d_stage, doubles * sizeof(double)) != hipSuccess)
     return fail(SU2HIP_ENOMEM, "staging buffer of %zu doubles", doubles);
   b->stage_cap = doubles;
   return SU2HIP_OK;
@@ -1215,7 +1228,7 @@ static int hop_alloc(su2hip_batch *b, int i) {
   if (over_budget(b, bytes))
     return fail(SU2HIP_ENOMEM, "HBM budget: %llu + %zu bytes of hopping-term cache exceeds %llu",
                 (unsigned long long)b->used, bytes, (unsigned long long)b->hbm_budget);
-  if (hipMalloc(&s.hop_mem, bytes) != hipSuccess) {
+  if (dev_alloc(&s.hop_mem, bytes) != hipSuccess) {
     s.hop_mem = nullptr;
     return fail(SU2HIP_ENOMEM, "device allocation of %zu bytes failed", bytes);
   }
@@ -1262,7 +1275,7 @@ static int alloc_slot(su2hip_batch *b, int i, const su2hip_params &p_in) {
   Slot &s = b->slots[i];
   s = Slot();
   s.p = p;
-  if (hipMalloc(&s.mem, bytes) != hipSuccess) {
+  if (dev_alloc(&s.mem, bytes) != hipSuccess) {
     s.mem = nullptr;
     return fail(SU2HIP_ENOMEM, "device allocation of %zu bytes failed", bytes);
   }
@@ -1442,9 +1455,9 @@ int su2hip_create(int n, const su2hip_params *params, int max_slots, uint64_t hb
   b->slots.resize(max_slots);
   int rc = SU2HIP_OK;
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&b->d_desc, sizeof(LatDesc) * max_slots) != hipSuccess ||
-      hipMalloc(&b->d_muca, sizeof(MucaDev) * max_slots) != hipSuccess ||
-      hipMalloc(&b->d_sums, sizeof(double) * SU2HIP_NSUMS * max_slots) != hipSuccess) {
+      dev_alloc(&b->d_desc, sizeof(LatDesc) * max_slots) != hipSuccess ||
+      dev_alloc(&b->d_muca, sizeof(MucaDev) * max_slots) != hipSuccess ||
+      dev_alloc(&b->d_sums, sizeof(double) * SU2HIP_NSUMS * max_slots) != hipSuccess) {
     su2hip_destroy(b);
     return fail(SU2HIP_ENOMEM, "handle allocation failed");
   }
@@ -2077,11 +2090,11 @@ int su2hip_muca_set(su2hip_batch_t *b, int slot, const su2hip_muca *m, const dou
     if (!s.bu_mem) {
       if (over_budget(b, bub))
         return fail(SU2HIP_ENOMEM, "HBM budget exceeded by the multicanonical backup");
-      if (hipMalloc(&newbu, bub) != hipSuccess) return fail(SU2HIP_ENOMEM, "backup allocation");
+      if (dev_alloc(&newbu, bub) != hipSuccess) return fail(SU2HIP_ENOMEM, "backup allocation");
     }
     int n = m->bins + 2;
     bytes = sizeof(double) * n * 6 + sizeof(int) * n + sizeof(long long) * n * 2 + 1024;
-    if (hipMalloc(&newmem, bytes) != hipSuccess) {
+    if (dev_alloc(&newmem, bytes) != hipSuccess) {
       if (newbu) (void)hipFree(newbu);
       return fail(SU2HIP_ENOMEM, "weight arrays");
     }
@@ -2300,8 +2313,8 @@ int su2hip_blocked_correlators(su2hip_batch_t *b, int slot, int levels, double *
   size_t words = align256(lw * w) + align256(6 * Vh1 * w);
   char *mem = nullptr;
   LatDesc *ddesc = nullptr;
-  if (hipMalloc(&mem, 2 * words) != hipSuccess) return fail(SU2HIP_ENOMEM, "blocked fields");
-  if (hipMalloc(&ddesc, sizeof(LatDesc)) != hipSuccess) {
+  if (dev_alloc(&mem, 2 * words) != hipSuccess) return fail(SU2HIP_ENOMEM, "blocked fields");
+  if (dev_alloc(&ddesc, sizeof(LatDesc)) != hipSuccess) {
     (void)hipFree(mem);
     return fail(SU2HIP_ENOMEM, "blocked descriptor");
   }
@@ -2464,7 +2477,7 @@ int su2hip_flow_force(su2hip_batch_t *b, int slot, double *force) {
   std::vector<BlockMap> bm(nb);
   for (int k = 0; k < nb; k++) bm[k] = BlockMap{slot, k * BLK};
   BlockMap *dblk = nullptr;
-  if (hipMalloc(&dblk, sizeof(BlockMap) * nb) != hipSuccess) return fail(SU2HIP_ENOMEM, "block table");
+  if (dev_alloc(&dblk, sizeof(BlockMap) * nb) != hipSuccess) return fail(SU2HIP_ENOMEM, "block table");
   hipError_t e = hipMemcpy(dblk, bm.data(), sizeof(BlockMap) * nb, hipMemcpyHostToDevice);
   LaunchCtx c;
   single_ctx(b, slot, b->d_desc, dblk, nb, c);
@@ -2490,7 +2503,7 @@ static int flow_enqueue(su2hip_batch *b, int slot, int scheme, double dt, double
     size_t fb = align256(flow_words(p) * w) + 4096;
     if (over_budget(b, fb))
       return fail(SU2HIP_ENOMEM, "HBM budget exceeded by the flow buffers");
-    if (hipMalloc(&s.flow_mem, fb) != hipSuccess) return fail(SU2HIP_ENOMEM, "flow buffers");
+    if (dev_alloc(&s.flow_mem, fb) != hipSuccess) return fail(SU2HIP_ENOMEM, "flow buffers");
     s.flow_bytes = fb;
     b->used += fb;
   }
@@ -2552,11 +2565,11 @@ static int flow_enqueue(su2hip_batch *b, int slot, int scheme, double dt, double
   // XCD j gets a contiguous run of chunks, as in the sweep's table
   std::vector<BlockMap> bm = deal_to_xcds(seq);
   size_t nrows = j.t.size();
-  if (hipMalloc(&j.ddesc, sizeof(LatDesc) * hd.size()) != hipSuccess ||
-      hipMalloc(&j.dblk, sizeof(BlockMap) * nb) != hipSuccess ||
-      hipMalloc(&j.d_partial, sizeof(double) * SU2HIP_NSUMS * (size_t)nb) != hipSuccess ||
-      hipMalloc(&j.d_sums, sizeof(double) * SU2HIP_NSUMS * (size_t)b->max_slots) != hipSuccess ||
-      hipMalloc(&j.d_rows, sizeof(double) * SU2HIP_NSUMS * nrows) != hipSuccess ||
+  if (dev_alloc(&j.ddesc, sizeof(LatDesc) * hd.size()) != hipSuccess ||
+      dev_alloc(&j.dblk, sizeof(BlockMap) * nb) != hipSuccess ||
+      dev_alloc(&j.d_partial, sizeof(double) * SU2HIP_NSUMS * (size_t)nb) != hipSuccess ||
+      dev_alloc(&j.d_sums, sizeof(double) * SU2HIP_NSUMS * (size_t)b->max_slots) != hipSuccess ||
+      dev_alloc(&j.d_rows, sizeof(double) * SU2HIP_NSUMS * nrows) != hipSuccess ||
       hipEventCreateWithFlags(&j.done, hipEventDisableTiming) != hipSuccess) {
     flow_release(j);
     return fail(SU2HIP_ENOMEM, "flow descriptors and measurement buffers");
@@ -2900,7 +2913,7 @@ int su2hip_autotune(su2hip_batch_t *b, int repeats, double *table) {
     if (!sl.used) continue;
     hd[i] = sl.hd;
     cnt[i] = sl.cnt;
-    if (hipMalloc(&save[i], sl.bytes) != hipSuccess) {
+    if (dev_alloc(&save[i], sl.bytes) != hipSuccess) {
       save[i] = nullptr;
       release();
       return fail(SU2HIP_ENOMEM, "autotune snapshot of %zu bytes", sl.bytes);
@@ -2973,8 +2986,8 @@ int su2hip_copy_probe(uint64_t bytes, int repeats, double *ms) {
   hipStream_t s = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   // every resource is released on every path: the first failure is kept in e
-  hipError_t e = hipMalloc(&a, n * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&c, n * sizeof(double));
+  hipError_t e = dev_alloc(&a, n * sizeof(double));
+  if (e == hipSuccess) e = dev_alloc(&c, n * sizeof(double));
   if (e != hipSuccess) {
     if (a) (void)hipFree(a);
     return fail(SU2HIP_ENOMEM, "probe buffers of %zu bytes", n * sizeof(double));

@@ -1,0 +1,195 @@
+// The host side of the handle (su2higgs_amd/csrc/su2hip_api.cpp) on the CPU:
+// device memory is host memory, kernels are the records of their launches,
+// and the runtime's calls can be made to fail.  Built and run by
+// test_host_alloc.py; argv[1] names a scenario, a failed check ends with 1.
+#include <hip/hip_runtime.h>
+#undef __align__
+#define __align__(n)
+#define HIP_SYMBOL(x) ((const void *)&(x))
+
+#include <stdlib.h>
+#include <string.h>
+#include <time.h>
+#include <unistd.h>
+
+#include <algorithm>
+#include <atomic>
+#include <functional>
+#include <set>
+#include <vector>
+
+namespace fake {
+hipError_t last = hipSuccess;  // as hipGetLastError: a later success does not clear it
+std::function<bool(size_t)> refuse = [](size_t) { return false; };
+std::function<hipError_t()> launch_fails = [] { return hipSuccess; };
+int wait_ms = 0;  // of an event
+std::atomic<int> waits{0};
+int singles = 0, pairs = 0, closes = 0;
+std::set<void *> live;
+
+hipError_t ret(hipError_t e) {
+  if (e != hipSuccess) last = e;
+  return e;
+}
+hipError_t alloc(void **p, size_t n) {
+  if (refuse(n)) return ret(hipErrorOutOfMemory);
+  *p = aligned_alloc(256, (n + 255) / 256 * 256);
+  live.insert(*p);
+  return hipSuccess;
+}
+hipError_t release(void *p) {
+  if (!p) return hipSuccess;
+  if (!live.erase(p)) abort();
+  free(p);
+  return hipSuccess;
+}
+hipError_t launch() {
+  ret(launch_fails());
+  return hipGetLastError();
+}
+}  // namespace fake
+
+extern "C" {
+hipError_t hipGetLastError(void) {
+  hipError_t e = fake::last;
+  fake::last = hipSuccess;
+  return e;
+}
+const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
+hipError_t hipMalloc(void **p, size_t n) { return fake::alloc(p, n); }
+hipError_t hipFree(void *p) { return fake::release(p); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return fake::alloc(p, n); }
+hipError_t hipHostFree(void *p) { return fake::release(p); }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) { memset(d, v, n); return hipSuccess; }
+hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
+hipError_t hipGetSymbolAddress(void **p, const void *s) { *p = (void *)s; return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = (hipStream_t)1; return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { *g = (hipGraph_t)1; return hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t *x, hipGraph_t, hipGraphNode_t *, char *, size_t) { *x = (hipGraphExec_t)1; return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) { *e = (hipEvent_t)1; return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { *e = (hipEvent_t)1; return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 1; return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) {
+  // the work before the first piece takes its time
+  if (fake::waits++ == 0 && fake::wait_ms) usleep(1000 * fake::wait_ms);
+  return hipSuccess;
+}
+int roctxRangePushA(const char *) { return 0; }
+int roctxRangePop(void) { return 0; }
+}
+
+#include "../su2higgs_amd/csrc/su2hip_api.cpp"
+
+namespace su2 {
+hipError_t launch_pass(const LaunchCtx &, int, int, int, int, int, int) { fake::singles++; return fake::launch(); }
+hipError_t launch_pair(const LaunchCtx &, const PairTile *, int, int, int, int, int, long long *, int) { fake::pairs++; return fake::launch(); }
+hipError_t launch_pair_close(const LaunchCtx &c) { if (c.alt) fake::closes++; return fake::launch(); }
+bool pair_kind(int kind, int, int) { return kind != SU2HIP_K_LINK_METROPOLIS; }
+int pair_bit(int kind, int dir) {
+  return kind <= SU2HIP_K_LINK_OVERRELAX ? 1 << dir
+         : kind == SU2HIP_K_U1_METROPOLIS ? 1 << (ALT_U1_SHIFT + dir)
+         : kind <= SU2HIP_K_DOUBLET_METROPOLIS ? ALT_F
+         : kind <= SU2HIP_K_TRIPLET_METROPOLIS ? ALT_G : ALT_S;
+}
+hipError_t launch_hop(const LaunchCtx &) { return fake::launch(); }
+hipError_t launch_end_sweep(const LaunchCtx &, int) { return fake::launch(); }
+hipError_t launch_cold(const LaunchCtx &, int, double, double, double) { return fake::launch(); }
+hipError_t launch_measure(const LaunchCtx &) { return fake::launch(); }
+hipError_t launch_orderparam_init(const LaunchCtx &, int) { return fake::launch(); }
+hipError_t launch_flow_stage(const LaunchCtx &, int, const void *, void *, const void *, void *, void *, void *, double, double, int) { return fake::launch(); }
+hipError_t launch_to_host_layout(const LaunchCtx &, int, int, int, double *) { return fake::launch(); }
+hipError_t launch_copy(const void *s, void *d, size_t n, hipStream_t) { memcpy(d, s, n); return fake::launch(); }
+}  // namespace su2
+
+static void must(bool ok, const char *what, int line) {
+  if (ok) return;
+  fprintf(stderr, "line %d: %s (%s)\n", line, what, g_err.c_str());
+  exit(1);
+}
+#define MUST(x) must(x, #x, __LINE__)
+
+static su2hip_params params(int L0, int L1, int L2, int nhiggs = 1, int u1 = 0) {
+  su2hip_params p{};
+  p.L[0] = L0;
+  p.L[1] = L1;
+  p.L[2] = L2;
+  p.precision = SU2HIP_FP32;
+  p.nhiggs = nhiggs;
+  p.u1 = u1;
+  p.betasu2 = 9.0;
+  p.betau1 = 9.0;
+  p.r_u1 = 1.0;
+  p.algorithm_su2link = SU2HIP_HEATBATH;
+  p.algorithm_u1link = SU2HIP_METROPOLIS;
+  p.algorithm_su2doublet = p.algorithm_su2triplet = p.algorithm_singlet = SU2HIP_OVERRELAX;
+  p.update_links = p.update_su2doublet = p.update_su2triplet = p.update_singlet = 1;
+  p.link_overrelax = 4;
+  p.scalar_sweeps = 2;
+  p.link_format = SU2HIP_LINKS_FULL;
+  return p;
+}
+
+static su2hip_batch_t *made(const std::vector<su2hip_params> &v, int max_slots = 0, uint64_t budget = 0) {
+  su2hip_batch_t *b = nullptr;
+  const int rc = su2hip_create((int)v.size(), v.data(), std::max(max_slots, (int)v.size()), budget, &b);
+  MUST(rc == SU2HIP_OK);
+  return b;
+}
+
+// a sweep's launches: whether the links were paired
+static bool sweep_pairs(su2hip_batch_t *b) {
+  fake::singles = fake::pairs = 0;
+  MUST(su2hip_update(b, 1) == SU2HIP_OK);
+  MUST(fake::singles + fake::pairs > 0);
+  return fake::pairs > 0;
+}
+
+// The optional second buffers are refused: sweeps of single passes, no error
+// left behind for the next launch.
+static void refused_buffers() {
+  const std::vector<su2hip_params> v{params(8, 8, 8)};
+  int refused = 0;
+  size_t slot = slot_bytes(v[0]);
+  int seen = 0;
+  fake::refuse = [&](size_t n) { return n == slot && ++seen == 2 && ++refused; };
+  su2hip_batch_t *b = made(v);
+  MUST(refused == 1);
+  MUST(!sweep_pairs(b));
+  MUST(hipGetLastError() == hipSuccess);
+  MUST(su2hip_destroy(b) == SU2HIP_OK);
+}
+
+// A call that is refused for want of memory leaves no error behind either.
+static void refused_call() {
+  su2hip_batch_t *b = made({params(8, 8, 8)});
+  fake::refuse = [](size_t) { return true; };
+  double rows[1 + SU2HIP_NSUMS];
+  int n = 0;
+  MUST(su2hip_flow(b, 0, SU2HIP_FLOW_RK3, 0.05, 0.5, 1, rows, 1, &n) == SU2HIP_ENOMEM);
+  MUST(su2hip_autotune(b, 1, nullptr) == SU2HIP_ENOMEM);
+  fake::refuse = [](size_t) { return false; };
+  MUST(sweep_pairs(b));
+  MUST(su2hip_destroy(b) == SU2HIP_OK);
+}
+
+int main(int argc, char **argv) {
+  const std::string s = argc > 1 ? argv[1] : "";
+  if (s == "refused_buffers") refused_buffers();
+  else if (s == "refused_call") refused_call();
+  else return 2;
+  MUST(fake::live.empty());
+  return 0;
+}
