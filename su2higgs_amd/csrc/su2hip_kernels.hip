@@ -2153,6 +2153,18 @@ __device__ double alpha_proj(const LatDesc &L, const T *U, const T *G, const Sit
   return ::atan2(u1.im[0] + u1.im[3], u1.re[0] + u1.re[3]) * ::sqrt(L.beta);
 }
 
+// Whether a measured site's plaquette links are all in flight at once.  Two
+// kinds of model have a term whose links the compiler then loads again and
+// whose registers cost more than the waits saved (kernel, us at 96^3, one by
+// one -> together): the triplet without a doublet FP64 30.1 -> 36.5, FP32 17.9
+// -> 19.1, and FP64 with two doublets 42.3 -> 55.0, with U(1) 90.5 -> 93.3.  The
+// others gain: FP64 pure gauge 25.8 -> 19.6, SU(2)xU(1)+Higgs 48.6 -> 41.7,
+// with both doublet and triplet 47.7 -> 45.2, FP32 two doublets 30.6 -> 29.8.
+template <typename T, int M>
+constexpr bool links_together() {
+  if ((M & M_TR) != 0) return (M & M_NH) != 0;
+  return (M & M_H2) == 0 || sizeof(T) == 4;
+}
 // the loads that follow start only once v is computed
 __device__ __forceinline__ void fence_loads(double &v) { asm volatile("" : "+v"(v) : : "memory"); }
 
@@ -2161,49 +2173,60 @@ __device__ void measure_site(const LatDesc &L, int par, int s, double *acc) {
   const T *U = (const T *)L.U, *A = (const T *)L.A, *F = (const T *)L.F, *G = (const T *)L.G,
           *S = (const T *)L.S;
   Site x = site_of(L, par, s);
-  // Every link and angle of the site's plaquettes in flight at once; the
-  // doublets after the plaquettes have freed their links' registers.  Left to
-  // itself the compiler waits for each term's loads (the cosines branch) and
+  // The links and angles of the site's plaquettes (links_together); the
+  // doublets come after the plaquettes have freed their links' registers.  Left
+  // to itself the compiler waits for each term's loads (the cosines branch) and
   // still holds 212 registers in FP64 SU(2)xU(1)+Higgs, two wavefronts per
-  // SIMD; now 160, three.  With the sums' reduction cut to the model's own,
-  // a whole measure call at 96^3 went from 83 to 68 us in FP64 (the kernel
+  // SIMD; together 154, three.  With the sums' reduction cut to the model's
+  // own, a whole measure call at 96^3 went from 83 to 68 us in FP64 (the kernel
   // 48 -> 41, its fields 19 us at the fabric's rate and its FP64 arithmetic
   // 20 us) and from 73 to 55 us in FP32.
+  constexpr bool together = links_together<T, M>();
   LinkRaw<M, T> u0[3], un[3][3];
   T a0[3], an[3][3];
+  if constexpr (together) {
 #pragma unroll
-  for (int d = 0; d < 3; d++) {
-    u0[d] = ldL<M>(link_run<M>(U, L.Vh, d, par), L.Vh, s);
-    if constexpr ((M & M_U1) != 0) a0[d] = A_at(L, A, x, d);
+    for (int d = 0; d < 3; d++) {
+      u0[d] = ldL<M>(link_run<M>(U, L.Vh, d, par), L.Vh, s);
+      if constexpr ((M & M_U1) != 0) a0[d] = A_at(L, A, x, d);
+    }
+#pragma unroll
+    for (int n = 0; n < 3; n++) {
+      const Site xn = shift(L, x, n, +1);
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+        if (d != n) {
+          un[d][n] = ldL<M>(link_run<M>(U, L.Vh, d, xn.par), L.Vh, xn.s);
+          if constexpr ((M & M_U1) != 0) an[d][n] = A_at(L, A, xn, d);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
-#pragma unroll
-  for (int n = 0; n < 3; n++) {
-    const Site xn = shift(L, x, n, +1);
-#pragma unroll
-    for (int d = 0; d < 3; d++)
-      if (d != n) {
-        un[d][n] = ldL<M>(link_run<M>(U, L.Vh, d, xn.par), L.Vh, xn.s);
-        if constexpr ((M & M_U1) != 0) an[d][n] = A_at(L, A, xn, d);
-      }
-  }
-  __builtin_amdgcn_sched_barrier(0);
+  // link d of x, of its neighbour in direction n; their angles
+  auto u_x = [&](int d) SU2_INLINE { return together ? u0[d].get() : U_at<M>(L, U, x, d); };
+  auto u_n = [&](int d, int n) SU2_INLINE {
+    return together ? un[d][n].get() : U_at<M>(L, U, shift(L, x, n, +1), d);
+  };
+  auto a_x = [&](int d) SU2_INLINE { return together ? a0[d] : A_at(L, A, x, d); };
+  auto a_n = [&](int d, int n) SU2_INLINE {
+    return together ? an[d][n] : A_at(L, A, shift(L, x, n, +1), d);
+  };
   // local_su2wilson (src/su2u1.c:143-157)
   double wl = 0.0;
 #pragma unroll
   for (int d1 = 0; d1 < 3; d1++)
 #pragma unroll
     for (int d2 = 0; d2 < d1; d2++) {
-      Q<double> t = qmul(qmul(qmul(qd(u0[d2].get()), qd(un[d1][d2].get())), qconj(qd(un[d2][d1].get()))),
-                         qconj(qd(u0[d1].get())));
+      Q<double> t = qmul(qmul(qmul(qd(u_x(d2)), qd(u_n(d1, d2))), qconj(qd(u_n(d2, d1)))), qconj(qd(u_x(d1))));
       wl += (1.0 - 0.5 * (2.0 * t.a));
     }
-  fence_loads(wl);
+  if constexpr (together) fence_loads(wl);
   Q<T> f0{}, fn[3];
   if constexpr ((M & M_NH) != 0) {
     f0 = ldF(F, L.Vh, par, s);
 #pragma unroll
     for (int d = 0; d < 3; d++) fn[d] = F_at(L, F, shift(L, x, d, +1));
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (together) __builtin_amdgcn_sched_barrier(0);
   }
   wl *= L.beta;
   double action = wl;
@@ -2215,7 +2238,7 @@ __device__ void measure_site(const LatDesc &L, int par, int s, double *acc) {
     for (int d1 = 0; d1 < 3; d1++)
 #pragma unroll
       for (int d2 = 0; d2 < d1; d2++) {
-        double pl = (double)a0[d2] + (double)an[d1][d2] - (double)an[d2][d1] - (double)a0[d1];
+        double pl = (double)a_x(d2) + (double)a_n(d1, d2) - (double)a_n(d2, d1) - (double)a_x(d1);
         u += (1.0 - ::cos(L.r_u1 * pl));
       }
     u *= L.betau1;
@@ -2230,11 +2253,11 @@ __device__ void measure_site(const LatDesc &L, int par, int s, double *acc) {
     double cov = 0.0;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-      Q<double> t = qmul(qmul(qconj(f), qd(u0[d].get())), qd(fn[d]));
+      Q<double> t = qmul(qmul(qconj(f), qd(u_x(d))), qd(fn[d]));
       double hop;
       if constexpr ((M & M_U1) != 0) {
         double sn, cs;
-        ::sincos((double)a0[d], &sn, &cs);
+        ::sincos((double)a_x(d), &sn, &cs);
         hop = -(t.a * cs + t.d * sn);
       } else {
         hop = -t.a;
