@@ -680,9 +680,16 @@ static void pair_drop(su2hip_batch *b) {
 }
 
 // Paired link passes for the lattices of the handle, where they gain
-// (k_pair_link) and their buffers fit the HBM budget; else single passes.
+// (k_pair_link), their buffers fit the HBM budget and the memory is to be had;
+// else single passes.
 static int build_pairs(su2hip_batch *b) {
   PairMap &m = b->pair;
+  auto single = [&] {
+    pair_drop(b);
+    m.n = 0;
+    m.ncnt = 0;
+    return SU2HIP_OK;
+  };
   uint64_t sites = 0;
   size_t bytes = 0;
   bool ok = b->tmpl.nhiggs < 2;
@@ -704,12 +711,7 @@ static int build_pairs(su2hip_batch *b) {
       m.bytes = bytes;
     }
   }
-  if (!ok) {
-    pair_drop(b);
-    m.n = 0;
-    m.ncnt = 0;
-    return SU2HIP_OK;
-  }
+  if (!ok) return single();
   char *q = (char *)m.mem;
   for (int i = 0; i < b->max_slots; i++) {
     Slot &s = b->slots[i];
@@ -728,12 +730,7 @@ static int build_pairs(su2hip_batch *b) {
   m.ncnt = 0;
   for (int dir = 0; dir < PAIR_TABLES; dir++) {
     int sel[3];
-    if (!pair_choose(b, dir, sel, m.threads[dir])) {
-      pair_drop(b);
-      m.n = 0;
-      m.ncnt = 0;
-      return SU2HIP_OK;
-    }
+    if (!pair_choose(b, dir, sel, m.threads[dir])) return single();
     m.first[dir] = (int)m.h.size();
     for (int i = 0; i < b->max_slots; i++)
       if (b->slots[i].used)
@@ -751,7 +748,7 @@ static int build_pairs(su2hip_batch *b) {
     m.cap = m.cnt_cap = 0;
     if (dev_alloc(&m.d, sizeof(PairTile) * m.n) != hipSuccess ||
         dev_alloc(&m.d_cnt, sizeof(long long) * m.ncnt) != hipSuccess)
-      return fail(SU2HIP_ENOMEM, "tile table allocation failed");
+      return single();
     m.cap = m.n;
     m.cnt_cap = m.ncnt;
   }

@@ -185,10 +185,33 @@ static void refused_call() {
   MUST(su2hip_destroy(b) == SU2HIP_OK);
 }
 
+// The tables of paired passes, allocated after the second buffers, are refused:
+// single passes, and paired ones when the tables are next built.
+static void refused_tables() {
+  const size_t slot = slot_bytes(params(8, 8, 8));
+  for (int k = 0; k < 2; k++) {
+    int buffers = 0, tables = 0;
+    fake::refuse = [&](size_t n) {
+      if (n == slot) return ++buffers > 2;
+      return buffers == 2 && tables++ == k;
+    };
+    su2hip_batch_t *b = made({params(8, 8, 8)}, 2);
+    MUST(tables > k);
+    fake::refuse = [](size_t) { return false; };
+    MUST(!sweep_pairs(b));
+    int i = -1;
+    const su2hip_params p = params(4, 4, 4);
+    MUST(su2hip_add(b, &p, &i) == SU2HIP_OK);
+    MUST(sweep_pairs(b));
+    MUST(su2hip_destroy(b) == SU2HIP_OK);
+  }
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "refused_buffers") refused_buffers();
   else if (s == "refused_call") refused_call();
+  else if (s == "refused_tables") refused_tables();
   else return 2;
   MUST(fake::live.empty());
   return 0;

@@ -23,6 +23,7 @@ def harness(tmp_path_factory):
 @pytest.mark.parametrize("scenario", [
     "refused_buffers",
     "refused_call",
+    "refused_tables",
 ])
 def test_host_side(harness, scenario):
     r = subprocess.run([harness, scenario], capture_output=True, text=True, timeout=120)
