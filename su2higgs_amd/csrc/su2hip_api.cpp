@@ -552,6 +552,7 @@ static int build_alt(su2hip_batch *b, AltMap &m, int chunk) {
     if (m.d_cnt) HIPTRY(hipFree(m.d_cnt));
     m.d_blk = nullptr;
     m.d_cnt = nullptr;
+    m.cap = 0;
     int cap = std::max(n, 256);
     if (dev_alloc(&m.d_blk, sizeof(BlockMap) * cap) != hipSuccess ||
         dev_alloc(&m.d_cnt, sizeof(long long) * NCOUNT * 2 * cap) != hipSuccess)
@@ -784,6 +785,7 @@ static int rebuild_map(su2hip_batch *b) {
     if (b->d_cnt) HIPTRY(hipFree(b->d_cnt));
     b->d_blk = nullptr;
     b->d_cnt = nullptr;
+    b->nblk_cap = 0;
     int cap = std::max(n, 64);
     if (dev_alloc(&b->d_blk, sizeof(BlockMap) * cap) != hipSuccess ||
         dev_alloc(&b->d_cnt, sizeof(long long) * NCOUNT * 2 * cap) != hipSuccess)
@@ -794,6 +796,7 @@ static int rebuild_map(su2hip_batch *b) {
   if (need > b->partial_cap) {
     if (b->d_partial) HIPTRY(hipFree(b->d_partial));
     b->d_partial = nullptr;
+    b->partial_cap = 0;
     if (dev_alloc(&b->d_partial, need * sizeof(double)) != hipSuccess)
       return fail(SU2HIP_ENOMEM, "partial-sum buffer allocation failed");
     b->partial_cap = need;
@@ -1074,6 +1077,7 @@ static int ensure_stage(su2hip_batch *b, size_t doubles) {
   if (doubles <= b->stage_cap) return SU2HIP_OK;
   if (b->d_stage) HIPTRY(hipFree(b->d_stage));
   b->d_stage = nullptr;
+  b->stage_cap = 0;
   if (dev_alloc(&b->d_stage, doubles * sizeof(double)) != hipSuccess)
     return fail(SU2HIP_ENOMEM, "staging buffer of %zu doubles", doubles);
   b->stage_cap = doubles;

@@ -207,11 +207,41 @@ static void refused_tables() {
   }
 }
 
+// A buffer that could not grow is not taken for one of its old size.
+static void refused_growth() {
+  int i = -1;
+  const su2hip_params p = params(64, 64, 64);
+  // each of the block tables, in su2hip_add
+  for (int k = 0; k < 7; k++) {
+    su2hip_batch_t *b = made({params(8, 8, 8)}, 2);
+    int left = k;
+    fake::refuse = [&](size_t n) { return n < slot_bytes(p) / 2 && left-- == 0; };
+    MUST(su2hip_add(b, &p, &i) == SU2HIP_ENOMEM);
+    fake::refuse = [](size_t) { return false; };
+    MUST(su2hip_remove(b, 1) == SU2HIP_OK);
+    MUST(b->d_blk && b->d_cnt && b->d_partial);
+    for (const auto &m : b->alt) MUST(m.d_blk && m.d_cnt);
+    MUST(su2hip_update(b, 1) == SU2HIP_OK);
+    MUST(su2hip_destroy(b) == SU2HIP_OK);
+  }
+  // the staging buffer
+  su2hip_batch_t *b = made({params(8, 8, 8), p});
+  std::vector<double> small(12 * 512), big((size_t)12 << 18);
+  MUST(su2hip_get_fields(b, 0, small.data(), nullptr, nullptr, nullptr, nullptr) == SU2HIP_OK);
+  fake::refuse = [](size_t) { return true; };
+  MUST(su2hip_get_fields(b, 1, big.data(), nullptr, nullptr, nullptr, nullptr) == SU2HIP_ENOMEM);
+  fake::refuse = [](size_t) { return false; };
+  MUST(su2hip_get_fields(b, 0, small.data(), nullptr, nullptr, nullptr, nullptr) == SU2HIP_OK);
+  MUST(b->d_stage);
+  MUST(su2hip_destroy(b) == SU2HIP_OK);
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "refused_buffers") refused_buffers();
   else if (s == "refused_call") refused_call();
   else if (s == "refused_tables") refused_tables();
+  else if (s == "refused_growth") refused_growth();
   else return 2;
   MUST(fake::live.empty());
   return 0;
