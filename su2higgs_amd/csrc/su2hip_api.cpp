@@ -1213,12 +1213,17 @@ static int resolve_links(int n, const su2hip_params *params) {
   return bytes > SU2HIP_LINKS_PACKED_ABOVE ? SU2HIP_LINKS_PACKED : SU2HIP_LINKS_FULL;
 }
 
-// whether bytes more would exceed the handle's HBM budget; the second link
-// buffers of paired passes give way to any other use
+// whether bytes more would exceed the handle's HBM budget; the second buffers
+// of paired passes give way to any other use that then fits, and the next
+// rebuild of the tables takes what is left for them
 static bool over_budget(su2hip_batch *b, size_t bytes) {
   if (!b->hbm_budget) return false;
-  if (b->used + b->pair.bytes + bytes > b->hbm_budget) pair_drop(b);
-  return b->used + bytes > b->hbm_budget;
+  if (b->used + bytes > b->hbm_budget) return true;
+  if (b->used + b->pair.bytes + bytes > b->hbm_budget) {
+    pair_drop(b);
+    b->map_dirty = true;
+  }
+  return false;
 }
 
 // the slot's hopping-term cache, inside the handle's HBM budget
@@ -1242,6 +1247,7 @@ static int hop_alloc(su2hip_batch *b, int i) {
 static void hop_release(su2hip_batch *b, int i) {
   Slot &s = b->slots[i];
   if (s.hop_mem) (void)hipFree(s.hop_mem);
+  if (s.hop_mem && b->hbm_budget && !b->pair_on) b->map_dirty = true;  // room for second buffers
   b->used -= s.hop_bytes;
   s.hop_mem = nullptr;
   s.hop_bytes = 0;

@@ -236,12 +236,38 @@ static void refused_growth() {
   MUST(su2hip_destroy(b) == SU2HIP_OK);
 }
 
+// The second buffers give way to a request that fits without them, and only to
+// such a one; where it is given back they return.
+static void budget_requests() {
+  const std::vector<su2hip_params> v{params(8, 8, 8), params(8, 8, 8)};
+  const uint64_t slots = 2 * slot_bytes(v[0]), hop = hop_cache_bytes(v[0]);
+  double rows[1 + SU2HIP_NSUMS];
+  int n = 0;
+  // the fields, their caches and the second buffers
+  su2hip_batch_t *b = made(v, 2, 2 * slots + 2 * hop);
+  MUST(sweep_pairs(b));
+  // flow buffers of a lattice: more than the second buffers hold
+  MUST(flow_words(v[0]) * wsize(v[0]) > slots);
+  MUST(su2hip_flow(b, 0, SU2HIP_FLOW_RK3, 0.05, 0.5, 1, rows, 1, &n) == SU2HIP_ENOMEM);
+  MUST(sweep_pairs(b));
+  MUST(su2hip_destroy(b) == SU2HIP_OK);
+  // room for the caches or for the second buffers
+  b = made(v, 2, 2 * slots + hop);
+  MUST(!sweep_pairs(b));
+  MUST(su2hip_set_hop_cache(b, 0) == SU2HIP_OK);
+  MUST(sweep_pairs(b));
+  MUST(su2hip_set_hop_cache(b, 1) == SU2HIP_OK);
+  MUST(!sweep_pairs(b));
+  MUST(su2hip_destroy(b) == SU2HIP_OK);
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "refused_buffers") refused_buffers();
   else if (s == "refused_call") refused_call();
   else if (s == "refused_tables") refused_tables();
   else if (s == "refused_growth") refused_growth();
+  else if (s == "budget_requests") budget_requests();
   else return 2;
   MUST(fake::live.empty());
   return 0;

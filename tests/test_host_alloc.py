@@ -25,6 +25,7 @@ def harness(tmp_path_factory):
     "refused_call",
     "refused_tables",
     "refused_growth",
+    "budget_requests",
 ])
 def test_host_side(harness, scenario):
     r = subprocess.run([harness, scenario], capture_output=True, text=True, timeout=120)
