@@ -2182,6 +2182,8 @@ int su2hip_muca_set(su2hip_batch_t *b, int slot, const su2hip_muca *m, const dou
   b->graph_valid = false;
   rc = prepare(b);
   if (rc) return rc;
+  rc = pull_desc(b);  // keep the device-owned pass counters and budgets
+  if (rc) return rc;
   rc = push_desc(b);
   if (rc) return rc;
   return orderparam_refresh(b, slot);

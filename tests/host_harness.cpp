@@ -1,7 +1,7 @@
 // The host side of the handle (su2higgs_amd/csrc/su2hip_api.cpp) on the CPU:
 // device memory is host memory, kernels are the records of their launches,
 // and the runtime's calls can be made to fail.  Built and run by
-// test_host_alloc.py; argv[1] names a scenario, a failed check ends with 1.
+// test_host_side.py; argv[1] names a scenario, a failed check ends with 1.
 #include <hip/hip_runtime.h>
 #undef __align__
 #define __align__(n)
@@ -105,7 +105,15 @@ int pair_bit(int kind, int dir) {
          : kind <= SU2HIP_K_TRIPLET_METROPOLIS ? ALT_G : ALT_S;
 }
 hipError_t launch_hop(const LaunchCtx &) { return fake::launch(); }
-hipError_t launch_end_sweep(const LaunchCtx &, int) { return fake::launch(); }
+hipError_t launch_end_sweep(const LaunchCtx &c, int passes) {
+  for (int i = 0; i < c.max_slots; i++) {
+    LatDesc &L = c.desc[i];
+    if (!L.active || L.budget == 0) continue;
+    L.pass += passes;
+    if (L.budget > 0) L.budget--;
+  }
+  return fake::launch();
+}
 hipError_t launch_cold(const LaunchCtx &, int, double, double, double) { return fake::launch(); }
 hipError_t launch_measure(const LaunchCtx &) { return fake::launch(); }
 hipError_t launch_orderparam_init(const LaunchCtx &, int) { return fake::launch(); }
@@ -261,6 +269,29 @@ static void budget_requests() {
   MUST(su2hip_destroy(b) == SU2HIP_OK);
 }
 
+// Installing a weight leaves every lattice at its place in its stream of draws.
+static void weight_keeps_draws() {
+  su2hip_batch_t *b = made({params(8, 8, 8), params(4, 4, 4)});
+  su2hip_muca m{};
+  m.enabled = 1;
+  m.bins = 4;
+  m.checks_per_sweep = 1;
+  m.orderparam = SU2HIP_PHISQ;
+  const double pos[6] = {0, 1, 2, 3, 4, 5}, W[6] = {};
+  MUST(su2hip_set_budget(b, 1, 7) == SU2HIP_OK);
+  MUST(su2hip_update(b, 5) == SU2HIP_OK);
+  MUST(su2hip_muca_set(b, 0, &m, pos, W) == SU2HIP_OK);
+  uint64_t seed, pass;
+  for (int i = 0; i < 2; i++) {
+    MUST(su2hip_rng_get(b, i, &seed, &pass) == SU2HIP_OK);
+    MUST(pass == 5 * (uint64_t)b->passes);
+  }
+  int64_t left[2];
+  MUST(su2hip_get_budgets(b, left) == SU2HIP_OK);
+  MUST(left[0] == -1 && left[1] == 2);
+  MUST(su2hip_destroy(b) == SU2HIP_OK);
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "refused_buffers") refused_buffers();
@@ -268,6 +299,7 @@ int main(int argc, char **argv) {
   else if (s == "refused_tables") refused_tables();
   else if (s == "refused_growth") refused_growth();
   else if (s == "budget_requests") budget_requests();
+  else if (s == "weight_keeps_draws") weight_keeps_draws();
   else return 2;
   MUST(fake::live.empty());
   return 0;

@@ -1,5 +1,6 @@
-"""The handle's host side where memory is refused, on the CPU: host_harness.cpp
-holds su2hip_api.cpp with a runtime whose allocations can fail."""
+"""The handle's host side on the CPU, where memory is refused and where it
+keeps what the device owns: host_harness.cpp holds su2hip_api.cpp with a runtime
+whose allocations can fail and kernels that only record their launches."""
 import os
 import subprocess
 
@@ -26,6 +27,7 @@ def harness(tmp_path_factory):
     "refused_tables",
     "refused_growth",
     "budget_requests",
+    "weight_keeps_draws",
 ])
 def test_host_side(harness, scenario):
     r = subprocess.run([harness, scenario], capture_output=True, text=True, timeout=120)
