@@ -68,6 +68,7 @@ struct FlowJob {
 
 struct Slot {
   bool used = false;
+  bool fresh = false;  // its descriptor has not been on the device yet
   su2hip_params p{};
   LatDesc hd{};
   void *mem = nullptr;
@@ -406,7 +407,7 @@ static int pull_desc(su2hip_batch *b) {
                         hipMemcpyDeviceToHost, b->stream));
   HIPTRY(hipStreamSynchronize(b->stream));
   for (int i = 0; i < b->max_slots; i++)
-    if (b->slots[i].used) {
+    if (b->slots[i].used && !b->slots[i].fresh) {
       b->slots[i].hd.pass = tmp[i].pass;
       b->slots[i].hd.budget = tmp[i].budget;
     }
@@ -426,6 +427,7 @@ static int push_desc(su2hip_batch *b) {
   HIPTRY(hipMemcpyAsync(b->d_desc, tmp.data(), sizeof(LatDesc) * b->max_slots,
                         hipMemcpyHostToDevice, b->stream));
   HIPTRY(hipStreamSynchronize(b->stream));
+  for (auto &s : b->slots) s.fresh = false;
   return SU2HIP_OK;
 }
 
@@ -1287,7 +1289,7 @@ static int alloc_slot(su2hip_batch *b, int i, const su2hip_params &p_in) {
     return fail(SU2HIP_ENOMEM, "device allocation of %zu bytes failed", bytes);
   }
   s.bytes = bytes;
-  s.used = true;
+  s.used = s.fresh = true;
   b->used += bytes;
   fill_desc(s);
   s.hd.budget = -1;

@@ -292,6 +292,26 @@ static void weight_keeps_draws() {
   MUST(su2hip_destroy(b) == SU2HIP_OK);
 }
 
+// A lattice added to a handle is swept like those it was created with.
+static void added_lattice_sweeps() {
+  for (int n = 0; n < 2; n++) {
+    su2hip_batch_t *b = nullptr;
+    const su2hip_params p = params(8, 8, 8), q = params(4, 4, 4);
+    MUST(su2hip_create(n, &p, 3, 0, &b) == SU2HIP_OK);
+    for (int k = 0; k < 2; k++) {  // a new slot, and one used before
+      int i = -1;
+      MUST(su2hip_add(b, &q, &i) == SU2HIP_OK && i == n);
+      MUST(su2hip_update(b, 2) == SU2HIP_OK);
+      int64_t left[3];
+      uint64_t seed, pass;
+      MUST(su2hip_get_budgets(b, left) == SU2HIP_OK && left[i] == -1);
+      MUST(su2hip_rng_get(b, i, &seed, &pass) == SU2HIP_OK && pass == 2 * (uint64_t)b->passes);
+      MUST(su2hip_remove(b, i) == SU2HIP_OK);
+    }
+    MUST(su2hip_destroy(b) == SU2HIP_OK);
+  }
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "refused_buffers") refused_buffers();
@@ -300,6 +320,7 @@ int main(int argc, char **argv) {
   else if (s == "refused_growth") refused_growth();
   else if (s == "budget_requests") budget_requests();
   else if (s == "weight_keeps_draws") weight_keeps_draws();
+  else if (s == "added_lattice_sweeps") added_lattice_sweeps();
   else return 2;
   MUST(fake::live.empty());
   return 0;

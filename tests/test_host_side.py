@@ -28,6 +28,7 @@ def harness(tmp_path_factory):
     "refused_growth",
     "budget_requests",
     "weight_keeps_draws",
+    "added_lattice_sweeps",
 ])
 def test_host_side(harness, scenario):
     r = subprocess.run([harness, scenario], capture_output=True, text=True, timeout=120)
