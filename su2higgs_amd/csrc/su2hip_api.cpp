@@ -1144,12 +1144,12 @@ static hipError_t download(su2hip_batch *b, const std::vector<DownPiece> &v, Sta
   };
   std::thread th[DOWN_THREADS];
   int started = 0;
-  if (e == hipSuccess && n > 1) {
+  auto start = [&] {
     try {
-      for (; started < nthreads; started++) th[started] = std::thread(work, started);
+      for (; n > 1 && started < nthreads; started++) th[started] = std::thread(work, started);
     } catch (...) {
     }
-  }
+  };
   // without all of its threads the caller moves the pieces of the missing ones
   auto finish = [&](int i) {
     const int t = i % nthreads;
@@ -1158,11 +1158,13 @@ static hipError_t download(su2hip_batch *b, const std::vector<DownPiece> &v, Sta
       moved[t].store(i + 1, std::memory_order_release);
     }
   };
-  // the next piece in flight has arrived: handed on
+  // the next piece in flight has arrived: handed on.  The threads, which spin
+  // from piece to piece, begin with the first, whatever is queued before it.
   int arrived = 0;
   auto arrive = [&] {
     e = hipEventSynchronize(ev[arrived % slots]);
     if (e != hipSuccess) return;
+    if (arrived == 0) start();
     ready.store(arrived + 1, std::memory_order_release);
     finish(arrived++);
   };

@@ -118,7 +118,11 @@ hipError_t launch_cold(const LaunchCtx &, int, double, double, double) { return 
 hipError_t launch_measure(const LaunchCtx &) { return fake::launch(); }
 hipError_t launch_orderparam_init(const LaunchCtx &, int) { return fake::launch(); }
 hipError_t launch_flow_stage(const LaunchCtx &, int, const void *, void *, const void *, void *, void *, void *, double, double, int) { return fake::launch(); }
-hipError_t launch_to_host_layout(const LaunchCtx &, int, int, int, double *) { return fake::launch(); }
+hipError_t launch_to_host_layout(const LaunchCtx &, int, int Vh, int f, double *h) {
+  const int dofs[6] = {12, 3, 4, 3, 1, 4};
+  for (size_t i = 0; i < (size_t)2 * Vh * dofs[f]; i++) h[i] = 1e8 * f + (double)i;
+  return fake::launch();
+}
 hipError_t launch_copy(const void *s, void *d, size_t n, hipStream_t) { memcpy(d, s, n); return fake::launch(); }
 }  // namespace su2
 
@@ -312,6 +316,28 @@ static void added_lattice_sweeps() {
   }
 }
 
+// Fetching fields behind queued sweeps: no thread is busy while the GPU is, and
+// every value arrives.
+static void fetch_waits_idle() {
+  const su2hip_params p = params(64, 48, 32, 1, 1);
+  su2hip_batch_t *b = made({p});
+  const size_t V = (size_t)vol_of(p);
+  std::vector<double> u(12 * V), a(3 * V), f(4 * V);
+  fake::waits = 0;
+  fake::wait_ms = 400;
+  timespec t0, t1;
+  clock_gettime(CLOCK_PROCESS_CPUTIME_ID, &t0);
+  MUST(su2hip_get_fields(b, 0, u.data(), a.data(), f.data(), nullptr, nullptr) == SU2HIP_OK);
+  clock_gettime(CLOCK_PROCESS_CPUTIME_ID, &t1);
+  const double cpu = (t1.tv_sec - t0.tv_sec) + 1e-9 * (t1.tv_nsec - t0.tv_nsec);
+  MUST(fake::waits > DOWN_SLOTS);
+  for (size_t i = 0; i < u.size(); i++) MUST(u[i] == (double)i);
+  for (size_t i = 0; i < a.size(); i++) MUST(a[i] == 1e8 + (double)i);
+  for (size_t i = 0; i < f.size(); i++) MUST(f[i] == 2e8 + (double)i);
+  MUST(cpu < 0.3);  // four threads in a loop: 1.6 s
+  MUST(su2hip_destroy(b) == SU2HIP_OK);
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "refused_buffers") refused_buffers();
@@ -321,6 +347,7 @@ int main(int argc, char **argv) {
   else if (s == "budget_requests") budget_requests();
   else if (s == "weight_keeps_draws") weight_keeps_draws();
   else if (s == "added_lattice_sweeps") added_lattice_sweeps();
+  else if (s == "fetch_waits_idle") fetch_waits_idle();
   else return 2;
   MUST(fake::live.empty());
   return 0;

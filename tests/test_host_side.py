@@ -29,6 +29,7 @@ def harness(tmp_path_factory):
     "budget_requests",
     "weight_keeps_draws",
     "added_lattice_sweeps",
+    "fetch_waits_idle",
 ])
 def test_host_side(harness, scenario):
     r = subprocess.run([harness, scenario], capture_output=True, text=True, timeout=120)
