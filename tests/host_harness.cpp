@@ -338,6 +338,26 @@ static void fetch_waits_idle() {
   MUST(su2hip_destroy(b) == SU2HIP_OK);
 }
 
+// Choosing the tiles of paired passes, on every admission of a lattice, costs by
+// the shapes of lattice in the handle and not by the lattices.
+static void many_alike() {
+  double cpu[2];
+  for (int k = 0; k < 2; k++) {
+    su2hip_batch_t *b = made(std::vector<su2hip_params>(k ? 1500 : 1, params(4, 4, 4, 0)));
+    cpu[k] = 1e9;
+    for (int r = 0; r < 9; r++) {
+      timespec t0, t1;
+      clock_gettime(CLOCK_THREAD_CPUTIME_ID, &t0);
+      MUST(build_pairs(b) == SU2HIP_OK && b->pair_on);
+      clock_gettime(CLOCK_THREAD_CPUTIME_ID, &t1);
+      cpu[k] = std::min(cpu[k], (t1.tv_sec - t0.tv_sec) + 1e-9 * (t1.tv_nsec - t0.tv_nsec));
+    }
+    MUST(su2hip_destroy(b) == SU2HIP_OK);
+  }
+  // the tables grow with the lattices; the search alone grew by 900
+  MUST(cpu[1] < 300 * cpu[0]);
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "refused_buffers") refused_buffers();
@@ -348,6 +368,7 @@ int main(int argc, char **argv) {
   else if (s == "weight_keeps_draws") weight_keeps_draws();
   else if (s == "added_lattice_sweeps") added_lattice_sweeps();
   else if (s == "fetch_waits_idle") fetch_waits_idle();
+  else if (s == "many_alike") many_alike();
   else return 2;
   MUST(fake::live.empty());
   return 0;

@@ -30,6 +30,7 @@ def harness(tmp_path_factory):
     "weight_keeps_draws",
     "added_lattice_sweeps",
     "fetch_waits_idle",
+    "many_alike",
 ])
 def test_host_side(harness, scenario):
     r = subprocess.run([harness, scenario], capture_output=True, text=True, timeout=120)
