@@ -1017,9 +1017,9 @@ static hipError_t enqueue_sweep(su2hip_batch *b) {
   // doublet and the U(1) links change only in the passes between rounds
   bool hop_fresh = false;
   LaunchCtx c = ctx_of(b);
-  for (size_t i = 0; i < b->sched.size(); i++) {
+  hipError_t e = hipSuccess;
+  for (size_t i = 0; i < b->sched.size() && e == hipSuccess; i++) {
     const Step &st = b->sched[i];
-    hipError_t e = hipSuccess;
     if (!su2_link_kind(st.kind))
       hop_fresh = false;
     else if (!hop_fresh && b->hop_on) {
@@ -1037,19 +1037,19 @@ static hipError_t enqueue_sweep(su2hip_batch *b) {
                            m.count[t]);
       });
       b->touched |= 8;
-      c.alt ^= pair_bit(st.kind, st.dir);
+      if (e == hipSuccess) c.alt ^= pair_bit(st.kind, st.dir);
       i++;
     } else if (e == hipSuccess) {
       e = enqueue_step(b, st, c.alt);
     }
-    if (e != hipSuccess) return e;
   }
-  // between sweeps every field is in its first buffer
+  // between sweeps every field is in its first buffer, after a failed launch too
   if (c.alt) {
-    hipError_t e = timed(b, SU2HIP_K_AUX, 1, [&] { return launch_pair_close(c); });
-    if (e != hipSuccess) return e;
+    const hipError_t ec = timed(b, SU2HIP_K_AUX, 1, [&] { return launch_pair_close(c); });
+    if (e == hipSuccess) e = ec;
     c.alt = 0;
   }
+  if (e != hipSuccess) return e;
   return timed(b, SU2HIP_K_AUX, 1, [&] { return launch_end_sweep(c, b->passes); });
 }
 

@@ -24,7 +24,8 @@ std::function<bool(size_t)> refuse = [](size_t) { return false; };
 std::function<hipError_t()> launch_fails = [] { return hipSuccess; };
 int wait_ms = 0;  // of an event
 std::atomic<int> waits{0};
-int singles = 0, pairs = 0, closes = 0;
+int singles = 0, pairs = 0;
+int alt = 0;  // the fields in second buffers
 std::set<void *> live;
 
 hipError_t ret(hipError_t e) {
@@ -95,14 +96,22 @@ int roctxRangePop(void) { return 0; }
 
 namespace su2 {
 hipError_t launch_pass(const LaunchCtx &, int, int, int, int, int, int) { fake::singles++; return fake::launch(); }
-hipError_t launch_pair(const LaunchCtx &, const PairTile *, int, int, int, int, int, long long *, int) { fake::pairs++; return fake::launch(); }
-hipError_t launch_pair_close(const LaunchCtx &c) { if (c.alt) fake::closes++; return fake::launch(); }
 bool pair_kind(int kind, int, int) { return kind != SU2HIP_K_LINK_METROPOLIS; }
 int pair_bit(int kind, int dir) {
   return kind <= SU2HIP_K_LINK_OVERRELAX ? 1 << dir
          : kind == SU2HIP_K_U1_METROPOLIS ? 1 << (ALT_U1_SHIFT + dir)
          : kind <= SU2HIP_K_DOUBLET_METROPOLIS ? ALT_F
          : kind <= SU2HIP_K_TRIPLET_METROPOLIS ? ALT_G : ALT_S;
+}
+hipError_t launch_pair(const LaunchCtx &, const PairTile *, int, int, int kind, int dir, int, long long *, int) {
+  fake::pairs++;
+  const hipError_t e = fake::launch();
+  if (e == hipSuccess) fake::alt ^= pair_bit(kind, dir);
+  return e;
+}
+hipError_t launch_pair_close(const LaunchCtx &c) {
+  if (c.alt == fake::alt) fake::alt = 0;
+  return fake::launch();
 }
 hipError_t launch_hop(const LaunchCtx &) { return fake::launch(); }
 hipError_t launch_end_sweep(const LaunchCtx &c, int passes) {
@@ -358,6 +367,25 @@ static void many_alike() {
   MUST(cpu[1] < 300 * cpu[0]);
 }
 
+// A launch that fails in the middle of a sweep leaves no field in its second
+// buffer, which nothing reads between sweeps.
+static void failed_launch() {
+  su2hip_batch_t *b = made({params(8, 8, 8, 1, 1)});
+  int n = 0;
+  fake::launch_fails = [&] { return n++, hipSuccess; };
+  MUST(sweep_pairs(b));
+  MUST(fake::alt == 0);
+  const int launches = n;
+  MUST(launches > 12);
+  for (int k = 0; k < launches; k++) {
+    n = 0;
+    fake::launch_fails = [&] { return n++ == k ? hipErrorLaunchFailure : hipSuccess; };
+    MUST(su2hip_update(b, 1) == SU2HIP_EDEVICE);
+    MUST(fake::alt == 0);
+  }
+  MUST(su2hip_destroy(b) == SU2HIP_OK);
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "refused_buffers") refused_buffers();
@@ -369,6 +397,7 @@ int main(int argc, char **argv) {
   else if (s == "added_lattice_sweeps") added_lattice_sweeps();
   else if (s == "fetch_waits_idle") fetch_waits_idle();
   else if (s == "many_alike") many_alike();
+  else if (s == "failed_launch") failed_launch();
   else return 2;
   MUST(fake::live.empty());
   return 0;

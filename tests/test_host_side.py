@@ -31,6 +31,7 @@ def harness(tmp_path_factory):
     "added_lattice_sweeps",
     "fetch_waits_idle",
     "many_alike",
+    "failed_launch",
 ])
 def test_host_side(harness, scenario):
     r = subprocess.run([harness, scenario], capture_output=True, text=True, timeout=120)
