@@ -113,6 +113,7 @@ hipError_t launch_pair_close(const LaunchCtx &c) {
   if (c.alt == fake::alt) fake::alt = 0;
   return fake::launch();
 }
+hipError_t launch_order(const LaunchCtx &, uint8_t *, const uint16_t *, int, int, int) { return fake::launch(); }
 hipError_t launch_hop(const LaunchCtx &) { return fake::launch(); }
 hipError_t launch_end_sweep(const LaunchCtx &c, int passes) {
   for (int i = 0; i < c.max_slots; i++) {
@@ -386,6 +387,92 @@ static void failed_launch() {
   MUST(su2hip_destroy(b) == SU2HIP_OK);
 }
 
+// Which passes of a sweep are paired, for the handles of test_gpu_pairs.py and
+// test_gpu_pairs_mixed.py.
+static su2hip_params shaped(int form, int a, int b, int c, int nhiggs, int u1, int triplet, int singlet) {
+  su2hip_params p = params(a, b, c, nhiggs, u1);
+  p.precision = form ? SU2HIP_FP32 : SU2HIP_FP64;
+  p.link_format = form == 2 ? SU2HIP_LINKS_PACKED : form == 1 ? SU2HIP_LINKS_FULL : SU2HIP_LINKS_AUTO;
+  p.triplet = triplet;
+  p.singlet = singlet;
+  return p;
+}
+static uint64_t footprints(const std::vector<su2hip_params> &v) {
+  uint64_t total = 0;
+  for (const auto &p : v) {
+    uint64_t n = 0;
+    MUST(su2hip_footprint(&p, 0, &n) == SU2HIP_OK);
+    total += n;
+  }
+  return total;
+}
+static void which_sweeps_pair() {
+  using Ext = std::vector<std::array<int, 3>>;
+  const std::vector<Ext> small = {
+      {{4, 4, 2}, {2, 4, 6}, {8, 8, 8}}, {{34, 10, 14}}, {{128, 6, 4}, {4, 26, 12}},
+      {{24, 24, 24}, {16, 30, 10}, {12, 6, 50}}, {{12, 10, 14}, {8, 8, 8}, {4, 26, 12}},
+      {{8, 8, 8}, {12, 10, 8}, {16, 16, 16}, {6, 8, 10}}};
+  const std::vector<Ext> links = {{{40, 34, 30}}, {{24, 30, 26}, {34, 26, 22}}};
+  const std::vector<Ext> none = {{{64, 48, 40}}, {{130, 4, 4}}};
+  const int models[][4] = {{0, 0, 0, 0}, {1, 1, 0, 0}, {1, 1, 0, 1}, {0, 0, 1, 0}, {1, 0, 1, 0}};
+  auto batch = [&](const Ext &x, int form, const int *m) {
+    std::vector<su2hip_params> v;
+    for (const auto &e : x) v.push_back(shaped(form, e[0], e[1], e[2], m[0], m[1], m[2], m[3]));
+    return v;
+  };
+  for (int form = 0; form < 3; form++)
+    for (const auto &m : models) {
+      for (const auto &x : small) {
+        su2hip_batch_t *b = made(batch(x, form, m));
+        MUST(sweep_pairs(b) && b->pair_fields);
+        MUST(su2hip_destroy(b) == SU2HIP_OK);
+        // a budget of the footprints leaves no room
+        b = made(batch(x, form, m), 0, footprints(batch(x, form, m)));
+        MUST(!sweep_pairs(b));
+        MUST(su2hip_destroy(b) == SU2HIP_OK);
+      }
+      for (const auto &x : links) {
+        su2hip_batch_t *b = made(batch(x, form, m));
+        MUST(sweep_pairs(b) && !b->pair_fields);
+        MUST(fake::pairs == 15 && (fake::singles > 0) == (m[0] + m[2] > 0));
+        MUST(su2hip_destroy(b) == SU2HIP_OK);
+        b = made(batch(x, form, m), 0, footprints(batch(x, form, m)));
+        MUST(!sweep_pairs(b));
+        MUST(su2hip_destroy(b) == SU2HIP_OK);
+      }
+      for (const auto &x : none) {
+        su2hip_batch_t *b = made(batch(x, form, m));
+        MUST(!sweep_pairs(b));
+        MUST(su2hip_destroy(b) == SU2HIP_OK);
+      }
+    }
+  // one round of Metropolis, one of overrelaxation
+  su2hip_params p = params(12, 10, 8, 1, 1);
+  p.algorithm_su2link = SU2HIP_METROPOLIS;
+  p.link_overrelax = 1;
+  su2hip_batch_t *b = made({p});
+  MUST(sweep_pairs(b) && fake::singles == 6);
+  // the shuffled order
+  MUST(su2hip_set_random_order(b, 1) == SU2HIP_OK);
+  MUST(!sweep_pairs(b));
+  MUST(su2hip_destroy(b) == SU2HIP_OK);
+  // two doublets
+  b = made({params(8, 8, 8, 2)});
+  MUST(!sweep_pairs(b));
+  MUST(su2hip_destroy(b) == SU2HIP_OK);
+  // a flow's buffers in place of the second ones, until its lattice leaves
+  const std::vector<su2hip_params> v(3, params(12, 10, 14));
+  b = made(v, 0, footprints(v) * 29 / 20);
+  std::vector<double> rows(100 * (1 + SU2HIP_NSUMS));
+  int n = 0;
+  MUST(sweep_pairs(b));
+  MUST(su2hip_flow(b, 0, SU2HIP_FLOW_RK3, 0.05, 0.2, 2, rows.data(), 100, &n) == SU2HIP_OK);
+  MUST(!sweep_pairs(b));
+  MUST(su2hip_remove(b, 0) == SU2HIP_OK);
+  MUST(sweep_pairs(b));
+  MUST(su2hip_destroy(b) == SU2HIP_OK);
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "refused_buffers") refused_buffers();
@@ -398,6 +485,7 @@ int main(int argc, char **argv) {
   else if (s == "fetch_waits_idle") fetch_waits_idle();
   else if (s == "many_alike") many_alike();
   else if (s == "failed_launch") failed_launch();
+  else if (s == "which_sweeps_pair") which_sweeps_pair();
   else return 2;
   MUST(fake::live.empty());
   return 0;

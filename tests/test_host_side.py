@@ -32,6 +32,7 @@ def harness(tmp_path_factory):
     "fetch_waits_idle",
     "many_alike",
     "failed_launch",
+    "which_sweeps_pair",
 ])
 def test_host_side(harness, scenario):
     r = subprocess.run([harness, scenario], capture_output=True, text=True, timeout=120)
