@@ -964,21 +964,20 @@ static hipError_t enqueue_step(su2hip_batch *b, const Step &st, int alt, bool in
     c.order = b->d_order;
     c.npass = b->passes;
   }
-  int reunit = b->tmpl.reunitarize && !b->fp64;
   if (!st.muca) {
     LaunchCtx ct = ctx_for(b, st.kind);
     ct.alt = alt;
     ct.order = c.order;
     ct.npass = c.npass;
     return timed(b, st.kind, 1, [&] {
-      return launch_pass(ct, st.kind, st.parity, st.dir, st.pass_off, -1, reunit);
+      return launch_pass(ct, st.kind, st.parity, st.dir, st.pass_off, -1);
     });
   }
   c.waves = b->waves[st.kind];  // multicanonical steps keep the 256-site table
   b->touched |= 1;
   for (int k = 0; k < b->muca_steps; k++) {
     hipError_t e = timed(b, st.kind, 1, [&] {
-      return launch_pass(c, st.kind, st.parity, st.dir, st.pass_off, k, reunit);
+      return launch_pass(c, st.kind, st.parity, st.dir, st.pass_off, k);
     });
     if (e != hipSuccess) return e;
     e = timed(b, SU2HIP_K_MUCA, 1,
@@ -2799,7 +2798,6 @@ static int time_pass_impl(su2hip_batch *b, int kind, int repeats, double *ms_ker
   hipError_t e = hipSuccess;
   for (size_t i = 0; i < ev.size() && e == hipSuccess; i++) e = hipEventCreate(&ev[i]);
   LaunchCtx c = ctx_for(b, kind);
-  int reunit = b->tmpl.reunitarize && !b->fp64;
   hipEvent_t s0 = ev[2 * (size_t)repeats], s1 = ev[2 * (size_t)repeats + 1];
   // link passes read the hopping-term cache, filled once outside the timing
   if (e == hipSuccess && b->hop_on && su2_link_kind(kind)) e = launch_hop(ctx_of(b));
@@ -2807,7 +2805,7 @@ static int time_pass_impl(su2hip_batch *b, int kind, int repeats, double *ms_ker
   for (int i = 0; i < repeats && e == hipSuccess; i++) {
     c.ev_start = ev[2 * (size_t)i];
     c.ev_stop = ev[2 * (size_t)i + 1];
-    e = launch_pass(c, kind, i & 1, (i >> 1) % ndir, i, -1, reunit);
+    e = launch_pass(c, kind, i & 1, (i >> 1) % ndir, i, -1);
   }
   if (e == hipSuccess) e = hipEventRecord(s1, b->stream);
   if (e == hipSuccess) e = hipEventSynchronize(s1);

@@ -184,7 +184,7 @@ struct LaunchCtx {
 // a doublet kind).  muca_step < 0: plain pass; otherwise the pass is step
 // `muca_step` of a multicanonical parity sweep.
 hipError_t launch_pass(const LaunchCtx &c, int kind, int parity, int dir,
-                       int pass_off, int muca_step, int reunit);
+                       int pass_off, int muca_step);
 // whether launch_pair takes a pass kind of a model
 bool pair_kind(int kind, int model, int fp64);
 // the bit of LaunchCtx::alt that a paired pass changes

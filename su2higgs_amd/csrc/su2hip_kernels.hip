@@ -596,10 +596,6 @@ __device__ void hb_dir_wave(const Rng &r, bool want, double &r1o, double &r2o, d
 // ------------------------------------------------------------------------
 // per-site updates; each returns 1 if accepted and stores the new value
 
-struct Fields {
-  void *U, *A, *F, *G, *S, *B;
-};
-
 // The move of an SU(2) link kind from the link `old` and its staple V (a1,
 // a2: the triplets at its ends): 1 with the new link in nu, 0 rejected, 2
 // counted as accepted and unchanged.  Lanes with `on` false only keep a full
@@ -1232,7 +1228,7 @@ template <typename T, int M, int KIND>
 __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
                                           const MucaDev *__restrict__ mucas,
                                           const BlockMap *__restrict__ blk, int one, int chunk, int alt,
-                                          int par_in, int mu_in, int pass_off, int step, int reunit,
+                                          int par_in, int mu_in, int pass_off, int step,
                                           long long *__restrict__ cnt, int nblk,
                                           double *__restrict__ partial,
                                           const uint8_t *__restrict__ order, int npass,
@@ -1330,13 +1326,13 @@ __device__ __forceinline__ void pass_body(const LatDesc *__restrict__ lats,
 #define K_PASS_ARGS                                                                          \
   const LatDesc *__restrict__ lats, const MucaDev *__restrict__ mucas,                       \
       const BlockMap *__restrict__ blk, int one, int chunk, int alt, int par_in, int mu_in,  \
-      int pass_off, int step, int reunit, long long *__restrict__ cnt, int nblk, double *__restrict__ partial,       \
+      int pass_off, int step, long long *__restrict__ cnt, int nblk, double *__restrict__ partial,       \
       const uint8_t *__restrict__ order, int npass
 
 template <typename T, int M, int KIND>
 __global__ __launch_bounds__(BLK) void k_pass(K_PASS_ARGS) {
   __shared__ double lds[BLK / 64];
-  pass_body<T, M, KIND>(lats, mucas, blk, one, chunk, alt, par_in, mu_in, pass_off, step, reunit, cnt, nblk,
+  pass_body<T, M, KIND>(lats, mucas, blk, one, chunk, alt, par_in, mu_in, pass_off, step, cnt, nblk,
                         partial, order, npass, lds);
 }
 
@@ -1349,7 +1345,7 @@ template <typename T, int M, int KIND>
 __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(5))) void k_pass_w5(
     K_PASS_ARGS) {
   __shared__ double lds[BLK / 64];
-  pass_body<T, M, KIND>(lats, mucas, blk, one, chunk, alt, par_in, mu_in, pass_off, step, reunit, cnt, nblk,
+  pass_body<T, M, KIND>(lats, mucas, blk, one, chunk, alt, par_in, mu_in, pass_off, step, cnt, nblk,
                         partial, order, npass, lds);
 }
 
@@ -3172,8 +3168,7 @@ static hipError_t with_prec(int fp64, Fn &&fn) {
 }
 
 template <typename T, int M, int KIND>
-static hipError_t pass_one(const LaunchCtx &c, int parity, int dir, int pass_off, int step,
-                           int reunit) {
+static hipError_t pass_one(const LaunchCtx &c, int parity, int dir, int pass_off, int step) {
   if constexpr (kind_valid<M, KIND>()) {
     // multicanonical steps use the 256-site table: their order-parameter
     // partials are indexed by 256-site chunk
@@ -3185,10 +3180,10 @@ static hipError_t pass_one(const LaunchCtx &c, int parity, int dir, int pass_off
         if (c.ev_start || c.ev_stop) {
           hipExtLaunchKernelGGL((k_pass_w5<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream,
                                 c.ev_start, c.ev_stop, 0, c.desc, c.muca, c.blk, c.one, c.block, c.alt, parity, dir,
-                                pass_off, step, reunit, c.cnt, c.nblk, c.partial, c.order, c.npass);
+                                pass_off, step, c.cnt, c.nblk, c.partial, c.order, c.npass);
         } else {
           hipLaunchKernelGGL((k_pass_w5<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream,
-                             c.desc, c.muca, c.blk, c.one, c.block, c.alt, parity, dir, pass_off, step, reunit, c.cnt,
+                             c.desc, c.muca, c.blk, c.one, c.block, c.alt, parity, dir, pass_off, step, c.cnt,
                              c.nblk, c.partial, c.order, c.npass);
         }
         return hipGetLastError();
@@ -3197,10 +3192,10 @@ static hipError_t pass_one(const LaunchCtx &c, int parity, int dir, int pass_off
     if (c.ev_start || c.ev_stop) {
       hipExtLaunchKernelGGL((k_pass<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream,
                             c.ev_start, c.ev_stop, 0, c.desc, c.muca, c.blk, c.one, c.block, c.alt, parity, dir, pass_off,
-                            step, reunit, c.cnt, c.nblk, c.partial, c.order, c.npass);
+                            step, c.cnt, c.nblk, c.partial, c.order, c.npass);
     } else {
       hipLaunchKernelGGL((k_pass<T, M, KIND>), dim3(c.nblk), dim3(c.block), 0, c.stream, c.desc,
-                         c.muca, c.blk, c.one, c.block, c.alt, parity, dir, pass_off, step, reunit, c.cnt, c.nblk,
+                         c.muca, c.blk, c.one, c.block, c.alt, parity, dir, pass_off, step, c.cnt, c.nblk,
                          c.partial, c.order, c.npass);
     }
     return hipGetLastError();
@@ -3209,23 +3204,23 @@ static hipError_t pass_one(const LaunchCtx &c, int parity, int dir, int pass_off
 }
 
 hipError_t launch_pass(const LaunchCtx &c, int kind, int parity, int dir, int pass_off,
-                       int muca_step, int reunit) {
+                       int muca_step) {
   if (c.nblk == 0) return hipSuccess;
   return with_prec(c.fp64, [&](auto t) {
     using T = decltype(t);
     return with_model_of<T>(c.model, [&](auto m) -> hipError_t {
       constexpr int M = decltype(m)::value;
       switch (kind) {
-        case SU2HIP_K_LINK_HEATBATH: return pass_one<T, M, SU2HIP_K_LINK_HEATBATH>(c, parity, dir, pass_off, muca_step, reunit);
-        case SU2HIP_K_LINK_METROPOLIS: return pass_one<T, M, SU2HIP_K_LINK_METROPOLIS>(c, parity, dir, pass_off, muca_step, reunit);
-        case SU2HIP_K_LINK_OVERRELAX: return pass_one<T, M, SU2HIP_K_LINK_OVERRELAX>(c, parity, dir, pass_off, muca_step, reunit);
-        case SU2HIP_K_U1_METROPOLIS: return pass_one<T, M, SU2HIP_K_U1_METROPOLIS>(c, parity, dir, pass_off, muca_step, reunit);
-        case SU2HIP_K_DOUBLET_OVERRELAX: return pass_one<T, M, SU2HIP_K_DOUBLET_OVERRELAX>(c, parity, dir, pass_off, muca_step, reunit);
-        case SU2HIP_K_DOUBLET_METROPOLIS: return pass_one<T, M, SU2HIP_K_DOUBLET_METROPOLIS>(c, parity, dir, pass_off, muca_step, reunit);
-        case SU2HIP_K_TRIPLET_OVERRELAX: return pass_one<T, M, SU2HIP_K_TRIPLET_OVERRELAX>(c, parity, dir, pass_off, muca_step, reunit);
-        case SU2HIP_K_TRIPLET_METROPOLIS: return pass_one<T, M, SU2HIP_K_TRIPLET_METROPOLIS>(c, parity, dir, pass_off, muca_step, reunit);
-        case SU2HIP_K_SINGLET_OVERRELAX: return pass_one<T, M, SU2HIP_K_SINGLET_OVERRELAX>(c, parity, dir, pass_off, muca_step, reunit);
-        case SU2HIP_K_SINGLET_METROPOLIS: return pass_one<T, M, SU2HIP_K_SINGLET_METROPOLIS>(c, parity, dir, pass_off, muca_step, reunit);
+        case SU2HIP_K_LINK_HEATBATH: return pass_one<T, M, SU2HIP_K_LINK_HEATBATH>(c, parity, dir, pass_off, muca_step);
+        case SU2HIP_K_LINK_METROPOLIS: return pass_one<T, M, SU2HIP_K_LINK_METROPOLIS>(c, parity, dir, pass_off, muca_step);
+        case SU2HIP_K_LINK_OVERRELAX: return pass_one<T, M, SU2HIP_K_LINK_OVERRELAX>(c, parity, dir, pass_off, muca_step);
+        case SU2HIP_K_U1_METROPOLIS: return pass_one<T, M, SU2HIP_K_U1_METROPOLIS>(c, parity, dir, pass_off, muca_step);
+        case SU2HIP_K_DOUBLET_OVERRELAX: return pass_one<T, M, SU2HIP_K_DOUBLET_OVERRELAX>(c, parity, dir, pass_off, muca_step);
+        case SU2HIP_K_DOUBLET_METROPOLIS: return pass_one<T, M, SU2HIP_K_DOUBLET_METROPOLIS>(c, parity, dir, pass_off, muca_step);
+        case SU2HIP_K_TRIPLET_OVERRELAX: return pass_one<T, M, SU2HIP_K_TRIPLET_OVERRELAX>(c, parity, dir, pass_off, muca_step);
+        case SU2HIP_K_TRIPLET_METROPOLIS: return pass_one<T, M, SU2HIP_K_TRIPLET_METROPOLIS>(c, parity, dir, pass_off, muca_step);
+        case SU2HIP_K_SINGLET_OVERRELAX: return pass_one<T, M, SU2HIP_K_SINGLET_OVERRELAX>(c, parity, dir, pass_off, muca_step);
+        case SU2HIP_K_SINGLET_METROPOLIS: return pass_one<T, M, SU2HIP_K_SINGLET_METROPOLIS>(c, parity, dir, pass_off, muca_step);
       }
       return hipErrorInvalidValue;
     });

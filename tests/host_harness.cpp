@@ -95,7 +95,7 @@ int roctxRangePop(void) { return 0; }
 #include "../su2higgs_amd/csrc/su2hip_api.cpp"
 
 namespace su2 {
-hipError_t launch_pass(const LaunchCtx &, int, int, int, int, int, int) { fake::singles++; return fake::launch(); }
+hipError_t launch_pass(const LaunchCtx &, int, int, int, int, int) { fake::singles++; return fake::launch(); }
 bool pair_kind(int kind, int, int) { return kind != SU2HIP_K_LINK_METROPOLIS; }
 int pair_bit(int kind, int dir) {
   return kind <= SU2HIP_K_LINK_OVERRELAX ? 1 << dir
