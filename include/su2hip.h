@@ -225,7 +225,9 @@ const char *su2hip_last_error(void);
  * src/layout.c:657-704, src/alloc.c:103-125) for n lattices at once.
  * max_slots >= n reserves room for lattices added later (serving); n = 0
  * makes an empty handle whose template is params[0];
- * hbm_budget (bytes, 0 = unlimited) caps the field memory of all slots. */
+ * hbm_budget (bytes, 0 = unlimited) caps the field memory of all slots.  Small
+ * handles keep a second copy of the fields for their sweeps (su2hip_set_chunk)
+ * in what the budget leaves free, and give it up to any other use. */
 int su2hip_create(int n, const su2hip_params *params, int max_slots,
                   uint64_t hbm_budget, su2hip_batch_t **out);
 int su2hip_destroy(su2hip_batch_t *b);
@@ -449,9 +451,17 @@ int su2hip_time_pass(su2hip_batch_t *b, int kind, int repeats, double *ms_kernel
  * of one lattice (chunks dealt to the 8 XCDs in contiguous runs).  The
  * chunk of a pass kind is the one set here, or with 0 (default) the widest
  * that still gives 4 workgroups per CU for the batch.  Results do not depend
- * on the chunk.  Multicanonical steps always use 256. */
+ * on the chunk.  Multicanonical steps always use 256.
+ * The sweeps of small handles (at most 120000 sites in FP32, 65536 in FP64,
+ * L1 <= 128, room for second field buffers in the HBM budget) make both
+ * parities' link passes in one launch whose workgroups are tiles of the
+ * lattices, and up to 36000 sites most passes of the other fields; those
+ * launches have neither a chunk nor an occupancy target.  There the settings
+ * below, and what su2hip_autotune measures, apply to the passes that are
+ * launched one by one: su2hip_pass, su2hip_time_pass, multicanonical passes,
+ * link Metropolis, two doublets and the random pass order. */
 int su2hip_set_chunk(su2hip_batch_t *b, int kind, int chunk);
-/* The chunk a pass kind launches with now. */
+/* The chunk a pass kind launches with now, where it is launched on its own. */
 int su2hip_get_chunk(su2hip_batch_t *b, int kind, int *chunk);
 /* Occupancy target of a pass kind's kernel: 0 = the compiler's own register
  * allocation, 5 = registers capped so that 5 waves fit per SIMD.  The link
@@ -459,7 +469,8 @@ int su2hip_get_chunk(su2hip_batch_t *b, int kind, int *chunk);
  * with 0, and asking it for 5 fails with SU2HIP_EINVAL.  Which one is
  * faster depends on the lattice; results do not depend on it. */
 int su2hip_set_waves(su2hip_batch_t *b, int kind, int waves);
-/* The occupancy target a pass kind launches with now. */
+/* The occupancy target a pass kind launches with now, where it is launched on
+ * its own. */
 int su2hip_get_waves(su2hip_batch_t *b, int kind, int *waves);
 /* Hopping-term cache (no reference counterpart; the doublet part of the
  * link staple, src/staples.c:150-190).  With one doublet the handle can keep,

@@ -580,7 +580,11 @@ static int build_alt(su2hip_batch *b, AltMap &m, int chunk) {
 constexpr uint64_t PAIR_SITES_FP32 = 120000, PAIR_SITES_FP64 = 65536;
 // and those of the other kinds: sweeps with five link rounds, links paired ->
 // all: FP32 24^3 113.8 -> 110.6 us, 32^3 113.7 -> 113.3, 48^3 139 -> 146; FP64
-// triplet 24^3 166 -> 158
+// triplet 24^3 166 -> 158, with U(1) 40^3 231 -> 251.  One line for all kinds
+// and both precisions, just above the largest size at which each was measured
+// to gain; a kind alone gains differently (FP64 18 x 14 x 26: singlet 9.3 -> 5.0
+// us for two passes, FP32 24^3 doublet 6.1 -> 5.4), so a line by kind may lie
+// elsewhere.
 constexpr uint64_t PAIR_SITES_FIELDS = 36000;
 
 // Tiles of link direction dir in one lattice: whole rows in x and n1 of them

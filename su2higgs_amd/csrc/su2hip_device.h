@@ -284,7 +284,8 @@ __device__ __forceinline__ gptr<T> gmem(T *p) {
 // that each 16-byte load of a wavefront covers one contiguous 1 KiB; as 32
 // bytes a site, each of the two loads touched the lines of both and the L1s
 // were the FP64 link passes' second limit after the fabric (96^3 sweep 969 ->
-// 949 us, four 48^3 adjoint lattices 498 -> 484).  32-bit byte offsets from a uniform base (2^27 sites of 32 bytes).
+// 949 us, four 48^3 adjoint lattices 498 -> 484).  32-bit byte offsets from a
+// uniform base: at most 2^27 sites of a parity, 16 bytes each.
 template <typename T>
 __device__ __forceinline__ Q<T> ld4(const T *run, int Vh, int s) {
   const char *b = reinterpret_cast<const char *>(run);

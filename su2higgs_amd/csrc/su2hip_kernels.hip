@@ -1337,10 +1337,11 @@ __global__ __launch_bounds__(BLK) void k_pass(K_PASS_ARGS) {
 }
 
 // The same pass with an occupancy target of 5 waves per SIMD, built for the
-// link overrelaxation only: whether it wins depends on the lattice (FP64
-// 96^3 22.5 against 22.9 us, 192^3 232 against 222 us, in one GPU
-// session), so the autotuner picks per handle; the other kinds either do
-// not change or spill under it.
+// link overrelaxation only; the other kinds either do not change or spill
+// under it.  Alternating in one GPU session the two are within 0.5% (us, target
+// against the compiler's own: FP64 96^3 16.6 / 16.6, 192^3 187.7 / 187.4, FP32
+// 192^3 56.4 / 56.4); with the loads of earlier kernels they differed by up to
+// 4%, either way by the lattice, so the autotuner still times both.
 template <typename T, int M, int KIND>
 __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(5))) void k_pass_w5(
     K_PASS_ARGS) {
@@ -2477,8 +2478,9 @@ __device__ __forceinline__ void store_row(const double *v, double *lds, double *
 // Each thread measures site s of parity 0, then of parity 1, so every sum
 // of a thread is (0 + site0) + site1 in that order.  The loop is kept
 // rolled: interleaving the two sites doubles the live registers.  Only the
-// model's own sums are reduced: the butterflies of all 24 were 288 cross-lane
-// reads per wavefront, 20 remain.
+// model's own sums are reduced: a sum's butterfly is 12 cross-lane reads per
+// wavefront (six steps of two words), 288 for all 24, 72 for the six of
+// SU(2)xU(1)+Higgs.
 template <typename T, int M>
 __device__ __forceinline__ void measure_chunk(const LatDesc &L, int s0, double *row, double *lds) {
   const int s = s0 + (int)threadIdx.x;
@@ -2510,8 +2512,8 @@ __device__ __forceinline__ void magcharge_chunk(const LatDesc &L, int s0, double
 // The rows of one lattice added up, one workgroup of FIN threads: G groups of
 // threads take every G-th row, a thread one sum, and the groups are added in
 // a tree.  A row per thread and all its sums in a loop waited for 7 rows one
-// after another at 96^3 (17.1 us); this has every row in flight at once
-// (6.4 us).
+// after another at 96^3 (17.1 us); here a thread has one sum of 10 or 11 rows
+// there (1 728 rows, 170 groups), eight of them in flight (6.4 us).
 constexpr int FIN = 1024;
 __device__ __forceinline__ void sum_rows(const double *__restrict__ rows, int n, uint32_t live,
                                          double *out, double *lds) {
