@@ -2157,6 +2157,8 @@ __device__ double alpha_proj(const LatDesc &L, const T *U, const T *G, const Sit
 // -> 19.1, and FP64 with two doublets 42.3 -> 55.0, with U(1) 90.5 -> 93.3.  The
 // others gain: FP64 pure gauge 25.8 -> 19.6, SU(2)xU(1)+Higgs 48.6 -> 41.7,
 // with both doublet and triplet 47.7 -> 45.2, FP32 two doublets 30.6 -> 29.8.
+// (FP64 with one doublet alone: 33.8 -> 32.4, where the kernel before the halves
+// layout took 30.7; four 48^3 lattices 19.3 -> 17.9 and 19.0.)
 template <typename T, int M>
 constexpr bool links_together() {
   if ((M & M_TR) != 0) return (M & M_NH) != 0;
